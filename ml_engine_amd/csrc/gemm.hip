@@ -4,6 +4,7 @@
 // (Engine/kernels.cu:387-539): every C element is written by exactly one lane,
 // so results are deterministic.
 #include "activation.hpp"
+#include "gemm_args.hpp"
 #include "gemm_core.hpp"
 
 #include <float.h>
@@ -14,72 +15,6 @@ using namespace mle;
 using namespace gemm;
 
 namespace {
-
-struct GemmArgs {
-  const float* A;
-  const float* B;
-  float* C;
-  float* colsum;
-  int64_t lda, ldb, ldc, sa, sb, sc;
-  int M, N, K;
-  float alpha, beta;
-  // split-K: blockIdx.z = batch item * splits + split; each split covers
-  // kchunk of K and writes its raw tile to part (and its column sums to
-  // part_cs); split_reduce_kernel combines them in split order.
-  int splits, kchunk;
-  float* part;
-  float* part_cs;
-  const float* bias;  // nullable: C[r, c] += bias[c] after alpha/beta
-  // Two-level batch: item z = zo * inner + zi sits at zo * s + zi * s2 of
-  // each operand (inner == 1: one stride).  Lets per-head products address
-  // the heads of a [batch, seq, heads * dim] tensor in place.
-  int inner;
-  int64_t sa2, sb2, sc2;
-  // Per batch item bias and column-sum strides (0: shared).
-  int64_t sbias, scs;
-  // Sum of products: when grouped, split s multiplies A + s*gsa by B + s*gsb
-  // over the whole K (the splits are the terms), and the reduce adds them in
-  // term order.
-  int grouped;
-  int64_t gsa, gsb;
-  // Sum of products folded into K (register-direct kernel, one split): stage
-  // kt of the K loop reads term kt / (K / KD) of A + t*gsa and B + t*gsb.
-  int kterms;
-  // Row statistics of C (persistent kernel): for row r and 64-column block b,
-  // rowpart[r * rp_ld + 2 b] = max over the block, [.. + 1] = sum of
-  // exp(C - max).  nullptr: none.
-  float* rowpart;
-  int64_t rp_ld;
-  // Activation epilogues (persistent kernel, C's layout): forward writes
-  // act_y = act(C); backward writes act_dx (+)= C * act'(act_x).
-  float* act_y;
-  const float* act_x;
-  float* act_dx;
-  int act_acc;
-  // 1 + an activation kind: the split reduce also writes act_y = act(C) in
-  // C's layout (0: not).
-  int act_red;
-  // Column sums: 0 adds them into colsum (the default), 1 assigns (colsum is
-  // logically zero).
-  int cs_assign;
-  // 1 + an activation kind: the small-product kernels (simple, K-split) also
-  // write act_dx (+)= act'(act_x) * C in C's layout, act_acc choosing add or
-  // assign (0: not).
-  int act_bwd;
-};
-
-// colsum[i] (+)= v as GemmArgs::cs_assign says.
-__device__ __forceinline__ void put_colsum(const GemmArgs& g, int64_t i, float v) {
-  g.colsum[i] = g.cs_assign ? v : g.colsum[i] + v;
-}
-
-// Epilogue modes of the persistent kernel.
-constexpr int kEpiPlain = 0, kEpiRowstats = 1, kEpiActFwd = 2, kEpiActBwd = 3;
-
-__device__ __forceinline__ int64_t batch_off(int64_t z, const GemmArgs& g, int64_t s, int64_t s2) {
-  if (g.inner == 1) return z * s;
-  return (z / g.inner) * s + (z % g.inner) * s2;
-}
 
 // Load 4 consecutive elements base[r*ld + c .. c+3] with bounds (R rows, Cc cols).
 template <bool VEC>
@@ -98,26 +33,6 @@ __device__ __forceinline__ f32x4 ld_guard(const float* __restrict__ base, int64_
   return v;
 }
 
-// Branch-free operand reads through a raw buffer resource: lanes outside the
-// matrix use an offset beyond the resource's extent and the hardware range
-// check returns zeros (buffer_load_dwordx4 ... offen).  Used when every
-// operand extent is below 2 GiB and the contiguous bound is a multiple of 4,
-// so a float4 is either wholly inside or wholly outside.
-constexpr uint32_t kBufOOB = 0x80000000u;
-constexpr int kBufWord3 = 0x00020000;  // gfx9-family raw buffer descriptor word 3
-
-struct BufOperand {
-  __amdgpu_buffer_rsrc_t rsrc;
-  int64_t ld;
-  __device__ BufOperand(const float* base, int64_t ld_, uint32_t bytes)
-      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, (int)bytes, kBufWord3)), ld(ld_) {}
-  __device__ __forceinline__ f32x4 load(int r, int c, int R, int Cc) const {
-    const bool ok = (r < R) & (c < Cc);
-    const uint32_t off = ok ? (uint32_t)(((int64_t)r * ld + c) * 4) : kBufOOB;
-    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0));
-  }
-};
-
 // Global -> registers for one stage.  A tile is TM x KD (TM*KD/1024 float4
 // per thread), a B tile KD x TN.  A_MC == trans_a (A stored K x M); B_KC ==
 // trans_b.  `kend` bounds K for this workgroup's split.  k-contiguous tiles
@@ -133,26 +48,24 @@ __device__ __forceinline__ void tile_coord(int f, int& r, int& c) {
   }
 }
 
-template <bool A_MC, int VEC, int TM, int KD>
-__device__ __forceinline__ void load_a(const GemmArgs& g, const float* A, const BufOperand& Ab, int m0, int k0,
-                                       int kend, int tid, f32x4 (&r)[TM * KD / 1024]) {
+template <bool A_MC, bool VEC, int TM, int KD>
+__device__ __forceinline__ void load_a(const GemmArgs& g, const float* A, int m0, int k0, int kend, int tid,
+                                       f32x4 (&r)[TM * KD / 1024]) {
 #pragma unroll
   for (int i = 0; i < TM * KD / 1024; ++i) {
     int a, b;
     tile_coord<A_MC, TM, KD>(tid + NT * i, a, b);
-    if (!A_MC) r[i] = VEC == 2 ? Ab.load(m0 + a, k0 + b, g.M, kend) : ld_guard<VEC == 1>(A, g.lda, m0 + a, k0 + b, g.M, kend);
-    else r[i] = VEC == 2 ? Ab.load(k0 + a, m0 + b, kend, g.M) : ld_guard<VEC == 1>(A, g.lda, k0 + a, m0 + b, kend, g.M);
+    r[i] = A_MC ? ld_guard<VEC>(A, g.lda, k0 + a, m0 + b, kend, g.M) : ld_guard<VEC>(A, g.lda, m0 + a, k0 + b, g.M, kend);
   }
 }
-template <bool B_KC, int VEC, int TN, int KD>
-__device__ __forceinline__ void load_b(const GemmArgs& g, const float* B, const BufOperand& Bb, int n0, int k0,
-                                       int kend, int tid, f32x4 (&r)[TN * KD / 1024]) {
+template <bool B_KC, bool VEC, int TN, int KD>
+__device__ __forceinline__ void load_b(const GemmArgs& g, const float* B, int n0, int k0, int kend, int tid,
+                                       f32x4 (&r)[TN * KD / 1024]) {
 #pragma unroll
   for (int i = 0; i < TN * KD / 1024; ++i) {
     int a, b;
     tile_coord<!B_KC, TN, KD>(tid + NT * i, a, b);
-    if (B_KC) r[i] = VEC == 2 ? Bb.load(n0 + a, k0 + b, g.N, kend) : ld_guard<VEC == 1>(B, g.ldb, n0 + a, k0 + b, g.N, kend);
-    else r[i] = VEC == 2 ? Bb.load(k0 + a, n0 + b, kend, g.N) : ld_guard<VEC == 1>(B, g.ldb, k0 + a, n0 + b, kend, g.N);
+    r[i] = B_KC ? ld_guard<VEC>(B, g.ldb, n0 + a, k0 + b, g.N, kend) : ld_guard<VEC>(B, g.ldb, k0 + a, n0 + b, kend, g.N);
   }
 }
 
@@ -167,13 +80,6 @@ __device__ __forceinline__ void store_tile(float* S, int tid, const f32x4 (&r)[T
   }
 }
 
-// Tile order.  Workgroups are handed to the 8 XCDs round-robin (linear id
-// L on XCD L % 8), and each XCD has its own L2.  XCD x therefore gets the
-// contiguous logical range [x*T/8, (x+1)*T/8) of the T tiles, walked in
-// groups of 8 tile-rows with the columns inside a group, so the workgroups
-// resident on one XCD share a few A row-panels and B column-panels.  A
-// bijection on [0, T): every tile is still computed by exactly one workgroup.
-constexpr int kXcds = 8, kGroupRows = 8;
 __device__ __forceinline__ void tile_of(int gx, int gy, int& tm, int& tn) {
   const int T = gx * gy;
   const int L = blockIdx.x + gx * blockIdx.y;
@@ -187,18 +93,19 @@ __device__ __forceinline__ void tile_of(int gx, int gy, int& tm, int& tn) {
   tn = in_group / rows;
 }
 
-// VEC: 0 = guarded scalar loads, 1 = guarded float4 loads, 2 = buffer loads.
-// WM x WN MFMA blocks per wave: the workgroup tile is (32 WM) x (32 WN).
-template <int TA, int TB, int VEC, bool COLSUM, int WM, int WN, int KD>
-__global__ __launch_bounds__(NT, KD == 16 ? 3 : 2) void gemm_kernel(GemmArgs g) {
+// The general fp32 MFMA kernel, 64-bit addresses and guarded loads: products
+// that the split-bf16 kernel (gemm_split.hpp) does not take, i.e. an operand of
+// 2 GiB or more, a column sum beside an untransposed A or a transposed B, an
+// empty K.  VEC: 16-byte loads.
+template <int TA, int TB, bool VEC, bool COLSUM>
+__global__ __launch_bounds__(NT, 3) void gemm_kernel(GemmArgs g) {
+  constexpr int WM = 4, WN = 4, KD = 16;
   constexpr bool A_MC = TA != 0;
   constexpr bool B_KC = TB != 0;
   constexpr int TM = 32 * WM, TN = 32 * WN;
   constexpr int ASZ = a_tile_floats<A_MC, TM, KD>();
   constexpr int BSZ = b_tile_floats<B_KC, TN, KD>();
-  constexpr int EPI_LD = 16 * WN + 4;  // epilogue staging row stride (16-byte aligned rows)
-  constexpr int SMEM = 2 * (ASZ + BSZ) > 4 * 32 * EPI_LD ? 2 * (ASZ + BSZ) : 4 * 32 * EPI_LD;
-  __shared__ __attribute__((aligned(16))) float smem[SMEM];
+  __shared__ __attribute__((aligned(16))) float smem[2 * (ASZ + BSZ)];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -214,10 +121,6 @@ __global__ __launch_bounds__(NT, KD == 16 ? 3 : 2) void gemm_kernel(GemmArgs g) 
   float* C = g.C + batch_off(z, g, g.sc, g.sc2);
   const int kbeg = g.grouped ? 0 : split * g.kchunk;
   const int kend = g.grouped ? g.K : min(g.K, kbeg + g.kchunk);
-  const uint32_t a_bytes = (uint32_t)(((int64_t)((A_MC ? g.K : g.M) - 1) * g.lda + (A_MC ? g.M : g.K)) * 4);
-  const uint32_t b_bytes = (uint32_t)(((int64_t)((B_KC ? g.N : g.K) - 1) * g.ldb + (B_KC ? g.K : g.N)) * 4);
-  const BufOperand Ab(A, g.lda, a_bytes), Bb(B, g.ldb, b_bytes);
-
   f32x4 acc[WM][WN];
 #pragma unroll
   for (int i = 0; i < WM; ++i)
@@ -230,8 +133,8 @@ __global__ __launch_bounds__(NT, KD == 16 ? 3 : 2) void gemm_kernel(GemmArgs g) 
   const int nk = kend > kbeg ? (kend - kbeg + KD - 1) / KD : 0;
   f32x4 ra[TM * KD / 1024], rb[TN * KD / 1024];
   if (nk > 0) {
-    load_a<A_MC, VEC, TM, KD>(g, A, Ab, m0, kbeg, kend, tid, ra);
-    load_b<B_KC, VEC, TN, KD>(g, B, Bb, n0, kbeg, kend, tid, rb);
+    load_a<A_MC, VEC, TM, KD>(g, A, m0, kbeg, kend, tid, ra);
+    load_b<B_KC, VEC, TN, KD>(g, B, n0, kbeg, kend, tid, rb);
     store_tile<!A_MC, TM, KD>(smem, tid, ra);
     store_tile<B_KC, TN, KD>(smem + 2 * ASZ, tid, rb);
   }
@@ -243,8 +146,8 @@ __global__ __launch_bounds__(NT, KD == 16 ? 3 : 2) void gemm_kernel(GemmArgs g) 
     const float* Bs = smem + 2 * ASZ + cur * BSZ;
     const bool more = kt + 1 < nk;
     if (more) {
-      load_a<A_MC, VEC, TM, KD>(g, A, Ab, m0, kbeg + (kt + 1) * KD, kend, tid, ra);
-      load_b<B_KC, VEC, TN, KD>(g, B, Bb, n0, kbeg + (kt + 1) * KD, kend, tid, rb);
+      load_a<A_MC, VEC, TM, KD>(g, A, m0, kbeg + (kt + 1) * KD, kend, tid, ra);
+      load_b<B_KC, VEC, TN, KD>(g, B, n0, kbeg + (kt + 1) * KD, kend, tid, rb);
     }
     mma_stage<A_MC, B_KC, WM, WN, KD>(As, Bs, acc, wm, wn, lr, q);
     if (do_cs) {
@@ -265,45 +168,7 @@ __global__ __launch_bounds__(NT, KD == 16 ? 3 : 2) void gemm_kernel(GemmArgs g) 
   const float alpha = g.alpha, beta = g.beta;
   const bool split_mode = g.splits > 1;
   float* P = split_mode ? g.part + (int64_t)blockIdx.z * g.M * g.N : nullptr;
-  if (VEC == 2 && (g.N & 3) == 0 && (g.ldc & 3) == 0 && ((reinterpret_cast<uintptr_t>(C) & 15) == 0)) {
-    // Stage each wave's (16 WM) x (16 WN) block through LDS, 32 rows at a
-    // time, and write rows back with 16-byte stores.
-    constexpr int F4_ROW = 4 * WN;          // float4 per staged row
-    constexpr int ROWS_PASS = 64 / F4_ROW;  // rows a wave writes per pass
-    float* T = smem + wave * (32 * EPI_LD);
-#pragma unroll
-    for (int half = 0; half < WM / 2; ++half) {
-#pragma unroll
-      for (int ii = 0; ii < 2; ++ii) {
-        const int i = half * 2 + ii;
-#pragma unroll
-        for (int n = 0; n < WN; ++n)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) T[(ii * 16 + 4 * q + r) * EPI_LD + n * 16 + lr] = acc[i][n][r];
-      }
-      __syncthreads();
-#pragma unroll
-      for (int it = 0; it < 32 / ROWS_PASS; ++it) {
-        const int rr = it * ROWS_PASS + lane / F4_ROW;
-        const int cc = (lane % F4_ROW) * 4;
-        const int row = m0 + wm * 16 * WM + half * 32 + rr;
-        const int col = n0 + wn * 16 * WN + cc;
-        if (row < g.M && col < g.N) {
-          f32x4 v = *reinterpret_cast<const f32x4*>(T + rr * EPI_LD + cc);
-          if (split_mode) {
-            *reinterpret_cast<f32x4*>(P + (int64_t)row * g.N + col) = v;
-          } else {
-            float* p = C + (int64_t)row * g.ldc + col;
-            v = alpha * v;
-            if (beta != 0.f) v += beta * *reinterpret_cast<const f32x4*>(p);
-            if (g.bias) v += *reinterpret_cast<const f32x4*>(g.bias + z * g.sbias + col);
-            *reinterpret_cast<f32x4*>(p) = v;
-          }
-        }
-      }
-      __syncthreads();
-    }
-  } else {
+  {
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -342,505 +207,6 @@ __global__ __launch_bounds__(NT, KD == 16 ? 3 : 2) void gemm_kernel(GemmArgs g) 
   }
 }
 
-// Register-direct variant for 128 x 128 tiles: no LDS and no barrier.  Each
-// lane loads its own MFMA fragments from global memory with 16-byte reads,
-// D - 1 K stages (KD deep each) ahead of the MFMAs, through D register sets.
-// Within a stage, lane group q = lane / 16 feeds k = (KD/4) q + j to MFMA
-// step j (j < KD/4); A and B use the same k permutation, so the contraction
-// is unchanged.
-//  * an operand stored k-contiguous gives lane (lr, q) KD/4 consecutive k
-//    values of one row (column) in KD/16 loads per 16-row block; with KD = 32
-//    the four lane groups cover a full 128-byte line of each row per stage;
-//  * an operand stored m- (or n-) contiguous is read along m instead: one
-//    load of 4 consecutive rows at k = (KD/4) q + j holds that lane's values
-//    for all four blocks (one load per MFMA step j).
-// Rows and columns inside the wave's 64 x 64 block are permuted so that
-// every lane ends with 4 consecutive C columns per row: block n, lane column
-// c is column 4c + n for both B layouts, and block i, accumulator row d is
-// row 4d + i (A m-contiguous) or 16i + d (A k-contiguous).  The epilogue
-// therefore writes 16-byte row segments straight from the accumulators.
-// A wave issues KD/4 loads per operand per stage; the two waves that share a
-// row (column) panel hit the same lines, which the L1 serves.
-// One 128 x 128 tile (tm, tn) of batch item / split bz of the register-direct
-// kernel; shared by gemm_direct_kernel and gemm_pair_kernel.
-template <int TA, int TB, bool COLSUM, int KD, int D, bool TERMS>
-__device__ __forceinline__ void direct_tile(const GemmArgs& g, int tm, int tn, int bz) {
-  constexpr bool A_MC = TA != 0;
-  constexpr bool B_KC = TB != 0;
-  constexpr int TM = 128, TN = 128;
-  constexpr int S = KD / 4;   // MFMA steps (and loads per operand) per stage
-  constexpr int H = KD / 16;  // loads per 16-row block of a k-contiguous operand
-  static_assert(D >= 2 && (KD == 16 || KD == 32), "unsupported stage shape");
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int lr = lane & 15, q = lane >> 4;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int m0 = tm * TM + wm * 64, n0 = tn * TN + wn * 64;  // this wave's 64 x 64 block
-  const int64_t z = bz / g.splits;
-  const int split = bz % g.splits;
-  const float* A = g.A + batch_off(z, g, g.sa, g.sa2) + (g.grouped ? split * g.gsa : 0);
-  const float* B = g.B + batch_off(z, g, g.sb, g.sb2) + (g.grouped ? split * g.gsb : 0);
-  float* C = g.C + batch_off(z, g, g.sc, g.sc2);
-  const int kbeg = g.grouped ? 0 : split * g.kchunk;
-  const int kend = g.grouped ? g.K : min(g.K, kbeg + g.kchunk);
-  // With TERMS the resources span every term (the host checks the extent).
-  const int64_t a_terms = TERMS ? (int64_t)(g.kterms - 1) * g.gsa : 0;
-  const int64_t b_terms = TERMS ? (int64_t)(g.kterms - 1) * g.gsb : 0;
-  const uint32_t a_bytes =
-      (uint32_t)((a_terms + (int64_t)((A_MC ? g.K : g.M) - 1) * g.lda + (A_MC ? g.M : g.K)) * 4);
-  const uint32_t b_bytes =
-      (uint32_t)((b_terms + (int64_t)((B_KC ? g.N : g.K) - 1) * g.ldb + (B_KC ? g.K : g.N)) * 4);
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), (short)0, (int)a_bytes, kBufWord3);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), (short)0, (int)b_bytes, kBufWord3);
-  const int nkt = kend > kbeg ? (kend - kbeg + KD - 1) / KD : 0;  // stages per term
-  const int nk = TERMS ? g.kterms * nkt : nkt;
-
-  // Byte offsets at k = kbeg of the S loads per operand, and the per-stage
-  // advance.  K and the split's chunk are multiples of KD (checked on the
-  // host), so every stage is full.  A row (column) outside the matrix starts
-  // at kBufOOB, past the buffer's extent; the hardware range check returns
-  // zeros for it, and its products only reach C rows (columns) that are never
-  // stored.  Stages fetched past the end of K (up to D - 1) are never
-  // consumed; a buffer load never faults, whatever its offset.
-  const int kq = kbeg + S * q;  // first k of this lane group
-  uint32_t a_off[S], b_off[S];
-#pragma unroll
-  for (int x = 0; x < S; ++x) {
-    if (!A_MC) {  // x = (block i, half h): row m0 + 16 i + lr, k = kq + 4 h
-      const int row = m0 + 16 * (x / H) + lr;
-      a_off[x] = row < g.M ? (uint32_t)(row * (int)g.lda + kq + 4 * (x % H)) * 4u : kBufOOB;
-    } else {  // x = step j: k = kq + x, rows m0 + 4 lr .. + 3
-      a_off[x] = m0 + 4 * lr < g.M ? (uint32_t)((kq + x) * (int)g.lda + m0 + 4 * lr) * 4u : kBufOOB;
-    }
-    if (B_KC) {  // x = (block n, half h): column n0 + 4 lr + n, k = kq + 4 h
-      const int col = n0 + 4 * lr + x / H;
-      b_off[x] = col < g.N ? (uint32_t)(col * (int)g.ldb + kq + 4 * (x % H)) * 4u : kBufOOB;
-    } else {  // x = step j: k = kq + x, columns n0 + 4 lr .. + 3
-      b_off[x] = n0 + 4 * lr < g.N ? (uint32_t)((kq + x) * (int)g.ldb + n0 + 4 * lr) * 4u : kBufOOB;
-    }
-  }
-  const uint32_t a_step = 4u * (A_MC ? KD * (uint32_t)g.lda : KD);
-  const uint32_t b_step = 4u * (B_KC ? KD : KD * (uint32_t)g.ldb);
-
-  // Terms: stage kt is stage kt % nkt of term kt / nkt, so the offset jumps
-  // by (term stride - nkt stages) at each term boundary (modulo 2^32; the
-  // true offsets stay below 2^31, OOB rows included).  Stages prefetched past
-  // the last term are never consumed.
-  const uint32_t a_jump = TERMS ? (uint32_t)(g.gsa * 4) - (uint32_t)nkt * a_step : 0u;
-  const uint32_t b_jump = TERMS ? (uint32_t)(g.gsb * 4) - (uint32_t)nkt * b_step : 0u;
-  auto load = [&](int kt, f32x4(&fa)[S], f32x4(&fb)[S]) {
-    uint32_t da = (uint32_t)kt * a_step, db = (uint32_t)kt * b_step;
-    if (TERMS) {
-      const uint32_t t = (uint32_t)min(kt / nkt, g.kterms - 1);
-      da += t * a_jump;
-      db += t * b_jump;
-    }
-#pragma unroll
-    for (int x = 0; x < S; ++x) {
-      fa[x] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(a_off[x] + da), 0, 0));
-      fb[x] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, (int)(b_off[x] + db), 0, 0));
-    }
-  };
-
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int n = 0; n < 4; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const bool do_cs = COLSUM && tm == 0 && wm == 0;
-  float csum[4] = {0.f, 0.f, 0.f, 0.f};  // per lane: partial sums of columns 4 lr + n
-
-  // Operand value of (block i or n, step j).
-  auto av = [&](const f32x4(&fa)[S], int i, int j) { return A_MC ? fa[j][i] : fa[i * H + j / 4][j % 4]; };
-  auto bv = [&](const f32x4(&fb)[S], int n, int j) { return B_KC ? fb[n * H + j / 4][j % 4] : fb[j][n]; };
-  auto mfma = [&](const f32x4(&fa)[S], const f32x4(&fb)[S]) {
-#pragma unroll
-    for (int j = 0; j < S; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int n = 0; n < 4; ++n)
-          acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(av(fa, i, j), bv(fb, n, j), acc[i][n], 0, 0, 0);
-    if (do_cs) {
-#pragma unroll
-      for (int n = 0; n < 4; ++n)
-#pragma unroll
-        for (int j = 0; j < S; ++j) csum[n] += bv(fb, n, j);
-    }
-  };
-
-  // The epilogue's bias, loaded before the K loop so that its wait is long
-  // satisfied when the stores start (loaded after the loop, it cost the
-  // epilogue a memory round trip).  A column past N, or no bias, reads 0.
-  const bool split_mode = g.splits > 1;
-  const int col = n0 + 4 * lr;
-  f32x4 b4;
-  {
-    const bool has_b = !split_mode && g.bias;
-    const __amdgpu_buffer_rsrc_t rbias = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(has_b ? g.bias + z * g.sbias : nullptr), (short)0, has_b ? g.N * 4 : 0, kBufWord3);
-    b4 = __builtin_bit_cast(
-        f32x4, __builtin_amdgcn_raw_buffer_load_b128(rbias, (int)(col < g.N ? (uint32_t)col * 4u : kBufOOB), 0, 0));
-  }
-
-  // Stage s lives in register set s % D.  Each pass of the loop consumes D
-  // stages and issues the loads D - 1 stages ahead of each.
-  f32x4 fa[D][S], fb[D][S];
-#pragma unroll
-  for (int s = 0; s < D - 1; ++s) load(s, fa[s], fb[s]);
-  int kt = 0;
-  for (; kt + D - 1 < nk; kt += D) {
-#pragma unroll
-    for (int s = 0; s < D; ++s) {
-      load(kt + s + D - 1, fa[(s + D - 1) % D], fb[(s + D - 1) % D]);
-      __builtin_amdgcn_sched_barrier(0);
-      mfma(fa[s], fb[s]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-  // Fewer than D stages remain, all of them already loaded (sets 0 .. D - 2).
-#pragma unroll
-  for (int s = 0; s < D - 1; ++s)
-    if (kt + s < nk) mfma(fa[s], fb[s]);
-
-  // Epilogue: lane (lr, q) holds C[row(i, 4q + r)][4 lr + n] in acc[i][n][r],
-  // so each (i, r) is one 16-byte store of 4 consecutive columns.  N, ldc and
-  // C are 16-byte aligned on this path (checked on the host).
-  float* P = split_mode ? g.part + (int64_t)bz * g.M * g.N : nullptr;
-  auto rmap = [&](int i, int d) { return A_MC ? 4 * d + i : 16 * i + d; };
-  if (col < g.N) {
-    const float alpha = g.alpha, beta = g.beta;
-    // beta != 0: every previous value is loaded before the first store (the
-    // vector memory counter counts stores too, so loading each one between
-    // two stores made every store wait for the one before).
-    f32x4 old[4][4];
-    if (!split_mode && beta != 0.f) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = m0 + rmap(i, 4 * q + r);
-          old[i][r] = row < g.M ? *reinterpret_cast<const f32x4*>(C + (int64_t)row * g.ldc + col)
-                                : f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + rmap(i, 4 * q + r);
-        if (row < g.M) {
-          f32x4 v = {acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]};
-          if (split_mode) {
-            *reinterpret_cast<f32x4*>(P + (int64_t)row * g.N + col) = v;
-          } else {
-            float* p = C + (int64_t)row * g.ldc + col;
-            v = alpha * v;
-            if (beta != 0.f) v += beta * old[i][r];
-            *reinterpret_cast<f32x4*>(p) = v + b4;
-          }
-        }
-      }
-  }
-  if (do_cs) {
-    // lanes lr + 16 q hold partial sums of the same 4 columns: fixed-order
-    // reduction over q, then lane q == 0 owns columns col .. col + 3.
-#pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      float v = csum[n];
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
-      csum[n] = v;
-    }
-    if (q == 0 && col < g.N) {
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        if (split_mode) g.part_cs[(int64_t)bz * g.N + col + n] = csum[n];
-        else put_colsum(g, z * g.scs + col + n, csum[n]);
-      }
-    }
-  }
-}
-
-// Tile (tm, tn) and batch item z of work item L of a launch over `items` =
-// gx * gy * batch tiles.  The same XCD-aware order as tile_of: item L runs on
-// XCD L % 8 (workgroups are dispatched round-robin), XCD x owns a contiguous
-// logical range, walked in groups of 8 tile-rows per batch item.  A bijection
-// on [0, items).
-__device__ __forceinline__ void item_tile(int L, int items, int gx, int gy, int& tm, int& tn, int& z) {
-  const int q = items / kXcds, r = items % kXcds, x = L % kXcds;
-  const int logical = x * q + min(x, r) + L / kXcds;
-  const int T = gx * gy;
-  z = logical / T;
-  const int t = logical - z * T;
-  const int per_group = kGroupRows * gx;
-  const int grp = t / per_group;
-  const int first_m = grp * kGroupRows;
-  const int rows = min(gy - first_m, kGroupRows);
-  const int in_group = t - grp * per_group;
-  tm = first_m + in_group % rows;
-  tn = in_group / rows;
-}
-
-// One tile per workgroup.  The tile and the batch item / K split come from
-// the workgroup's linear id over the whole grid (x, then y, then z), so each
-// XCD gets a contiguous range that stays within one split: the column tiles
-// that share an A row panel share that XCD's L2 (with z walked per slice,
-// every XCD read every panel of a split -- 3.6x the algorithmic bytes for a
-// 2048 x 512 x 8192 weight gradient in 4 splits).
-template <int TA, int TB, bool COLSUM, int KD, int D, int OCC, bool TERMS = false>
-__global__ __launch_bounds__(NT, OCC) void gemm_direct_kernel(GemmArgs g) {
-  int tm, tn, z;
-  const int L = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
-  item_tile(L, (int)(gridDim.x * gridDim.y * gridDim.z), gridDim.x, gridDim.y, tm, tn, z);
-  direct_tile<TA, TB, COLSUM, KD, D, TERMS>(g, tm, tn, z);
-}
-
-// Persistent register-direct GEMM for grids of more 128 x 128 tiles than two
-// per CU: two workgroups per CU walk work items L = blockIdx.x + j * gridDim.x.
-// Each wave computes its 64 x 64 block of a tile exactly as
-// gemm_direct_kernel does (same fragment loads, same MFMA order, so the same
-// bits).  The operand loads run D - 1 stages ahead straight across tile
-// boundaries: in the last D stages of a tile they fetch the next tile's first
-// D - 1 stages (offsets selected without branches), so a new tile starts with
-// its operands in registers instead of waiting for a prologue, and no
-// workgroup is launched or retired per tile.  One loop with a straight-line
-// body: every pass issues the same loads in the same places, so the
-// compiler's load waits stay tight.  At a tile boundary the wave writes its
-// block from the accumulators through a buffer resource (elements outside
-// the matrix get offset kBufOOB: the store is dropped, a read returns zeros);
-// those stores are issued after the next tile's first loads, so the waits
-// for those loads never include them.
-// Measured on MI355X against the per-tile launch of gemm_direct_kernel:
-// equal or faster on every C4 shape with more than 512 tiles (LM-head
-// forward 604 -> 581 us, 8192 x 2048 x 512 NT 150 -> 135 us).  A variant
-// with one workgroup per CU and a fifth wave writing C from an LDS staging
-// tile was slower (one compute wave per SIMD hides less load latency).
-// Requires: one split, no column sum, K a positive multiple of KD * D, C
-// addressable by a buffer resource, and the direct kernel's alignment
-// conditions (checked on the host).
-template <int TA, int TB, int KD, int D, int EPI = kEpiPlain, int ACT = 0>
-__global__ __launch_bounds__(NT, 2) void gemm_stream_kernel(GemmArgs g, int gx, int gy, int items) {
-  constexpr bool ROWSTATS = EPI == kEpiRowstats;
-  constexpr bool A_MC = TA != 0;
-  constexpr bool B_KC = TB != 0;
-  constexpr int S = KD / 4;   // MFMA steps (and loads per operand) per stage
-  constexpr int H = KD / 16;  // loads per 16-row block of a k-contiguous operand
-  static_assert(D >= 2 && (KD == 16 || KD == 32), "unsupported stage shape");
-  constexpr int kRsLd = 64 + 4;  // ROWSTATS staging row stride (floats)
-  __shared__ __attribute__((aligned(16))) float rs_lds[ROWSTATS ? 4 * 64 * kRsLd : 4];
-
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
-  const int G = gridDim.x;
-
-  const int lr = lane & 15, q = lane >> 4;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int nk = g.K / KD;
-  const uint32_t a_bytes = (uint32_t)(((int64_t)((A_MC ? g.K : g.M) - 1) * g.lda + (A_MC ? g.M : g.K)) * 4);
-  const uint32_t b_bytes = (uint32_t)(((int64_t)((B_KC ? g.N : g.K) - 1) * g.ldb + (B_KC ? g.K : g.N)) * 4);
-  const uint32_t a_step = 4u * (A_MC ? KD * (uint32_t)g.lda : KD);
-  const uint32_t b_step = 4u * (B_KC ? KD : KD * (uint32_t)g.ldb);
-  const uint32_t c_bytes = (uint32_t)(((int64_t)(g.M - 1) * g.ldc + g.N) * 4);
-
-  // Buffer resources and this lane's byte offsets at stage 0 of an item (the
-  // direct kernel's offsets with kbeg = 0).  Past the last item the first
-  // item is decoded and every offset becomes kBufOOB, so those (never
-  // consumed) loads return zeros.
-  auto locate = [&](int L, __amdgpu_buffer_rsrc_t& ra, __amdgpu_buffer_rsrc_t& rb, uint32_t(&ao)[S],
-                    uint32_t(&bo)[S]) {
-    const bool live = L < items;
-    int tm, tn, z;
-    item_tile(live ? L : (int)blockIdx.x, items, gx, gy, tm, tn, z);
-    const float* A = g.A + batch_off(z, g, g.sa, g.sa2);
-    const float* B = g.B + batch_off(z, g, g.sb, g.sb2);
-    ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), (short)0, (int)a_bytes, kBufWord3);
-    rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), (short)0, (int)b_bytes, kBufWord3);
-    const int m0 = tm * 128 + wm * 64, n0 = tn * 128 + wn * 64;
-    const int kq = S * q;
-#pragma unroll
-    for (int x = 0; x < S; ++x) {
-      if (!A_MC) {
-        const int row = m0 + 16 * (x / H) + lr;
-        ao[x] = live && row < g.M ? (uint32_t)(row * (int)g.lda + kq + 4 * (x % H)) * 4u : kBufOOB;
-      } else {
-        ao[x] = live && m0 + 4 * lr < g.M ? (uint32_t)((kq + x) * (int)g.lda + m0 + 4 * lr) * 4u : kBufOOB;
-      }
-      if (B_KC) {
-        const int col = n0 + 4 * lr + x / H;
-        bo[x] = live && col < g.N ? (uint32_t)(col * (int)g.ldb + kq + 4 * (x % H)) * 4u : kBufOOB;
-      } else {
-        bo[x] = live && n0 + 4 * lr < g.N ? (uint32_t)((kq + x) * (int)g.ldb + n0 + 4 * lr) * 4u : kBufOOB;
-      }
-    }
-  };
-  __amdgpu_buffer_rsrc_t ra, rb, ra_n, rb_n;  // current and next item
-  uint32_t a_off[S], b_off[S], a_nx[S], b_nx[S];
-  locate(blockIdx.x, ra, rb, a_off, b_off);
-  locate(blockIdx.x + G, ra_n, rb_n, a_nx, b_nx);
-
-  // Stage ks of the current item, or stage kn of the next one when `nxt`.
-  auto load = [&](bool nxt, int ks, int kn, f32x4(&fa)[S], f32x4(&fb)[S]) {
-    const __amdgpu_buffer_rsrc_t xa = nxt ? ra_n : ra, xb = nxt ? rb_n : rb;
-    const uint32_t da = (uint32_t)(nxt ? kn : ks) * a_step, db = (uint32_t)(nxt ? kn : ks) * b_step;
-#pragma unroll
-    for (int x = 0; x < S; ++x) {
-      const uint32_t oa = (nxt ? a_nx[x] : a_off[x]) + da, ob = (nxt ? b_nx[x] : b_off[x]) + db;
-      fa[x] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xa, (int)oa, 0, 0));
-      fb[x] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xb, (int)ob, 0, 0));
-    }
-  };
-
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int n = 0; n < 4; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto av = [&](const f32x4(&fa)[S], int i, int j) { return A_MC ? fa[j][i] : fa[i * H + j / 4][j % 4]; };
-  auto bv = [&](const f32x4(&fb)[S], int n, int j) { return B_KC ? fb[n * H + j / 4][j % 4] : fb[j][n]; };
-  auto mfma = [&](const f32x4(&fa)[S], const f32x4(&fb)[S]) {
-#pragma unroll
-    for (int j = 0; j < S; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int n = 0; n < 4; ++n)
-          acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(av(fa, i, j), bv(fb, n, j), acc[i][n], 0, 0, 0);
-  };
-
-  // Stage kt of every item lives in register set kt % D (nk is a multiple of
-  // D, so each item starts at set 0).
-  f32x4 fa[D][S], fb[D][S];
-#pragma unroll
-  for (int s = 0; s < D - 1; ++s) load(false, s, 0, fa[s], fb[s]);
-  int kt = 0, c_item = blockIdx.x;
-  // The epilogue's bias, loaded ahead of the item's last D stages: issued
-  // before the next item's first loads, its wait in the epilogue does not
-  // cover them (the vector memory counter completes in order).  A column
-  // past N, or no bias, reads 0.
-  f32x4 b4 = {0.f, 0.f, 0.f, 0.f};
-  for (;;) {
-    const bool last = kt + D == nk;  // the item's last D stages
-    if (last) {
-      int tm, tn, z;
-      item_tile(c_item, items, gx, gy, tm, tn, z);
-      const int col = tn * 128 + wn * 64 + 4 * lr;
-      const __amdgpu_buffer_rsrc_t rbias = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<float*>(g.bias ? g.bias + z * g.sbias : g.bias), (short)0, g.bias ? g.N * 4 : 0, kBufWord3);
-      b4 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rbias, (int)(col < g.N ? (uint32_t)col * 4u : kBufOOB), 0, 0));
-    }
-#pragma unroll
-    for (int s = 0; s < D; ++s) {
-      const int ls = kt + s + D - 1;  // stage to fetch; past nk it is the next item's
-      load(s > 0 && last, ls, ls - nk, fa[(s + D - 1) % D], fb[(s + D - 1) % D]);
-      __builtin_amdgcn_sched_barrier(0);
-      mfma(fa[s], fb[s]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (!last) {
-      kt += D;
-      continue;
-    }
-    {
-      // Epilogue: lane (lr, q) holds C[row(i, 4q + r)][4 lr + n] of the
-      // wave's block in acc[i][n][r] (the direct kernel's permutation), so
-      // each (i, r) is one 16-byte store of 4 consecutive columns.
-      int tm, tn, z;
-      item_tile(c_item, items, gx, gy, tm, tn, z);
-      float* C = g.C + batch_off(z, g, g.sc, g.sc2);
-      const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(C, (short)0, (int)c_bytes, kBufWord3);
-      // Activation operands share C's layout (and batch offsets).
-      const int64_t zc = batch_off(z, g, g.sc, g.sc2);
-      __amdgpu_buffer_rsrc_t ry = rc, rx = rc, rd = rc;
-      if (EPI == kEpiActFwd) ry = __builtin_amdgcn_make_buffer_rsrc(g.act_y + zc, (short)0, (int)c_bytes, kBufWord3);
-      if (EPI == kEpiActBwd) {
-        rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(g.act_x) + zc, (short)0, (int)c_bytes, kBufWord3);
-        rd = __builtin_amdgcn_make_buffer_rsrc(g.act_dx + zc, (short)0, (int)c_bytes, kBufWord3);
-      }
-      const int m0 = tm * 128 + wm * 64, col = tn * 128 + wn * 64 + 4 * lr;
-      const float alpha = g.alpha, beta = g.beta;
-      // ROWSTATS: the wave's 64 x 64 block goes to LDS (row slot
-      // d' = 16 i + 4 q + r, columns outside the matrix as -FLT_MAX), then lane
-      // l reduces slot l's 64 columns to (max, sum of exp(x - max)).
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = m0 + (A_MC ? 4 * (4 * q + r) + i : 16 * i + 4 * q + r);
-          const uint32_t off = row < g.M && col < g.N ? (uint32_t)(row * (int)g.ldc + col) * 4u : kBufOOB;
-          f32x4 v = {acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]};
-          v = alpha * v;
-          if (beta != 0.f)
-            v += beta * __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rc, (int)off, 0, 0));
-          v += b4;
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, v),
-                                                 rc, (int)off, 0, 0);
-          if (EPI == kEpiActFwd) {
-            f32x4 y;
-#pragma unroll
-            for (int n = 0; n < 4; ++n) y[n] = act_f<ACT>(v[n]);
-            __builtin_amdgcn_raw_buffer_store_b128(
-                __builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, y), ry, (int)off, 0, 0);
-          }
-          if (EPI == kEpiActBwd) {
-            const f32x4 xh = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)off, 0, 0));
-            f32x4 old = {0.f, 0.f, 0.f, 0.f};
-            if (g.act_acc) old = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rd, (int)off, 0, 0));
-            f32x4 d;  // the elementwise backward's bits: the product rounded before the add
-#pragma unroll
-            for (int n = 0; n < 4; ++n) d[n] = act_bwd_k<ACT>(xh[n], v[n], old[n], g.act_acc);
-            __builtin_amdgcn_raw_buffer_store_b128(
-                __builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, d), rd, (int)off, 0, 0);
-          }
-          if (ROWSTATS) {
-#pragma unroll
-            for (int n = 0; n < 4; ++n)
-              if (col + n >= g.N) v[n] = -FLT_MAX;
-            *reinterpret_cast<f32x4*>(rs_lds + (wave * 64 + 16 * i + 4 * q + r) * kRsLd + 4 * lr) = v;
-          }
-        }
-      if (ROWSTATS) {
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        const float* rp = rs_lds + (wave * 64 + lane) * kRsLd;
-        f32x4 x[16];
-#pragma unroll
-        for (int c = 0; c < 16; ++c) x[c] = *reinterpret_cast<const f32x4*>(rp + 4 * c);
-        float m = -FLT_MAX;
-#pragma unroll
-        for (int c = 0; c < 16; ++c) m = fmaxf(fmaxf(m, fmaxf(x[c][0], x[c][1])), fmaxf(x[c][2], x[c][3]));
-        float e = 0.f;
-#pragma unroll
-        for (int c = 0; c < 16; ++c)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) e += __expf(x[c][j] - m);
-        const int i = lane >> 4, d = lane & 15;
-        const int row = m0 + (A_MC ? 4 * d + i : 16 * i + d);
-        const int c0 = tn * 128 + wn * 64;  // this wave's 64-column block
-        if (row < g.M && c0 < g.N)
-          *reinterpret_cast<float2*>(g.rowpart + (int64_t)row * g.rp_ld + 2 * (c0 >> 6)) = make_float2(m, e);
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int n = 0; n < 4; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-    c_item += G;
-    if (c_item >= items) break;
-    kt = 0;
-    ra = ra_n;
-    rb = rb_n;
-#pragma unroll
-    for (int x = 0; x < S; ++x) {
-      a_off[x] = a_nx[x];
-      b_off[x] = b_nx[x];
-    }
-    locate(c_item + G, ra_n, rb_n, a_nx, b_nx);
-  }
-}
-
 // Row statistics of a finished C when the GEMM did not produce them in its
 // epilogue: one wave per (row, 64-column block): max and sum of exp(C - max).
 __global__ __launch_bounds__(256) void rowstats_kernel(const float* __restrict__ C, int64_t ldc, int M, int N,
@@ -858,35 +224,6 @@ __global__ __launch_bounds__(256) void rowstats_kernel(const float* __restrict__
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
   if (lane == 0) *reinterpret_cast<float2*>(part + (int64_t)row * ld + 2 * blk) = make_float2(m, e);
-}
-
-// Two independent register-direct GEMMs in one launch, one tile per
-// workgroup: workgroups [0, items0) take problem 0 and the rest problem 1,
-// each tile decoded by item_tile and computed by direct_tile exactly as
-// gemm_direct_kernel computes it.  A Linear layer's dX and dW products
-// (Engine/engine.cu:3553-3560) usually each fill about one workgroup per CU
-// with work items of equal depth; launched together they run two per CU in
-// a single round.
-// Problem 1 starts at workgroup start1, items0 rounded up to a multiple of 8
-// (the workgroups between do nothing), so that its item L runs on XCD L % 8
-// as item_tile assumes.
-struct PairGrid {
-  int items0, gx0, gy0;
-  int items1, gx1, gy1;
-  int start1;
-};
-
-template <int TA0, int TB0, bool CS0, bool T0, int TA1, int TB1, bool CS1, bool T1>
-__global__ __launch_bounds__(NT, 2) void gemm_pair_kernel(GemmArgs g0, GemmArgs g1, PairGrid pg) {
-  const int w = blockIdx.x;
-  int tm, tn, bz;
-  if (w < pg.items0) {
-    item_tile(w, pg.items0, pg.gx0, pg.gy0, tm, tn, bz);
-    direct_tile<TA0, TB0, CS0, 16, 3, T0>(g0, tm, tn, bz);
-  } else if (w >= pg.start1) {
-    item_tile(w - pg.start1, pg.items1, pg.gx1, pg.gy1, tm, tn, bz);
-    direct_tile<TA1, TB1, CS1, 16, 3, T1>(g1, tm, tn, bz);
-  }
 }
 
 // C = alpha * sum_s part[s] + beta * C (+ bias) and colsum (+)= sum_s
@@ -1212,131 +549,77 @@ __global__ __launch_bounds__(64 * NW) void gemm_ksplit_pair_kernel(GemmArgs g0, 
   }
 }
 
-// Workgroup tile: 128 x 128 unless a side is <= 64 (the 64-wide variants waste
-// nothing there) or the 128 x 128 grid would leave CUs idle and K is too short
-// for split-K to fill them (half-width tiles double the workgroups; measured
-// on MI355X, for K >= 4096 full tiles plus split-K are faster).  A function of
-// the shape only, as mle_gemm_ws_bytes needs.
-struct Tile {
-  int wm, wn;         // MFMA blocks per wave along M / N
-  int kd = 32;        // K depth of a stage
-  bool direct = false;  // register-direct kernel (128 x 128, no LDS in the K loop)
-  int tm() const { return 32 * wm; }
-  int tn() const { return 32 * wn; }
+// Tile and K splits of a product on the split kernel: the cheapest by a model
+// of its time in us -- rounds of workgroups times (stages x time of a stage +
+// prologue and epilogue), plus the reduce of the partial products.  A function
+// of the shape only, as mle_gemm_ws_bytes needs.
+//
+// Measured on MI355X under sustained load, us per stage and per tile beside
+// them, a whole round of 256 workgroups: large 2.6 + 8.5 (2.3 in short runs,
+// before the power limit lowers the clock), medium 1.75 + 6, small 0.75 + 4.5
+// alone on a CU and 0.55 + 3 a piece when three share it.
+constexpr double kStageUs[3] = {2.6, 1.75, 0.75}, kTileUs[3] = {8.5, 6.0, 4.5};
+constexpr double kSharedStageUs = 0.55, kSharedTileUs = 3.0;
+constexpr int kChipCus = 256;
+
+struct SplitChoice {
+  int tile = kSplitLarge, splits = 1, kchunk = 0;
+  double us = 0;
 };
 
-Tile choose_tile(int M, int N, int K, int batch) {
-  (void)K;
-  if (M <= 64 && N <= 64) return {2, 2};
-  if (N <= 64) return {4, 2};
-  if (M <= 64) return {2, 4};
-  const long long t128 = (long long)((M + 127) / 128) * ((N + 127) / 128) * batch;
-  if (t128 >= 192 || K >= 4096) return {4, 4, 16, true};
-  return N >= M ? Tile{2, 4} : Tile{4, 2};
+long long tiles_of(int tile, int M, int N) {
+  return (long long)((M + kSplitTm[tile] - 1) / kSplitTm[tile]) * ((N + kSplitTn[tile] - 1) / kSplitTn[tile]);
 }
 
-// Split count: a function of the shape only.  Splits are used when the tile
-// grid leaves most of the 256 CUs idle and K is long enough to share.
-int choose_splits(int M, int N, int K, int batch, int& kchunk) {
-  kchunk = K;
-  const Tile t = choose_tile(M, N, K, batch);
-  const long long tiles = (long long)((M + t.tm() - 1) / t.tm()) * ((N + t.tn() - 1) / t.tn()) * batch;
-  int s, smax;
-  if (t.direct) {
-    // A grid of >= 3/4 of the 256 CUs runs unsplit.  Below that, at most one
-    // workgroup per CU: a few CUs running two would take twice as long as the
-    // rest (measured on MI355X: 48 tiles x 8192 deep, 5 splits 113 us against
-    // 176 us for 6 and 122 us for 10; 16 tiles: 16 splits best, 64 tiles: 4).
-    if (tiles >= 192) return 1;
-    s = tiles <= 128 ? (int)(256 / tiles) : 2;
-    smax = K / 512;
-  } else {
-    // Measured on MI355X: with ~256 tiles a split only pays off for long K.
-    // A grid of a few tiles is latency-bound (each split walks its K chunk one
-    // stage after another), so it takes chunks down to one 32-deep stage: the
-    // C1 MLP step went from 0.136 to 0.118 ms with 64-deep chunks, and from
-    // 0.065 to 0.057 ms with 32-deep ones (K / 128 or fewer splits: slower).
-    if (tiles >= 384 || (tiles >= 128 && K < 4096)) return 1;
-    s = (int)((768 + tiles - 1) / tiles);
-    smax = tiles <= 16 ? K / 16 : K / 256;
-  }
-  if (s > smax) s = smax;
-  if (s < 2) return 1;
-  kchunk = (K + s - 1) / s;
-  kchunk = ((kchunk + 31) / 32) * 32;  // whole stages of either depth
-  s = (K + kchunk - 1) / kchunk;
-  if ((long long)s * batch > 65535) return 1;
-  return s;
+// Time of n workgroups of `stages` stages each on tile shape `tile`.
+double grid_us(int tile, long long n, int stages) {
+  const long long per = (n + kChipCus - 1) / kChipCus;  // workgroups per CU
+  const double alone = stages * kStageUs[tile] + kTileUs[tile];
+  if (tile != kSplitSmall) return (double)per * alone;
+  return std::max(alone, (double)per * (stages * kSharedStageUs + kSharedTileUs));
 }
 
-template <int TA, int TB, int WM, int WN, int KD>
-void launch_t(hipStream_t s, const GemmArgs& g, dim3 grid, int vec, bool cs) {
-  if (vec == 2) {
-    if (cs) mle::launch(gemm_kernel<TA, TB, 2, true, WM, WN, KD>, grid, NT, 0, s, g);
-    else mle::launch(gemm_kernel<TA, TB, 2, false, WM, WN, KD>, grid, NT, 0, s, g);
-  } else if (vec == 1) {
-    if (cs) mle::launch(gemm_kernel<TA, TB, 1, true, WM, WN, KD>, grid, NT, 0, s, g);
-    else mle::launch(gemm_kernel<TA, TB, 1, false, WM, WN, KD>, grid, NT, 0, s, g);
-  } else {
-    if (cs) mle::launch(gemm_kernel<TA, TB, 0, true, WM, WN, KD>, grid, NT, 0, s, g);
-    else mle::launch(gemm_kernel<TA, TB, 0, false, WM, WN, KD>, grid, NT, 0, s, g);
-  }
-}
-
-// Direct kernel configuration, measured on MI355X over the C3/C4 shapes:
-// 16-deep stages, 3 register sets (2 stages in flight), 2 workgroups per CU.
-// Deeper prefetch (up to 8 sets at 1 workgroup per CU), 32-deep stages and
-// 8-wave 256 x 128 tiles were all equal or slower: the kernel is held by the
-// shader clock it sustains (~2.15 GHz under load), not by load latency.
-template <int TA, int TB>
-void launch_direct(hipStream_t s, const GemmArgs& g, dim3 grid, bool cs) {
-  if (g.kterms > 1) mle::launch(gemm_direct_kernel<TA, TB, false, 16, 3, 2, true>, grid, NT, 0, s, g);
-  else if (cs) mle::launch(gemm_direct_kernel<TA, TB, true, 16, 3, 2>, grid, NT, 0, s, g);
-  else mle::launch(gemm_direct_kernel<TA, TB, false, 16, 3, 2>, grid, NT, 0, s, g);
-}
-
-// Compute units of the current device (queried once per device).
-int cu_count() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] <= 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
-template <int TA, int TB>
-void launch_tile(hipStream_t s, const GemmArgs& g, Tile t, dim3 grid, int vec, bool cs, bool direct_ok) {
-  if (t.direct && direct_ok && vec == 2 && g.K % 16 == 0 && g.kchunk % 16 == 0) {
-    // More tiles than two per CU, one split, no column sum: the persistent
-    // kernel (two workgroups per CU, tiles streamed without per-tile
-    // prologues).
-    const long long items = (long long)grid.x * grid.y * grid.z;
-    const int ncu = cu_count();
-    const bool c_buf = ((double)(g.M - 1) * (double)g.ldc + g.N) * 4.0 < 2147483648.0 - 64;
-    if (g.splits == 1 && g.kterms == 1 && !cs && g.K >= 64 && g.K % 64 == 0 && items > 2 * ncu &&
-        items < (1LL << 30) && c_buf) {
-      if (g.rowpart)
-        mle::launch(gemm_stream_kernel<TA, TB, 16, 4, kEpiRowstats>, dim3((unsigned)(2 * ncu)), NT, 0, s, g,
-                    (int)grid.x, (int)grid.y, (int)items);
-      else
-        mle::launch(gemm_stream_kernel<TA, TB, 16, 4>, dim3((unsigned)(2 * ncu)), NT, 0, s, g, (int)grid.x,
-                    (int)grid.y, (int)items);
-    } else {
-      launch_direct<TA, TB>(s, g, grid, cs);
+SplitChoice choose_split(int M, int N, int K, int batch, bool may_split) {
+  SplitChoice best;
+  best.us = 1e30;
+  const int st = (K + 31) / 32;
+  for (int tile = 0; tile < 3; ++tile) {
+    const long long tiles = tiles_of(tile, M, N) * batch;
+    // splits that fill one, two or three rounds, none deeper than 4 stages
+    long long last = 0;
+    for (int target = 0; target <= 6; ++target) {
+      long long sp = target == 0 ? 1 : (long long)target * (kChipCus / 2) / tiles;
+      if (sp < 1) sp = 1;
+      if (sp > st / 4) sp = st / 4 > 1 ? st / 4 : 1;
+      if (sp * batch > 65535) sp = 1;
+      if (!may_split) sp = 1;
+      if (sp == last) continue;
+      last = sp;
+      int depth = (int)((st + sp - 1) / sp);
+      sp = (st + depth - 1) / depth;
+      double us = grid_us(tile, tiles * sp, depth);
+      if (sp > 1) us += 5.0 + (double)(sp + 1) * M * N * batch * 4.0 / 4.0e6;
+      if (us < best.us) best = {tile, (int)sp, sp > 1 ? depth * 32 : K, us};
     }
-  } else if (t.wm == 4 && t.wn == 4) {
-    if (t.kd == 16) launch_t<TA, TB, 4, 4, 16>(s, g, grid, vec, cs);
-    else launch_t<TA, TB, 4, 4, 32>(s, g, grid, vec, cs);
-  } else if (t.wm == 4) {
-    launch_t<TA, TB, 4, 2, 32>(s, g, grid, vec, cs);
-  } else if (t.wn == 4) {
-    launch_t<TA, TB, 2, 4, 32>(s, g, grid, vec, cs);
+  }
+  return best;
+}
+
+// Split count, and the K range of a split.
+int choose_splits(int M, int N, int K, int batch, int& kchunk) {
+  const SplitChoice c = choose_split(M, N, K, batch, true);
+  kchunk = c.kchunk;
+  return c.splits;
+}
+
+template <int TA, int TB>
+void launch_lds(hipStream_t s, const GemmArgs& g, dim3 grid, bool vec, bool cs) {
+  if (vec) {
+    if (cs) mle::launch(gemm_kernel<TA, TB, true, true>, grid, NT, 0, s, g);
+    else mle::launch(gemm_kernel<TA, TB, true, false>, grid, NT, 0, s, g);
   } else {
-    launch_t<TA, TB, 2, 2, 32>(s, g, grid, vec, cs);
+    if (cs) mle::launch(gemm_kernel<TA, TB, false, true>, grid, NT, 0, s, g);
+    else mle::launch(gemm_kernel<TA, TB, false, false>, grid, NT, 0, s, g);
   }
 }
 
@@ -1348,10 +631,13 @@ double extent_bytes(int rows, int cols, int64_t ld) { return ((double)(rows - 1)
 // A GEMM call resolved to its arguments, tile shape, grid and kernel family.
 struct GemmPlan {
   GemmArgs g;
-  Tile tile;
+  int tile = kSplitLarge;
   dim3 grid;
-  int vec = 0, which = 0;
-  bool cs = false, direct_ok = false, empty = false;
+  bool vec = false;     // 16-byte operand loads (gemm_kernel)
+  bool tail = false;    // K % 4 != 0 beside a k-contiguous operand (split kernel)
+  int which = 0;
+  bool cs = false, empty = false;
+  bool split = false;   // the split-bf16 kernel; else (not simple, not ksplit) gemm_kernel
   bool simple = false;  // gemm_simple_kernel: one thread per C element, no split
   bool ksplit = false;  // gemm_ksplit_kernel: K split over a workgroup's waves
   int ks_nw = 16;       // its waves per workgroup
@@ -1407,9 +693,7 @@ static int gemm_plan(GemmPlan& P, int trans_a, int trans_b, int M, int N, int K,
   MLE_CHECK_ARG(ldc >= N, "mle_gemm: ldc %lld < N %d", (long long)ldc, N);
   MLE_CHECK_ARG(lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N), "mle_gemm: leading dimension too small");
   MLE_CHECK_ARG(colsum == nullptr || batch == 1 || scs != 0, "mle_gemm: fused colsum over a batch needs a stride");
-  const Tile tile = choose_tile(M, N, K, batch);
-  MLE_CHECK_ARG((M + tile.tm() - 1) / tile.tm() <= 65535 && batch <= 65535, "mle_gemm: grid too large (M %d, batch %d)",
-                M, batch);
+  MLE_CHECK_ARG((M + 127) / 128 <= 65535 && batch <= 65535, "mle_gemm: grid too large (M %d, batch %d)", M, batch);
   MLE_CHECK_ARG(inner >= 1 && batch % inner == 0, "mle_gemm: batch %d not a multiple of inner %d", batch, inner);
   GemmArgs g{A,    B,    C,       colsum,  lda,  ldb,    ldc,  stride_a, stride_b, stride_c, M,    N,   K,
              alpha, beta, 1,       K,       nullptr, nullptr, bias, inner,    sa2,      sb2,      sc2,      sbias, scs,
@@ -1417,28 +701,32 @@ static int gemm_plan(GemmPlan& P, int trans_a, int trans_b, int M, int N, int K,
   const bool v4 = (lda % 4 == 0) && (ldb % 4 == 0) && (stride_a % 4 == 0) && (stride_b % 4 == 0) &&
                   (sa2 % 4 == 0) && (sb2 % 4 == 0) && (gsa % 4 == 0) && (gsb % 4 == 0) && aligned16(A) &&
                   aligned16(B);
-  // Buffer loads need the contiguous bound of each operand to be a multiple of
-  // 4 and every extent (all terms of a sum) addressable with a 31-bit offset.
+  // The split kernel reads its operands through 31-bit buffer offsets (all
+  // terms of a sum, and for a row-contiguous operand the rows that the last
+  // stage and the prefetch compute offsets of).
   const int a_rows = trans_a ? K : M, a_cols = trans_a ? M : K;
   const int b_rows = trans_b ? N : K, b_cols = trans_b ? K : N;
   const double t_extra = terms > 1 ? (double)(terms - 1) : 0.0;
-  const bool buf = v4 && a_cols % 4 == 0 && b_cols % 4 == 0 && K > 0 &&
-                   extent_bytes(a_rows, a_cols, lda) + t_extra * 4.0 * (double)gsa < 2147483648.0 - 64 &&
-                   extent_bytes(b_rows, b_cols, ldb) + t_extra * 4.0 * (double)gsb < 2147483648.0 - 64;
-  const int vec = buf ? 2 : (v4 ? 1 : 0);
   const bool cs = colsum != nullptr;
-  // The direct kernel stores 16-byte row segments of C (and reads bias as float4).
-  const bool direct_ok = N % 4 == 0 && ldc % 4 == 0 && stride_c % 4 == 0 && sc2 % 4 == 0 && aligned16(C) &&
-                         (bias == nullptr || (aligned16(bias) && sbias % 4 == 0));
+  bool split = K > 0 && (!cs || (trans_a && !trans_b)) && gsa >= 0 && gsb >= 0 &&
+               extent_bytes(a_rows + (trans_a ? 64 : 0), a_cols, lda) + t_extra * 4.0 * (double)gsa < 2147483648.0 - 64 &&
+               extent_bytes(b_rows + (trans_b ? 0 : 64), b_cols, ldb) + t_extra * 4.0 * (double)gsb < 2147483648.0 - 64;
+  // Folded terms end on whole stages unless both operands are k-contiguous
+  // (whose last stage is masked).
+  const bool fold = K % 32 == 0 || (!trans_a && trans_b);
+  SplitChoice ch = choose_split(M, N, K, batch, ws != nullptr && terms <= 1);
+  if (terms > 1) ch = choose_split(M, N, (int)std::min(2147483000.0, (double)K * terms), batch, false);
+  const double items = (double)tiles_of(ch.tile, M, N) * batch * std::max(ch.splits, std::max(terms, 1));
+  split = split && items < 1073741824.0;
   if (terms > 1) {
     // Sum of `terms` products.  The workspace is part of the contract either
-    // way.  On the register-direct kernel the terms extend its K loop (one
+    // way.  On the split kernel the terms extend its K loop (one
     // accumulator, terms in order, no partials); otherwise one split per
     // term, reduced in term order.
     const size_t need = ((size_t)terms * batch * M * N + (size_t)terms * batch * N) * sizeof(float);
     MLE_CHECK_ARG(ws && ws_bytes >= need, "mle_gemm_sum: workspace of %zu bytes needed", need);
     MLE_CHECK_ARG(terms * batch <= 65535, "mle_gemm_sum: too many terms");
-    if (tile.direct && direct_ok && vec == 2 && K % 16 == 0 && (long long)terms * (K / 16) < (1LL << 24)) {
+    if (split && fold && (long long)terms * (K / 32 + 1) < (1LL << 24)) {
       g.kterms = terms;
     } else {
       g.grouped = 1;
@@ -1447,16 +735,12 @@ static int gemm_plan(GemmPlan& P, int trans_a, int trans_b, int M, int N, int K,
       g.part_cs = g.part + (size_t)terms * batch * M * N;
     }
   } else {
-    int kchunk = K;
-    const int splits = ws ? choose_splits(M, N, K, batch, kchunk) : 1;
-    if (splits > 1) {
-      const size_t need = mle_gemm_ws_bytes(M, N, K, batch);
-      if (ws_bytes >= need) {
-        g.splits = splits;
-        g.kchunk = kchunk;
-        g.part = static_cast<float*>(ws);
-        g.part_cs = g.part + (size_t)splits * batch * M * N;
-      }
+    if (ch.splits > 1 && ws_bytes < mle_gemm_ws_bytes(M, N, K, batch)) ch = choose_split(M, N, K, batch, false);
+    if (ch.splits > 1) {
+      g.splits = ch.splits;
+      g.kchunk = ch.kchunk;
+      g.part = static_cast<float*>(ws);
+      g.part_cs = g.part + (size_t)ch.splits * batch * M * N;
     }
   }
   if (simple_shape(M, N, K, batch, inner, terms)) {
@@ -1472,23 +756,34 @@ static int gemm_plan(GemmPlan& P, int trans_a, int trans_b, int M, int N, int K,
     P.ks_nw = ksplit_nw(K);
     P.ks_kc = ksplit_kc(K, P.ks_nw);
   }
+  // 16-byte stores of C's rows (and reads of the bias and of C)
+  g.c_vec = N % 4 == 0 && ldc % 4 == 0 && stride_c % 4 == 0 && sc2 % 4 == 0 && aligned16(C) &&
+            (bias == nullptr || (aligned16(bias) && sbias % 4 == 0)) && (g.splits == 1 || aligned16(g.part));
   P.g = g;
-  P.tile = tile;
-  P.grid = dim3((N + tile.tn() - 1) / tile.tn(), (M + tile.tm() - 1) / tile.tm(), batch * g.splits);
+  P.tile = ch.tile;
+  P.split = split && !P.simple && !P.ksplit;
+  P.vec = v4;
+  P.tail = K % 4 != 0 && (!trans_a || trans_b);
+  P.cs = cs;
+  const int tm = P.split ? kSplitTm[ch.tile] : 128, tn = P.split ? kSplitTn[ch.tile] : 128;
+  P.grid = dim3((N + tn - 1) / tn, (M + tm - 1) / tm, batch * g.splits);
   if (P.ksplit) {
     const int tt = ksplit_tile(M, N, batch);
     P.grid = dim3((N + tt - 1) / tt, (M + tt - 1) / tt, batch);
   }
-  P.vec = vec;
-  P.cs = cs;
-  P.direct_ok = direct_ok;
   P.which = (trans_a ? 2 : 0) + (trans_b ? 1 : 0);
   P.flop = 2.0 * M * (double)N * K * batch * (terms > 1 ? terms : 1);
   P.bytes = 4.0 * batch * ((double)M * K + (double)K * N + (double)M * N * (beta != 0.f ? 2 : 1));
   return MLE_OK;
 }
 
-static void gemm_launch_main(hipStream_t s, const GemmPlan& P) {
+static int split_items(const GemmPlan& P) { return (int)((long long)P.grid.x * P.grid.y * P.grid.z); }
+
+static void gemm_launch_main(hipStream_t s, const GemmPlan& P, int epi = kEpiPlain) {
+  if (P.split) {
+    launch_split(s, P.which, P.g, P.tile, P.tail, P.cs, epi, (int)P.grid.x, (int)P.grid.y, split_items(P));
+    return;
+  }
   if (P.simple) {
     const dim3 grid((unsigned)(((int64_t)P.g.M * P.g.N + 63) / 64), P.grid.z);
     switch (P.which) {
@@ -1528,10 +823,10 @@ static void gemm_launch_main(hipStream_t s, const GemmPlan& P) {
     return;
   }
   switch (P.which) {
-    case 0: launch_tile<0, 0>(s, P.g, P.tile, P.grid, P.vec, P.cs, P.direct_ok); break;
-    case 1: launch_tile<0, 1>(s, P.g, P.tile, P.grid, P.vec, P.cs, P.direct_ok); break;
-    case 2: launch_tile<1, 0>(s, P.g, P.tile, P.grid, P.vec, P.cs, P.direct_ok); break;
-    default: launch_tile<1, 1>(s, P.g, P.tile, P.grid, P.vec, P.cs, P.direct_ok); break;
+    case 0: launch_lds<0, 0>(s, P.g, P.grid, P.vec, P.cs); break;
+    case 1: launch_lds<0, 1>(s, P.g, P.grid, P.vec, P.cs); break;
+    case 2: launch_lds<1, 0>(s, P.g, P.grid, P.vec, P.cs); break;
+    default: launch_lds<1, 1>(s, P.g, P.grid, P.vec, P.cs); break;
   }
 }
 
@@ -1549,43 +844,11 @@ static void gemm_launch_reduce(hipStream_t s, const GemmPlan& P) {
   else mle::launch(split_reduce_kernel<false>, nmain + ncs, 256, 0, s, g, units, nmain);
 }
 
-// Work items of a plan that launch_tile would run on gemm_direct_kernel (one
-// per workgroup), or 0 when it would pick another kernel.
-static long long direct_items(const GemmPlan& P) {
-  const GemmArgs& g = P.g;
-  if (P.empty || P.simple || P.ksplit ||
-      !(P.tile.direct && P.direct_ok && P.vec == 2 && g.K % 16 == 0 && g.kchunk % 16 == 0))
-    return 0;
-  const long long items = (long long)P.grid.x * P.grid.y * P.grid.z;
-  const bool c_buf = ((double)(g.M - 1) * (double)g.ldc + g.N) * 4.0 < 2147483648.0 - 64;
-  const bool stream = g.splits == 1 && g.kterms == 1 && !P.cs && g.K >= 64 && g.K % 64 == 0 &&
-                      items > 2 * cu_count() && items < (1LL << 30) && c_buf;
-  return stream ? 0 : items;
+// True when the split kernel's epilogue can take an extra output of C's shape
+// (row statistics, an activation): whole 64-column blocks per wave, one split.
+static bool epilogue_ok(const GemmPlan& P) {
+  return !P.empty && P.split && !P.tail && P.g.c_vec && P.g.splits == 1 && P.tile != kSplitSmall;
 }
-
-// True when launch_tile would run the plan on the persistent kernel.
-static bool uses_stream(const GemmPlan& P) {
-  const GemmArgs& g = P.g;
-  if (P.empty || P.simple || P.ksplit ||
-      !(P.tile.direct && P.direct_ok && P.vec == 2 && g.K % 16 == 0 && g.kchunk % 16 == 0))
-    return false;
-  return direct_items(P) == 0;
-}
-
-// The persistent kernel with an activation epilogue (plan already known to
-// run on it).
-template <int TA, int TB, int EPI>
-static void launch_stream_act(hipStream_t s, const GemmPlan& P, int kind) {
-  const dim3 grid((unsigned)(2 * cu_count()));
-  const int gx = (int)P.grid.x, gy = (int)P.grid.y, items = (int)((long long)P.grid.x * P.grid.y * P.grid.z);
-  switch (kind) {
-    case MLE_RELU: mle::launch(gemm_stream_kernel<TA, TB, 16, 4, EPI, MLE_RELU>, grid, NT, 0, s, P.g, gx, gy, items); break;
-    case MLE_GELU: mle::launch(gemm_stream_kernel<TA, TB, 16, 4, EPI, MLE_GELU>, grid, NT, 0, s, P.g, gx, gy, items); break;
-    default: mle::launch(gemm_stream_kernel<TA, TB, 16, 4, EPI, MLE_SILU>, grid, NT, 0, s, P.g, gx, gy, items); break;
-  }
-}
-
-static bool epilogue_act(int kind) { return kind == MLE_RELU || kind == MLE_GELU || kind == MLE_SILU; }
 
 static int gemm_impl(mle_stream stream, int trans_a, int trans_b, int M, int N, int K, float alpha, const float* A,
                      int64_t lda, int64_t stride_a, const float* B, int64_t ldb, int64_t stride_b, float beta, float* C,
@@ -1612,7 +875,10 @@ extern "C" {
 
 size_t mle_gemm_ws_bytes(int M, int N, int K, int batch) {
   int kchunk;
-  const int splits = choose_splits(M, N, K, batch, kchunk);
+  int splits = choose_splits(M, N, K, batch, kchunk);
+  // A product of at most 4096 outputs runs on the simple kernel, which leaves
+  // the workspace unused; its size stays that of one split per 32 deep stage.
+  if ((double)M * N * batch <= 4096.0) splits = std::max(splits, (K + 31) / 32);
   if (splits <= 1) return 0;
   return ((size_t)splits * batch * M * N + (size_t)splits * batch * N) * sizeof(float);
 }
@@ -1649,11 +915,11 @@ int mle_gemm_rowstats(mle_stream stream, int trans_a, int trans_b, int M, int N,
                            bias, ws, ws_bytes);
   if (rc != MLE_OK || P.empty) return rc;
   hipStream_t s = as_stream(stream);
-  const bool fused = uses_stream(P);
+  const bool fused = epilogue_ok(P) && P.which == 0;
   if (fused) P.g.rowpart = rowpart, P.g.rp_ld = ldp;
   {
     ProbeScope probe(kFamily[P.which], s, P.flop, P.bytes);
-    gemm_launch_main(s, P);
+    gemm_launch_main(s, P, fused ? kEpiRowstats : kEpiPlain);
   }
   gemm_launch_reduce(s, P);
   if (!fused) {
@@ -1673,11 +939,12 @@ int mle_gemm_act_fwd(mle_stream stream, int trans_a, int trans_b, int M, int N, 
                      ws_bytes);
   if (rc != MLE_OK || P.empty) return rc;
   hipStream_t s = as_stream(stream);
-  if (uses_stream(P) && P.which == 0 && epilogue_act(kind) && aligned16(Y)) {
+  if (epilogue_ok(P) && P.which == 0 && aligned16(Y)) {
     P.g.act_y = Y;
+    P.g.act_kind = kind;
     {
       ProbeScope probe(kFamily[P.which], s, P.flop, P.bytes);
-      launch_stream_act<0, 0, kEpiActFwd>(s, P, kind);
+      gemm_launch_main(s, P, kEpiActFwd);
     }
     return check_launch("mle_gemm_act_fwd");
   }
@@ -1722,13 +989,14 @@ int mle_gemm_act_bwd(mle_stream stream, int trans_a, int trans_b, int M, int N, 
     }
     return check_launch("mle_gemm_act_bwd");
   }
-  if (uses_stream(P) && P.which == 1 && epilogue_act(kind) && aligned16(X) && aligned16(dX)) {
+  if (epilogue_ok(P) && P.which == 1 && aligned16(X) && aligned16(dX)) {
     P.g.act_x = X;
     P.g.act_dx = dX;
     P.g.act_acc = accumulate_dx ? 1 : 0;
+    P.g.act_kind = kind;
     {
       ProbeScope probe(kFamily[P.which], s, P.flop, P.bytes);
-      launch_stream_act<0, 1, kEpiActBwd>(s, P, kind);
+      gemm_launch_main(s, P, kEpiActBwd);
     }
     return check_launch("mle_gemm_act_bwd");
   }
@@ -1744,18 +1012,49 @@ int mle_gemm_act_bwd(mle_stream stream, int trans_a, int trans_b, int M, int N, 
 
 }  // extern "C"
 
-// A Linear whose weight gradient is one round of unsplit register-direct
-// tiles (192 to 256 tiles of 128 x 128: one workgroup, so one wave, per CU
-// and SIMD) and whose input gradient has too many tiles to share a launch
-// with it: the weight gradient then runs as two K splits (two workgroups per
-// CU, as the input gradient runs) and a reduce.  A function of the shape
-// only, as the workspace size must be (C3: 8192 x 1024 x 4096).
-static bool dw_two_splits(int rows, int in, int out, int layers) {
-  if (layers != 1 || rows < 4096 || rows % 32 != 0) return false;
-  const Tile tw = choose_tile(in, out, rows, 1), tx = choose_tile(rows, in, out, 1);
-  const long long nw = (long long)((in + 127) / 128) * ((out + 127) / 128);
-  const long long nx = (long long)((rows + 127) / 128) * ((in + 127) / 128);
-  return tw.direct && tx.direct && nw >= 192 && nw <= 256 && nx > 256;
+// The Linear backward's two products in one grid (gemm_split_pair_kernel): the
+// tile and the weight gradient's K splits.  Its depth is cut to about the
+// chip's share of the whole work, so that no CU is left with one deep tile
+// while the others are done; the input gradient is not split.  `us` is the
+// model's time of the pair, the reduce included.  A function of the shape only.
+struct PairChoice {
+  int tile = kSplitLarge, splits = 1, kchunk = 0;
+  double us = 1e30;
+};
+static PairChoice choose_pair(int rows, int in, int out, int layers) {
+  PairChoice best;
+  if (rows <= 0 || in <= 0 || out <= 0) return best;
+  for (int tile = 0; tile < 2; ++tile) {
+    const long long n0 = tiles_of(tile, rows, in), t1 = tiles_of(tile, in, out) * layers;
+    const long long d0 = (long long)layers * ((out + 31) / 32), st1 = (rows + 31) / 32;
+    if (n0 > (1 << 24) || t1 > (1 << 24)) continue;
+    const long long share = (n0 * d0 + t1 * st1 + kChipCus - 1) / kChipCus;
+    const long long want = share > 0 ? st1 / share : 1;
+    for (long long sp : {1LL, want, want + 1, 2 * want + 1}) {
+      sp = std::max(1LL, std::min({sp, st1 / 4, 65535LL / layers}));
+      const long long d1 = (st1 + sp - 1) / sp;
+      sp = (st1 + d1 - 1) / d1;
+      const long long n1 = t1 * sp;
+      // dW's n1 items first, then dX's n0: `full` rounds of the former on
+      // every CU, a last one on `busy` CUs, and the earliest end of the n0.
+      const double u0 = d0 * kStageUs[tile] + kTileUs[tile], u1 = d1 * kStageUs[tile] + kTileUs[tile];
+      const long long full = n1 / kChipCus, busy = n1 % kChipCus, idle = kChipCus - busy;
+      double us = busy ? u1 : 0.0;
+      for (long long k = 0, done = 0; done < n0 && k < 4096; ++k) {  // k dX rounds on the idle CUs
+        const long long late = k * u0 > u1 ? (long long)((k * u0 - u1) / u0) : 0;
+        done = idle * k + busy * late;
+        us = std::max(us, k * u0);
+        if (done < n0 && idle * k + busy * (late + 1) >= n0) {
+          us = std::max(us, u1 + (late + 1) * u0);
+          break;
+        }
+      }
+      us += (double)full * u1;
+      if (sp > 1) us += 5.0 + (double)(sp + 1) * in * out * layers * 4.0 / 4.0e6;
+      if (us < best.us) best = {tile, (int)sp, (int)(sp > 1 ? d1 * 32 : rows), us};
+    }
+  }
+  return best;
 }
 
 extern "C" {
@@ -1763,8 +1062,8 @@ extern "C" {
 size_t mle_linear_bwd_ws_bytes(int rows, int in, int out, int layers) {
   const size_t dx = layers > 1 ? mle_gemm_sum_ws_bytes(rows, in, layers) : mle_gemm_ws_bytes(rows, in, out, 1);
   size_t dw = mle_gemm_ws_bytes(in, out, rows, layers);
-  if (dw_two_splits(rows, in, out, layers))
-    dw = std::max(dw, (2 * (size_t)in * out + 2 * (size_t)out) * sizeof(float));
+  const PairChoice pc = choose_pair(rows, in, out, layers);
+  if (pc.splits > 1) dw = std::max(dw, (size_t)pc.splits * layers * ((size_t)in * out + out) * sizeof(float));
   return std::max(dx, dw);
 }
 
@@ -1814,16 +1113,6 @@ static int linear_bwd_impl(mle_stream stream, int rows, int in, int out, int lay
     if (code != MLE_OK || act_done) return code;
     return mle_act_bwd(stream, act_kind, act_x, dX, act_dx, (size_t)rows * in, act_acc);
   };
-  const int ncu = cu_count();
-  if (dw_two_splits(rows, in, out, layers) && P1.g.splits == 1 && direct_items(P1) > 0 && direct_items(P1) <= ncu &&
-      direct_items(P0) > ncu && P1.g.K % 32 == 0) {
-    P1.g.splits = 2;
-    P1.g.kchunk = P1.g.K / 2;
-    P1.g.part = static_cast<float*>(ws);
-    P1.g.part_cs = P1.g.part + 2 * (size_t)P1.g.M * P1.g.N;
-    P1.grid.z = 2;
-  }
-  const long long n0 = direct_items(P0), n1 = direct_items(P1);
   // Both small (gemm_simple_kernel, one batch item): one launch.
   if (!P0.empty && !P1.empty && P0.simple && P1.simple && P0.grid.z == 1 && P1.grid.z == 1) {
     const unsigned nb0 = (unsigned)(((int64_t)P0.g.M * P0.g.N + 63) / 64);
@@ -1852,28 +1141,39 @@ static int linear_bwd_impl(mle_stream stream, int rows, int in, int out, int lay
     }
     return finish(check_launch("gemm_pair"));
   }
-  // One launch when both would run on the register-direct kernel at most one
-  // workgroup per CU each, and the dX product needs no workspace (the dW
-  // product's split partials own it).
-  if (n0 > 0 && n1 > 0 && n0 <= ncu && n1 <= ncu && P0.g.splits == 1) {
-    const int start1 = (int)((n0 + 7) / 8 * 8);
-    const PairGrid pg{(int)n0, (int)P0.grid.x, (int)P0.grid.y, (int)n1, (int)P1.grid.x, (int)P1.grid.y, start1};
-    const dim3 grid((unsigned)(start1 + n1));
-    const bool t0 = P0.g.kterms > 1;
-    {
-      ProbeScope probe("gemm_pair", s, P0.flop + P1.flop, P0.bytes + P1.bytes);
-      auto k = t0 ? (P1.cs ? gemm_pair_kernel<0, 1, false, true, 1, 0, true, false>
-                           : gemm_pair_kernel<0, 1, false, true, 1, 0, false, false>)
-                  : (P1.cs ? gemm_pair_kernel<0, 1, false, false, 1, 0, true, false>
-                           : gemm_pair_kernel<0, 1, false, false, 1, 0, false, false>);
-      mle::launch(k, grid, NT, 0, s, P0.g, P1.g, pg);
-      gemm_launch_reduce(s, P1);
+  // One launch when both run on the split kernel without a K tail, and the
+  // model says that sharing the chip beats one product after the other.
+  if (!P0.empty && !P1.empty && P0.split && P1.split && !P0.tail && !P1.tail && !P0.g.grouped && !P1.g.grouped) {
+    const SplitChoice c0 = choose_split(rows, in, out * (layers > 1 ? layers : 1), 1, layers <= 1);
+    const SplitChoice c1 = choose_split(in, out, rows, layers, true);
+    const PairChoice pc = choose_pair(rows, in, out, layers);
+    const double parts = (double)pc.splits * layers * ((double)in * out + out) * sizeof(float);
+    if (pc.us < c0.us + c1.us + 3.0 && (pc.splits == 1 || (ws && (double)ws_bytes >= parts))) {
+      GemmArgs g0 = P0.g, g1 = P1.g;
+      g0.splits = 1;
+      g0.kchunk = out;
+      g1.splits = pc.splits;
+      g1.kchunk = pc.kchunk;
+      g1.part = static_cast<float*>(ws);
+      g1.part_cs = g1.part + (size_t)pc.splits * layers * in * out;
+      if (pc.splits > 1 && !aligned16(ws)) g1.c_vec = 0;
+      const int tm = kSplitTm[pc.tile], tn = kSplitTn[pc.tile];
+      PairGrid pg;
+      pg.gx0 = (in + tn - 1) / tn, pg.gy0 = (rows + tm - 1) / tm, pg.items0 = pg.gx0 * pg.gy0;
+      pg.gx1 = (out + tn - 1) / tn, pg.gy1 = (in + tm - 1) / tm, pg.items1 = pg.gx1 * pg.gy1 * layers * pc.splits;
+      pg.start0 = (pg.items1 + 7) / 8 * 8;
+      {
+        ProbeScope probe("gemm_pair", s, P0.flop + P1.flop, P0.bytes + P1.bytes);
+        launch_split_pair(s, g0, g1, pc.tile, P1.cs, pg);
+        GemmPlan R = P1;
+        R.g = g1;
+        R.grid.z = layers * pc.splits;
+        gemm_launch_reduce(s, R);
+      }
+      return finish(check_launch("gemm_pair"));
     }
-    return finish(check_launch("gemm_pair"));
   }
-  // Otherwise one launch each, in order (they may share the workspace).  (A
-  // dX on the persistent kernel writing the activation's gradient in its
-  // epilogue measured slower in the C4 step than the separate pass.)
+  // Otherwise one launch each, in order (they may share the workspace).
   if (!P0.empty) {
     ProbeScope probe(kFamily[P0.which], s, P0.flop, P0.bytes);
     gemm_launch_main(s, P0);

@@ -1,0 +1,110 @@
+"""The split-bf16 GEMM (csrc/split_core.hpp) at the edges of its tiles and
+stages, and on values that its split cannot represent.
+
+Bound: of the six partial products per multiply, the leading one is summed in
+one fp32 accumulator and the rest in another, one rounding (at most 2^-23,
+the matrix core truncates) per 32-deep stage and accumulator; splitting K adds
+a rounding per part, and the dropped terms are below 2^-25 of each product.
+So |C - exact| <= (2 ceil(K / 32) + 8) 2^-23 sum |a b|, element by element
+(half that for the fp32 MFMA fallback's K / 4 roundings of 2^-24 each)."""
+import numpy as np
+import pytest
+
+from conftest import rng
+
+pytestmark = pytest.mark.gpu
+
+
+def bound(K):
+    return (2 * ((K + 31) // 32) + 8) * 2.0 ** -23
+
+
+def run(hip, ta, tb, M, N, K, A, Bm, C0=None, bias=None, colsum=None):
+    """C (and the column sums) of mle_gemm_ex with its workspace."""
+    B = hip.Buffer.from_array
+    gA, gB = B(A), B(Bm)
+    gC = B(np.full((M, N), np.nan, np.float32) if C0 is None else C0)
+    gb = B(bias) if bias is not None else None
+    gs = B(colsum) if colsum is not None else None
+    nb = hip.lib().mle_gemm_ws_bytes(M, N, K, 1)
+    ws = hip.Buffer(nb) if nb else None
+    hip.call("mle_gemm_ex", None, ta, tb, M, N, K, 1.0, gA.ptr, A.shape[1], 0, gB.ptr, Bm.shape[1], 0,
+             0.0 if C0 is None else 1.0, gC.ptr, N, 0, 1, gs.ptr if gs else None, gb.ptr if gb else None,
+             ws.ptr if ws else None, nb)
+    return gC.numpy((M, N)), gs.numpy() if gs else None
+
+
+# Outputs above 4096 x 64 (the small-product kernels end there), each tile
+# shape, one row or column less and more than whole tiles, K around one stage,
+# no multiple of 4, and long enough to split.
+SHAPES = [(1000, 516, 330), (513, 515, 1), (640, 449, 31), (640, 449, 32), (768, 513, 33), (257, 1025, 35),
+          (255, 2047, 64), (2049, 129, 95), (4095, 127, 131), (4100, 65, 1027), (8192, 520, 70), (700, 400, 4099)]
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_split_gemm_edges(hip, ta, tb, M, N, K):
+    r = rng(M + 3 * N + 7 * K + ta + 2 * tb)
+    a, b = r.standard_normal((M, K), dtype=np.float32), r.standard_normal((K, N), dtype=np.float32)
+    bias = r.standard_normal(N, dtype=np.float32)
+    # row strides of no alignment: 3 columns that must not be read as part of the matrix
+    wide = lambda t: np.concatenate([t, np.full((t.shape[0], 3), 1e30, np.float32)], 1)  # noqa: E731
+    A, Bm = wide(a.T if ta else a), wide(b.T if tb else b)
+    cs0 = r.standard_normal(N, dtype=np.float32) if (ta, tb) == (1, 0) else None
+    C, cs = run(hip, ta, tb, M, N, K, np.ascontiguousarray(A), np.ascontiguousarray(Bm), bias=bias, colsum=cs0)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    want, terms = a64 @ b64 + bias, np.abs(a64) @ np.abs(b64) + np.abs(bias)
+    assert np.all(np.abs(C - want) <= bound(K) * terms)
+    if cs is not None:  # a sequential fp32 sum per lane group, then four of them
+        lim = (K / 4 + 8) * 2.0 ** -24 * (np.abs(b64).sum(0) + np.abs(cs0))
+        assert np.all(np.abs(cs - (b64.sum(0) + cs0)) <= lim)
+    # adding to C
+    C0 = r.standard_normal((M, N), dtype=np.float32)
+    C, _ = run(hip, ta, tb, M, N, K, np.ascontiguousarray(A), np.ascontiguousarray(Bm), C0=C0.copy())
+    assert np.all(np.abs(C - (a64 @ b64 + C0)) <= bound(K) * (terms + np.abs(C0)))
+
+
+@pytest.mark.parametrize("what", ["inf", "nan", "max", "tiny", "overflow"])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
+def test_split_gemm_special_values(hip, ta, tb, what):
+    """Infinities, NaN, the largest values (which round to infinity in bf16)
+    and values too small for three bf16 parts: as fp32 products give them."""
+    M, N, K = 700, 600, 200
+    r = rng(77 + ta + 2 * tb)
+    a, b = r.standard_normal((M, K), dtype=np.float32), r.standard_normal((K, N), dtype=np.float32)
+    fmax = np.finfo(np.float32).max
+    if what == "inf":
+        a[3, 5], a[300, 7], b[9, 400] = np.inf, -np.inf, np.inf
+    elif what == "nan":
+        a[699, 199], b[0, 0] = np.nan, np.nan
+    elif what == "max":  # finite results: the row's other values vanish against them
+        a[17, :], a[17, 3] = 0.0, -fmax
+        b[3, :] = np.clip(b[3], -0.9, 0.9)
+    elif what == "tiny":
+        a[400:, :] *= np.float32(2.0 ** -112)
+        b[:, 100:200] *= np.float32(2.0 ** 40)
+    else:
+        a[50, :], b[:, 60] = np.float32(1e30), np.float32(1e30)
+    A, Bm = np.ascontiguousarray(a.T if ta else a), np.ascontiguousarray(b.T if tb else b)
+    C, _ = run(hip, ta, tb, M, N, K, A, Bm)
+    with np.errstate(invalid="ignore", over="ignore"):
+        a64, b64 = a.astype(np.float64), b.astype(np.float64)
+        want = (a64 @ b64)
+        terms = np.abs(a64) @ np.abs(b64)
+        w32 = want.astype(np.float32)
+    assert np.array_equal(np.isnan(C), np.isnan(w32))
+    assert np.array_equal(C[np.isinf(w32)], w32[np.isinf(w32)])
+    ok = np.isfinite(w32)
+    assert np.all(np.isfinite(C[ok]))
+    # results below the normal range round to fp32's smallest step
+    lim = bound(K) * terms[ok] + 2.0 ** -140
+    assert np.all(np.abs(C[ok] - want[ok]) <= lim)
+
+
+def test_split_gemm_identity_exact(hip):
+    """A value times one is the value: the three parts add up to it exactly."""
+    M, N = 600, 640
+    r = rng(5)
+    a = (r.standard_normal((M, N)) * np.exp2(r.integers(-60, 60, (M, N)))).astype(np.float32)
+    C, _ = run(hip, 0, 0, M, N, N, a, np.eye(N, dtype=np.float32))
+    np.testing.assert_array_equal(C, a)
