@@ -8,102 +8,16 @@
 //   wgrad   : C[co][(ci,kh,kw)] = dY[co][(b,oh,ow)] * im2col(X)^T[(b,oh,ow)][(ci,kh,kw)]
 // wgrad splits its long K = B*OH*OW across workgroups; the partial tiles land
 // in the workspace and one pass adds them in split order (assign semantics).
+#include "conv_args.hpp"
 #include "gemm_core.hpp"
 
 #include <algorithm>
 
 using namespace mle;
 using namespace gemm;
+using namespace conv;
 
 namespace {
-
-struct ConvGeom {
-  int n, cin, h, w, cout, kh, kw, pad, stride, oh, ow;
-};
-
-// Each operand functor returns the GEMM element or 0 outside the problem.
-struct FwdOps {
-  const float* x;
-  const float* wt;
-  const float* bias;
-  float* y;
-  ConvGeom g;
-  int M, N, K;
-  __device__ float a(int m, int k) const { return (m < M && k < K) ? wt[(size_t)m * K + k] : 0.f; }
-  __device__ float b(int k, int n) const {
-    if (k >= K || n >= N) return 0.f;
-    const int khw = g.kh * g.kw;
-    const int ci = k / khw, r = k - ci * khw, kh = r / g.kw, kw = r - kh * g.kw;
-    const int ohw = g.oh * g.ow;
-    const int bb = n / ohw, pix = n - bb * ohw, oh = pix / g.ow, ow = pix - oh * g.ow;
-    const int ih = oh * g.stride - g.pad + kh, iw = ow * g.stride - g.pad + kw;
-    if (ih < 0 || ih >= g.h || iw < 0 || iw >= g.w) return 0.f;
-    return x[(((size_t)bb * g.cin + ci) * g.h + ih) * g.w + iw];
-  }
-  __device__ void store(int m, int n, float v, int) const {
-    const int ohw = g.oh * g.ow;
-    const int bb = n / ohw, pix = n - bb * ohw;
-    y[((size_t)bb * g.cout + m) * ohw + pix] = bias ? v + bias[m] : v;
-  }
-};
-
-struct DgradOps {
-  const float* dy;
-  const float* wt;
-  float* dx;
-  ConvGeom g;
-  int M, N, K;
-  int acc;
-  __device__ float a(int m, int k) const {
-    if (m >= M || k >= K) return 0.f;
-    const int khw = g.kh * g.kw;
-    const int co = k / khw, r = k - co * khw;
-    return wt[((size_t)co * g.cin + m) * khw + r];
-  }
-  __device__ float b(int k, int n) const {
-    if (k >= K || n >= N) return 0.f;
-    const int khw = g.kh * g.kw;
-    const int co = k / khw, r = k - co * khw, kh = r / g.kw, kw = r - kh * g.kw;
-    const int hw = g.h * g.w;
-    const int bb = n / hw, pix = n - bb * hw, ih = pix / g.w, iw = pix - ih * g.w;
-    const int nr = ih + g.pad - kh, nc = iw + g.pad - kw;
-    if (nr < 0 || nc < 0 || nr % g.stride != 0 || nc % g.stride != 0) return 0.f;
-    const int oy = nr / g.stride, ox = nc / g.stride;
-    if (oy >= g.oh || ox >= g.ow) return 0.f;
-    return dy[(((size_t)bb * g.cout + co) * g.oh + oy) * g.ow + ox];
-  }
-  __device__ void store(int m, int n, float v, int) const {
-    const int hw = g.h * g.w;
-    const int bb = n / hw, pix = n - bb * hw;
-    float* d = dx + ((size_t)bb * g.cin + m) * hw + pix;
-    *d = acc ? *d + v : v;
-  }
-};
-
-struct WgradOps {
-  const float* x;
-  const float* dy;
-  float* part;  // [splits][M*N]
-  ConvGeom g;
-  int M, N, K;
-  __device__ float a(int m, int k) const {
-    if (m >= M || k >= K) return 0.f;
-    const int ohw = g.oh * g.ow;
-    const int bb = k / ohw, pix = k - bb * ohw;
-    return dy[((size_t)bb * g.cout + m) * ohw + pix];
-  }
-  __device__ float b(int k, int n) const {
-    if (k >= K || n >= N) return 0.f;
-    const int khw = g.kh * g.kw;
-    const int ci = n / khw, r = n - ci * khw, kh = r / g.kw, kw = r - kh * g.kw;
-    const int ohw = g.oh * g.ow;
-    const int bb = k / ohw, pix = k - bb * ohw, oh = pix / g.ow, ow = pix - oh * g.ow;
-    const int ih = oh * g.stride - g.pad + kh, iw = ow * g.stride - g.pad + kw;
-    if (ih < 0 || ih >= g.h || iw < 0 || iw >= g.w) return 0.f;
-    return x[(((size_t)bb * g.cin + ci) * g.h + ih) * g.w + iw];
-  }
-  __device__ void store(int m, int n, float v, int split) const { part[(size_t)split * M * N + (size_t)m * N + n] = v; }
-};
 
 // B_KC selects the B tile layout: false = [BK][BN] (threads walk n), true =
 // [BN][BK] (threads walk k); chosen per operand so consecutive lanes read
@@ -250,36 +164,7 @@ void launch_split_reduce(hipStream_t s, const float* part, int splits, size_t mn
     mle::launch(split_reduce_kernel<false>, nmain + nb2, 256, 0, s, part, splits, mn, out, nmain, part2, n2, out2, acc2);
 }
 
-// ---------------------------------------------------------------------------
-// Fast path: stride 1, filter KH x KW known at compile time (3x3 and 1x1).
-// Same 128 x 128 x 32 MFMA tiles; what changes is the operand gather:
-//  * every filter-tap decode (k -> channel, kh, kw) divides by constants;
-//  * a thread's output pixel (forward / dgrad) or input pixel (wgrad) is
-//    decoded once per tile or once per K stage, not once per element;
-//  * reads go through raw buffer resources: a tap that falls in the zero
-//    padding, or past the tile, gets an offset beyond the extent and the
-//    hardware returns 0, so the K loop has no branches;
-//  * the epilogue stages each wave's block in LDS and writes 16-byte rows.
-// Requirements (checked on the host, else the generic kernel runs): every
-// tensor below 2 GiB, pixel counts and K multiples of 4 (float4 never
-// straddles an image), 16-byte aligned outputs.
-enum ConvKind { CONV_FWD = 0, CONV_DGRAD = 1, CONV_WGRAD = 2 };
-constexpr uint32_t kOOB = 0x80000000u;
-
-struct FastConv {
-  const float* src;   // gathered operand: x (fwd, wgrad) or dy (dgrad)
-  const float* wa;    // A operand: weights (fwd, dgrad) or dy (wgrad)
-  const float* bias;  // fwd only (nullable)
-  float* out;         // y (fwd, assign), dx (dgrad, accumulate), partials (wgrad)
-  uint32_t src_bytes, wa_bytes;
-  int M, N, K, kchunk;
-  // gathered tensor: channels, spatial size; output-pixel grid (pixels of C's n)
-  int sc, sh, sw, shw;
-  int ph, pw, phw;
-  int pad;
-  int cout, cin;  // for the A / output index maps
-  int acc;        // dgrad: 1 accumulates into dx, 0 assigns
-};
+constexpr uint32_t kOOB = 0x80000000u;  // byte offset past every buffer
 
 __device__ __forceinline__ float buf_ld1(__amdgpu_buffer_rsrc_t r, uint32_t off_bytes) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off_bytes, 0, 0));
@@ -289,185 +174,6 @@ __device__ __forceinline__ f32x4 buf_ld4(__amdgpu_buffer_rsrc_t r, uint32_t off_
 }
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const float* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), (short)0, (int)bytes, 0x00020000);
-}
-
-template <int KIND, int KH, int KW>
-__global__ __launch_bounds__(NT, 2) void conv_fast_kernel(FastConv c) {
-  constexpr int KHW = KH * KW;
-  constexpr bool B_KC = KIND == CONV_WGRAD;
-  constexpr int ASZ = a_tile_floats<false>();
-  constexpr int BSZ = b_tile_floats<B_KC>();
-  __shared__ __attribute__((aligned(16))) float smem[2 * (ASZ + BSZ)];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int lr = lane & 15, q = lane >> 4, wm = wave & 1, wn = wave >> 1;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int kbeg = blockIdx.z * c.kchunk;
-  const int kend = min(c.K, kbeg + c.kchunk);
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(c.src, c.src_bytes);
-  const __amdgpu_buffer_rsrc_t ra_rs = make_rsrc(c.wa, c.wa_bytes);
-
-  // Per-thread output pixel of the B gather (fwd / dgrad): fixed for the tile.
-  int g_base = 0, g_y0 = 0, g_x0 = 0;
-  bool g_nok = false;
-  if (KIND != CONV_WGRAD) {
-    const int n = n0 + (tid & 127);
-    g_nok = n < c.N;
-    const int b = n / c.phw, pix = n - b * c.phw, py = pix / c.pw, px = pix - py * c.pw;
-    g_base = b * c.sc * c.shw;
-    g_y0 = KIND == CONV_FWD ? py - c.pad : py + c.pad;
-    g_x0 = KIND == CONV_FWD ? px - c.pad : px + c.pad;
-  }
-
-  f32x4 ra4[4];
-  float ra1[16], rb[16];
-  auto load = [&](int k0) {
-    // ---- A ----
-    if (KIND == CONV_FWD) {  // W [cout][K], k-contiguous float4
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int f = tid + NT * i, row = m0 + (f >> 3), k = k0 + (f & 7) * 4;
-        const bool ok = (row < c.M) & (k < kend);
-        ra4[i] = buf_ld4(ra_rs, ok ? (uint32_t)(row * c.K + k) * 4u : kOOB);
-      }
-    } else if (KIND == CONV_DGRAD) {  // A[ci][(co,r)] = W[co][ci][r]
-      const int k = k0 + (tid & 31);
-      const int co = k / KHW, r = k - co * KHW;
-      const bool kok = k < kend;
-      const uint32_t kb = (uint32_t)(co * c.cin * KHW + r);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int row = m0 + (tid >> 5) + 8 * i;
-        const bool ok = kok & (row < c.M);
-        ra1[i] = buf_ld1(ra_rs, ok ? (kb + (uint32_t)(row * KHW)) * 4u : kOOB);
-      }
-    } else {  // WGRAD: A[co][pixel] = dy[b][co][pix], float4 along pixels
-      const int b0 = k0 / c.phw, p0 = k0 - b0 * c.phw;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int f = tid + NT * i, row = m0 + (f >> 3), kk = (f & 7) * 4;
-        int pix = p0 + kk, b = b0;
-        if (pix >= c.phw) {
-          pix -= c.phw;
-          ++b;
-        }
-        const bool ok = (row < c.M) & (k0 + kk < kend);
-        ra4[i] = buf_ld4(ra_rs, ok ? (uint32_t)((b * c.cout + row) * c.phw + pix) * 4u : kOOB);
-      }
-    }
-    // ---- B ----
-    if (KIND != CONV_WGRAD) {  // B[(ch,kh,kw)][pixel], n-contiguous
-      const int kq = tid >> 7;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int k = k0 + kq + 2 * i;
-        const int ch = k / KHW, r = k - ch * KHW, kh = r / KW, kw = r - kh * KW;
-        const int sy = KIND == CONV_FWD ? g_y0 + kh : g_y0 - kh;
-        const int sx = KIND == CONV_FWD ? g_x0 + kw : g_x0 - kw;
-        const bool ok = g_nok & (k < kend) & ((unsigned)sy < (unsigned)c.sh) & ((unsigned)sx < (unsigned)c.sw);
-        rb[i] = buf_ld1(rs, ok ? (uint32_t)(g_base + ch * c.shw + sy * c.sw + sx) * 4u : kOOB);
-      }
-    } else {  // WGRAD: B[pixel][(ci,kh,kw)] = x[b][ci][py - pad + kh][px - pad + kw], k-contiguous
-      const int k = k0 + (tid & 31);
-      const int b0 = k0 / c.phw;
-      int pix = k0 - b0 * c.phw + (tid & 31), b = b0;
-      if (pix >= c.phw) {
-        pix -= c.phw;
-        ++b;
-      }
-      const int py = pix / c.pw, px = pix - py * c.pw;
-      const bool kok = k < kend;
-      const int base = b * c.sc * c.shw;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int n = n0 + (tid >> 5) + 8 * i;
-        const int ch = n / KHW, r = n - ch * KHW, kh = r / KW, kw = r - kh * KW;
-        const int sy = py - c.pad + kh, sx = px - c.pad + kw;
-        const bool ok = kok & (n < c.N) & ((unsigned)sy < (unsigned)c.sh) & ((unsigned)sx < (unsigned)c.sw);
-        rb[i] = buf_ld1(rs, ok ? (uint32_t)(base + ch * c.shw + sy * c.sw + sx) * 4u : kOOB);
-      }
-    }
-  };
-  auto store = [&](int buf) {
-    float* As = smem + buf * ASZ;
-    float* Bs = smem + 2 * ASZ + buf * BSZ;
-    if (KIND == CONV_DGRAD) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) As[((tid >> 5) + 8 * i) * LDK + (tid & 31)] = ra1[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int f = tid + NT * i;
-        *reinterpret_cast<f32x4*>(As + (f >> 3) * LDK + (f & 7) * 4) = ra4[i];
-      }
-    }
-    if (KIND != CONV_WGRAD) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) Bs[((tid >> 7) + 2 * i) * LDMN + (tid & 127)] = rb[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) Bs[((tid >> 5) + 8 * i) * LDK + (tid & 31)] = rb[i];
-    }
-  };
-
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int n = 0; n < 4; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
-  if (nk > 0) {
-    load(kbeg);
-    store(0);
-  }
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    const bool more = kt + 1 < nk;
-    if (more) load(kbeg + (kt + 1) * BK);
-    mma_stage<false, B_KC>(smem + cur * ASZ, smem + 2 * ASZ + cur * BSZ, acc, wm, wn, lr, q);
-    if (more) store(cur ^ 1);
-    __syncthreads();
-  }
-
-  // Epilogue: each wave's 64 x 64 block through LDS, 32 rows at a time; a lane
-  // writes 4 consecutive columns (pixels, or weight taps for wgrad).
-  constexpr int EPI = 68;
-  float* T = smem + wave * (32 * EPI);
-#pragma unroll
-  for (int half = 0; half < 2; ++half) {
-#pragma unroll
-    for (int ii = 0; ii < 2; ++ii) {
-      const int i = half * 2 + ii;
-#pragma unroll
-      for (int n = 0; n < 4; ++n)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) T[(ii * 16 + 4 * q + r) * EPI + n * 16 + lr] = acc[i][n][r];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < 8; ++it) {
-      const int rr = it * 4 + (lane >> 4), cc = (lane & 15) * 4;
-      const int row = m0 + wm * 64 + half * 32 + rr, col = n0 + wn * 64 + cc;
-      if (row < c.M && col < c.N) {
-        f32x4 v = *reinterpret_cast<const f32x4*>(T + rr * EPI + cc);
-        if (KIND == CONV_WGRAD) {
-          *reinterpret_cast<f32x4*>(c.out + (size_t)blockIdx.z * c.M * c.N + (size_t)row * c.N + col) = v;
-        } else {
-          const int b = col / c.phw, pix = col - b * c.phw;
-          const int oc = KIND == CONV_FWD ? c.cout : c.cin;
-          f32x4* dst = reinterpret_cast<f32x4*>(c.out + ((size_t)b * oc + row) * c.phw + pix);
-          if (KIND == CONV_FWD) {
-            if (c.bias) v += c.bias[row];
-          } else if (c.acc) {
-            v += *dst;
-          }
-          *dst = v;
-        }
-      }
-    }
-    __syncthreads();
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -896,391 +602,23 @@ __global__ __launch_bounds__(64 * WM * WN * KS, 2) void conv1_direct_kernel(Conv
   conv1_direct_body<DG, WM, WN, KS, D>(c, blockIdx.x);
 }
 
-// Forward of a 3 x 3 (pad 1) and a 1 x 1 (pad 0) convolution of the same x
-// (a residual block's first convolution and its skip) in one grid: the 1 x 1
-// tiles first, then the 3 x 3 tiles, each product with its own XCD-aware
-// tile order.  Measured on the C5 shapes (16 x 64 -> 128 x 64 x 64):
-// 100.4 us against 109.4 us for the two launches.  The 3 x 3 tiles first ran
-// 104.5 us, each workgroup's 3 x 3 tile followed by the same pixels' 1 x 1
-// tile 103.6 us, and the two products alternating across the XCDs 154.7 us
-// (the 3 x 3 tiles slow down when they do not run in lockstep with their
-// neighbours).
-template <bool HALO, int WM3, int WM1>
-__global__ __launch_bounds__(256, 2) void conv_pair_fwd_kernel(Conv3Args a, Conv3Args b) {
-  const int L = blockIdx.x;
-  if (L < b.tiles)
-    conv1_direct_body<false, WM1, 2, WM1 == 1 ? 2 : 1, 4>(b, L);
-  else
-    conv3_direct_body<false, HALO, WM3, 2, WM3 == 1 ? 2 : 1, kC3U, kC3D>(a, a, L - b.tiles);
-}
-
-// Input gradient of the same pair: dx (+)= dgrad3(dy3) + dgrad1(dy1), the
+// Input gradient of a 3 x 3 (pad 1) and a 1 x 1 (pad 0) convolution of one
+// input: dx (+)= dgrad3(dy3) + dgrad1(dy1), the
 // 1 x 1 product as extra stages of each 3 x 3 tile.
-template <bool HALO, int WM>
+template <bool HALO>  // 64-row blocks
 __global__ __launch_bounds__(256, 2) void conv_pair_dgrad_kernel(Conv3Args a, Conv3Args b) {
-  conv3_direct_body<true, HALO, WM, 2, WM == 1 ? 2 : 1, kC3U, kC3D, true>(a, b, blockIdx.x);
+  conv3_direct_body<true, HALO, 1, 2, 2, kC3U, kC3D, true>(a, b, blockIdx.x);
 }
 
-// ---------------------------------------------------------------------------
-// Register-direct 3 x 3 weight gradient, stride 1, pad 1:
-//   dW[co][ci][kh][kw] = sum over pixels p of dy[co][p] * x[ci][p + (kh - 1, kw - 1)]
-// as C[co][(ci, kh, kw)] with K = the batch's pixels, split across workgroups
-// (each split writes its partial C; a second pass adds them in split order).
-// Lane (lr, q) of a wave owns one (ci, kh) pair (16 pairs per wave) and its
-// three kw taps are the wave's three MFMA column blocks, so a wave's block is
-// 64 output channels x 48 columns.  Per 16-pixel stage lane group q feeds
-// pixels P .. P + 3 (P = stage start + 4 q) to the four MFMA steps: dy as one
-// aligned float4 per 16-row block, x of its (ci, kh) row as one aligned
-// float4 plus the two neighbours x[P - 1] and x[P + 4], from which the three
-// taps' operands are picked in registers.  A neighbour in the column padding,
-// a row shift out of the image, a pixel past the split, a pair past cin * 3
-// or a row past cout reads at kOOB and gets 0.  The lane's pixel position
-// advances by 16 per stage with at most one row and one image carry (W >= 16).
-struct Wgrad3Args {
-  const float* x;   // [n][cin][h][w]
-  const float* dy;  // [n][cout][h][w]
-  float* out;       // one split: dW [cout][cin * 9]; else partials [splits][cout][cin * 9]
-  uint32_t x_bytes, dy_bytes, out_bytes;
-  int cout, cin, h, w, hw, npix;
-  int chunk;  // pixels per split, a multiple of 16
-  int tiles_m, tiles, items;
-  // Bias gradient from the dy rows the kernel already loads (sum over the
-  // pixels per output channel), taken by the waves of the first column block:
-  // db_mode 1 adds into db (one split), 3 assigns it; 2 writes the split's
-  // partial sums to bpart[split][cout].
-  float* db;
-  float* bpart;
-  int db_mode;
-};
-
-// Per lane, the dy row sums of stage `fa` (block i: four pixels of row
-// m0 + 16 i + lr), added pairwise.
-__device__ __forceinline__ void bias_stage(float (&bs)[4], const f32x4 (&fa)[4]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) bs[i] += (fa[i][0] + fa[i][1]) + (fa[i][2] + fa[i][3]);
-}
-
-// Combine the four lane groups' row sums (q order fixed by the xor tree) and
-// store them: lane (lr, q = 0) owns rows m0 + 16 i + lr.
-__device__ __forceinline__ void bias_store(const Wgrad3Args& c, float (&bs)[4], int m0, int split, int lr, int q) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float v = bs[i];
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
-    const int co = m0 + 16 * i + lr;
-    if (q == 0 && co < c.cout) {
-      if (c.db_mode == 1) c.db[co] += v;
-      else if (c.db_mode == 3) c.db[co] = v;
-      else c.bpart[(size_t)split * c.cout + co] = v;
-    }
-  }
-}
-
-template <int WM, int D>
-__global__ __launch_bounds__(256, 2) void conv3_wgrad_kernel(Wgrad3Args c) {
-  constexpr int WN = 4 / WM;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int lr = lane & 15, q = lane >> 4;
-  const int wm = wave % WM, wn = wave / WM;
-  // Workgroup -> (tile, split): consecutive items on one XCD, tiles of one
-  // split adjacent (they read the same dy and x pixels).
-  const int L = blockIdx.x, xq = c.items / 8, xr = c.items % 8, xc = L % 8;
-  const int item = xc * xq + min(xc, xr) + L / 8;
-  const int tile = item % c.tiles, split = item / c.tiles;
-  const int tm = tile % c.tiles_m, tn = tile / c.tiles_m;
-  const int m0 = (tm * WM + wm) * 64;
-  const int pair = (tn * WN + wn) * 16 + lr;
-  const bool pok = pair < 3 * c.cin;
-  const int ci = pair / 3, kh = pair - 3 * ci;
-  const int kbeg = split * c.chunk, kend = min(c.npix, kbeg + c.chunk);
-  const int nk = (kend - kbeg + 15) / 16;
-  const __amdgpu_buffer_rsrc_t rx = make_rsrc(c.x, c.x_bytes);
-  const __amdgpu_buffer_rsrc_t rd = make_rsrc(c.dy, c.dy_bytes);
-  uint32_t a_row[4];
-  bool a_ok[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int co = m0 + 16 * i + lr;
-    a_ok[i] = co < c.cout;
-    a_row[i] = (uint32_t)(co * c.hw) * 4u;
-  }
-  const uint32_t x_lane = (uint32_t)(ci * c.hw + (kh - 1) * c.w) * 4u;  // modulo 2^32
-  // Load cursor: the next stage's pixel P of this lane, its column px and row
-  // py, and its pixel byte offsets in dy and x (without the channel part).
-  // Advancing 16 pixels adds 64 bytes, plus the rest of an image's channel
-  // planes when P crosses into the next image; W >= 16, so at most one row
-  // and one image carry.  Only adds and selects: no multiplies in the loop.
-  int P = kbeg + 4 * q;
-  int py, px;
-  uint32_t dpix, xpix;
-  {
-    const int b = P / c.hw, pp = P - b * c.hw;
-    py = pp / c.w;
-    px = pp - py * c.w;
-    dpix = (uint32_t)(b * c.cout * c.hw + pp) * 4u;
-    xpix = (uint32_t)(b * c.cin * c.hw + pp) * 4u;
-  }
-  const uint32_t d_img = (uint32_t)((c.cout - 1) * c.hw) * 4u, x_img = (uint32_t)((c.cin - 1) * c.hw) * 4u;
-
-  auto load = [&](f32x4(&fa)[4], f32x4& fb, float& fl, float& fr) {
-    const bool pix = P < kend;
-    const bool rowok = (unsigned)(py + kh - 1) < (unsigned)c.h;
-    // Offsets are selected (bitwise conditions, no short circuit) so the
-    // loads stay unconditional.
-    uint32_t ao[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ao[i] = (pix & a_ok[i]) ? a_row[i] + dpix : kOOB;
-    const bool ok = pix & rowok & pok;
-    const uint32_t xo = x_lane + xpix;
-    const uint32_t xc = ok ? xo : kOOB;
-    const uint32_t xl = (ok & (px != 0)) ? xo - 4u : kOOB;
-    const uint32_t xr = (ok & (px + 4 != c.w)) ? xo + 16u : kOOB;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      fa[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rd, (int)ao[i], 0, 0));
-    fb = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)xc, 0, 0));
-    fl = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, (int)xl, 0, 0));
-    fr = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, (int)xr, 0, 0));
-    P += 16;
-    px += 16;
-    dpix += 64u;
-    xpix += 64u;
-    const bool cx = px >= c.w;
-    px = cx ? px - c.w : px;
-    py += cx ? 1 : 0;
-    const bool cy = py >= c.h;
-    py = cy ? 0 : py;
-    dpix += cy ? d_img : 0u;
-    xpix += cy ? x_img : 0u;
-  };
-
-  f32x4 acc[4][3];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int n = 0; n < 3; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const bool do_b = c.db_mode != 0 && tn == 0 && wn == 0;
-  float bs[4] = {0.f, 0.f, 0.f, 0.f};
-  auto mfma = [&](const f32x4(&fa)[4], const f32x4& v, float fl, float fr) {
-    if (do_b) bias_stage(bs, fa);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float b0 = j == 0 ? fl : v[j - 1];
-      const float b2 = j == 3 ? fr : v[j + 1];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        acc[i][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i][j], b0, acc[i][0], 0, 0, 0);
-        acc[i][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i][j], v[j], acc[i][1], 0, 0, 0);
-        acc[i][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i][j], b2, acc[i][2], 0, 0, 0);
-      }
-    }
-  };
-
-  f32x4 fa[D][4], fb[D];
-  float fl[D], fr[D];
-#pragma unroll
-  for (int s = 0; s < D - 1; ++s) load(fa[s], fb[s], fl[s], fr[s]);
-  int kt = 0;
-  for (; kt + D - 1 < nk; kt += D) {
-#pragma unroll
-    for (int s = 0; s < D; ++s) {
-      const int ls = (s + D - 1) % D;
-      load(fa[ls], fb[ls], fl[ls], fr[ls]);
-      __builtin_amdgcn_sched_barrier(0);
-      mfma(fa[s], fb[s], fl[s], fr[s]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-#pragma unroll
-  for (int s = 0; s < D - 1; ++s)
-    if (kt + s < nk) mfma(fa[s], fb[s], fl[s], fr[s]);
-
-  if (do_b) bias_store(c, bs, m0, split, lr, q);
-  // (i, r) is row m0 + 16 i + 4 q + r, columns 3 pair .. 3 pair + 2.
-  const __amdgpu_buffer_rsrc_t ro = make_rsrc(c.out, c.out_bytes);
-  const int ncol = 9 * c.cin;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = m0 + 16 * i + 4 * q + r;
-      const bool ok = pok && row < c.cout;
-      const uint32_t off = ok ? (uint32_t)(((split * c.cout + row) * ncol) + 3 * pair) * 4u : kOOB;
-      const f32x3 v = {acc[i][0][r], acc[i][1][r], acc[i][2][r]};
-      __builtin_amdgcn_raw_buffer_store_b96(__builtin_bit_cast(__attribute__((ext_vector_type(3))) unsigned, v), ro,
-                                            (int)off, 0, 0);
-    }
-}
-
-// Register-direct 1 x 1 weight gradient (stride 1, pad 0):
-//   dW[co][ci] = sum over pixels p of dy[co][p] * x[ci][p]
-// with the pixel splits, stages and dy loads of the 3 x 3 kernel.  Lane
-// (lr, q) owns the four columns ci0 .. ci0 + 3 (ci0 = the wave's first
-// column + 4 lr) as the four MFMA column blocks: one aligned float4 of x per
-// column per stage, and a 16-byte store per (block i, r).  The lane's pixel
-// advances 16 per stage with at most one image carry (H * W >= 16).  The
-// four waves are WM x WN blocks of 64 x 64 times KS = 4 / (WM WN) shares of
-// the split's stages (the host sizes WN to cin, so no wave computes columns
-// past cin); shares ks > 0 hand their blocks and bias sums to share 0
-// through LDS, which adds them in ks order.
-template <int WM, int WN, int D>
-__global__ __launch_bounds__(256, 2) void conv1_wgrad_kernel(Wgrad3Args c) {
-  constexpr int KS = 4 / (WM * WN);
-  static_assert(WM * WN * KS == 4, "four waves");
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int lr = lane & 15, q = lane >> 4;
-  const int wm = wave % WM, wn = (wave / WM) % WN, ks = wave / (WM * WN);
-  const int L = blockIdx.x, xq = c.items / 8, xr = c.items % 8, xc = L % 8;
-  const int item = xc * xq + min(xc, xr) + L / 8;
-  const int tile = item % c.tiles, split = item / c.tiles;
-  const int tm = tile % c.tiles_m, tn = tile / c.tiles_m;
-  const int m0 = (tm * WM + wm) * 64;
-  const int ci0 = (tn * WN + wn) * 64 + 4 * lr;
-  const bool cok = ci0 < c.cin;  // cin % 4 == 0: all four columns or none
-  // Share ks: pixels [kbeg, kend) of the split, whole 16-pixel stages.
-  const int sbeg = split * c.chunk, send = min(c.npix, sbeg + c.chunk);
-  const int nks = ((send - sbeg + 15) / 16 + KS - 1) / KS;
-  const int kbeg = min(send, sbeg + ks * nks * 16), kend = min(send, kbeg + nks * 16);
-  const int nk = (kend - kbeg + 15) / 16;
-  const __amdgpu_buffer_rsrc_t rx = make_rsrc(c.x, c.x_bytes);
-  const __amdgpu_buffer_rsrc_t rd = make_rsrc(c.dy, c.dy_bytes);
-  uint32_t a_row[4];
-  bool a_ok[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int co = m0 + 16 * i + lr;
-    a_ok[i] = co < c.cout;
-    a_row[i] = (uint32_t)(co * c.hw) * 4u;
-  }
-  const uint32_t x_lane = (uint32_t)(ci0 * c.hw) * 4u;
-  int P = kbeg + 4 * q, pp;
-  uint32_t dpix, xpix;
-  {
-    const int b = P / c.hw;
-    pp = P - b * c.hw;
-    dpix = (uint32_t)(b * c.cout * c.hw + pp) * 4u;
-    xpix = (uint32_t)(b * c.cin * c.hw + pp) * 4u;
-  }
-  const uint32_t d_img = (uint32_t)((c.cout - 1) * c.hw) * 4u, x_img = (uint32_t)((c.cin - 1) * c.hw) * 4u;
-  const uint32_t x_ch = (uint32_t)c.hw * 4u;
-
-  auto load = [&](f32x4(&fa)[4], f32x4(&fb)[4]) {
-    const bool pix = P < kend;
-    uint32_t ao[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ao[i] = (pix & a_ok[i]) ? a_row[i] + dpix : kOOB;
-    const uint32_t xo = (pix & cok) ? x_lane + xpix : kOOB;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      fa[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rd, (int)ao[i], 0, 0));
-#pragma unroll
-    for (int n = 0; n < 4; ++n)
-      fb[n] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(xo + n * x_ch), 0, 0));
-    P += 16;
-    pp += 16;
-    dpix += 64u;
-    xpix += 64u;
-    const bool cy = pp >= c.hw;
-    pp = cy ? pp - c.hw : pp;
-    dpix += cy ? d_img : 0u;
-    xpix += cy ? x_img : 0u;
-  };
-
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int n = 0; n < 4; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const bool do_b = c.db_mode != 0 && tn == 0 && wn == 0;
-  float bs[4] = {0.f, 0.f, 0.f, 0.f};
-  auto mfma = [&](const f32x4(&fa)[4], const f32x4(&fb)[4]) {
-    if (do_b) bias_stage(bs, fa);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int n = 0; n < 4; ++n)
-          acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i][j], fb[n][j], acc[i][n], 0, 0, 0);
-  };
-
-  f32x4 fa[D][4], fb[D][4];
-#pragma unroll
-  for (int s = 0; s < D - 1; ++s) load(fa[s], fb[s]);
-  int kt = 0;
-  for (; kt + D - 1 < nk; kt += D) {
-#pragma unroll
-    for (int s = 0; s < D; ++s) {
-      const int ls = (s + D - 1) % D;
-      load(fa[ls], fb[ls]);
-      __builtin_amdgcn_sched_barrier(0);
-      mfma(fa[s], fb[s]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-#pragma unroll
-  for (int s = 0; s < D - 1; ++s)
-    if (kt + s < nk) mfma(fa[s], fb[s]);
-
-  if (KS > 1) {
-    constexpr int RW = 64 * 64 + 4 * 64;  // a wave's block, then its bias sums
-    __shared__ float red[KS > 1 ? (KS - 1) * WM * WN * RW : 1];
-    const int blk = wave % (WM * WN);
-    if (ks > 0) {
-      float* dst = red + ((ks - 1) * WM * WN + blk) * RW + lane;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int n = 0; n < 4; ++n)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) dst[((i * 4 + n) * 4 + r) * 64] = acc[i][n][r];
-      if (do_b)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) dst[(64 + i) * 64] = bs[i];
-    }
-    __syncthreads();
-    if (ks > 0) return;
-#pragma unroll 1
-    for (int k = 1; k < KS; ++k) {
-      const float* src = red + ((k - 1) * WM * WN + blk) * RW + lane;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int n = 0; n < 4; ++n)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i][n][r] += src[((i * 4 + n) * 4 + r) * 64];
-      if (do_b)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) bs[i] += src[(64 + i) * 64];
-    }
-  }
-  if (do_b) bias_store(c, bs, m0, split, lr, q);
-  // (i, r) is row m0 + 16 i + 4 q + r, columns ci0 .. ci0 + 3.
-  const __amdgpu_buffer_rsrc_t ro = make_rsrc(c.out, c.out_bytes);
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = m0 + 16 * i + 4 * q + r;
-      const bool ok = cok && row < c.cout;
-      const uint32_t off = ok ? (uint32_t)((split * c.cout + row) * c.cin + ci0) * 4u : kOOB;
-      const f32x4 v = {acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]};
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ro, (int)off, 0, 0);
-    }
-}
-
-bool fits_2g(double elems) { return elems * 4.0 < 2147483647.0; }
 bool a16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 
 // 64-row blocks (M <= 64) split each block's stages over two waves, so the
-// grid still holds two waves per SIMD.
-template <bool DG, bool HALO, int WM>
+// grid still holds two waves per SIMD; the 3 x 3 kernel runs with them only
+// (direct_better).
+template <bool DG, bool HALO>
 void launch_conv3(hipStream_t s, const Conv3Args& c) {
-  constexpr int KS = WM == 1 ? 2 : 1;
-  mle::launch(conv3_direct_kernel<DG, HALO, WM, 2, KS, kC3U, kC3D>, c.tiles, 64 * WM * 2 * KS, 0, s, c);
+  mle::launch(conv3_direct_kernel<DG, HALO, 1, 2, 2, kC3U, kC3D>, c.tiles, 256, 0, s, c);
 }
 
 template <bool DG, int WM>
@@ -1332,6 +670,19 @@ bool direct_args(bool dg, const ConvGeom& g, const float* src, const float* wt, 
   return true;
 }
 
+// Where the register-direct fp32 kernels are still the faster ones (us, direct
+// against split-bf16): at most 64 rows of C, whose 64-wide tiles split each
+// element for few products (dgrad 16 x 64 <- 128 on 64 x 64: 79 / 95; forward
+// 32 x 32 -> 64 on 32 x 32: 17 / 22), except a forward of few tiles and some
+// depth, which two K groups share (16 x 64 -> 64 on 28 x 28: 27 / 20); and
+// 1 x 1 filters of at most 128 deep, bound by memory (16 x 64 -> 128 on 64 x 64:
+// 16 / 19).  Above that the split kernel wins (256 -> 256 on 32 x 32: 144 / 55).
+bool direct_better(bool dg, const ConvGeom& g) {
+  const int M = dg ? g.cin : g.cout, K = (dg ? g.cout : g.cin) * g.kh * g.kw;
+  if (g.kh == 1 && g.kw == 1 && K <= 128) return true;
+  return M <= 64 && (dg || K < 256 || !few_tiles(g));
+}
+
 // Register-direct path for one convolution (see direct_args).  Returns false,
 // launching nothing, when the shape is outside what the kernels assume.
 bool conv_direct(hipStream_t s, bool dg, const ConvGeom& g, const float* src, const float* wt, const float* bias,
@@ -1345,13 +696,8 @@ bool conv_direct(hipStream_t s, bool dg, const ConvGeom& g, const float* src, co
     else wm == 1 ? launch_conv1<false, 1>(s, c) : launch_conv1<false, 2>(s, c);
     return true;
   }
-  if (dg) {
-    if (halo) wm == 1 ? launch_conv3<true, true, 1>(s, c) : launch_conv3<true, true, 2>(s, c);
-    else wm == 1 ? launch_conv3<true, false, 1>(s, c) : launch_conv3<true, false, 2>(s, c);
-  } else {
-    if (halo) wm == 1 ? launch_conv3<false, true, 1>(s, c) : launch_conv3<false, true, 2>(s, c);
-    else wm == 1 ? launch_conv3<false, false, 1>(s, c) : launch_conv3<false, false, 2>(s, c);
-  }
+  if (dg) halo ? launch_conv3<true, true>(s, c) : launch_conv3<true, false>(s, c);
+  else halo ? launch_conv3<false, true>(s, c) : launch_conv3<false, false>(s, c);
   return true;
 }
 
@@ -1365,25 +711,6 @@ bool pair_geoms(int n, int cin, int h, int w, int cout3, int cout1, ConvGeom& g3
   return true;
 }
 
-template <bool HALO>
-void launch_pair_fwd(hipStream_t s, const Conv3Args& a, int wma, const Conv3Args& b, int wmb) {
-  const unsigned grid = (unsigned)(a.tiles + b.tiles);
-  if (wma == 1) {
-    if (wmb == 1) mle::launch(conv_pair_fwd_kernel<HALO, 1, 1>, grid, 256, 0, s, a, b);
-    else mle::launch(conv_pair_fwd_kernel<HALO, 1, 2>, grid, 256, 0, s, a, b);
-  } else {
-    if (wmb == 1) mle::launch(conv_pair_fwd_kernel<HALO, 2, 1>, grid, 256, 0, s, a, b);
-    else mle::launch(conv_pair_fwd_kernel<HALO, 2, 2>, grid, 256, 0, s, a, b);
-  }
-}
-
-template <int KIND>
-void launch_fast(hipStream_t s, const FastConv& c, int kh, int splits) {
-  dim3 grid((c.N + BN - 1) / BN, (c.M + BM - 1) / BM, splits);
-  if (kh == 3) mle::launch(conv_fast_kernel<KIND, 3, 3>, grid, NT, 0, s, c);
-  else mle::launch(conv_fast_kernel<KIND, 1, 1>, grid, NT, 0, s, c);
-}
-
 int geom(int n, int cin, int h, int w, int cout, int kh, int kw, int pad, int stride, ConvGeom& g) {
   if (n <= 0 || cin <= 0 || h <= 0 || w <= 0 || cout <= 0 || kh <= 0 || kw <= 0 || pad < 0 || stride <= 0)
     return set_error(MLE_ERR_INVALID, "conv2d: bad geometry");
@@ -1394,88 +721,6 @@ int geom(int n, int cin, int h, int w, int cout, int kh, int kw, int pad, int st
   if (big >= 2147483647.0 || bigo >= 2147483647.0)
     return set_error(MLE_ERR_UNSUPPORTED, "conv2d: tensor exceeds 2^31 elements");
   return MLE_OK;
-}
-
-bool fast_filter(const ConvGeom& g) {
-  return g.stride == 1 && ((g.kh == 3 && g.kw == 3) || (g.kh == 1 && g.kw == 1));
-}
-
-// Workgroups of `kernel` (256 threads) resident at once on the current
-// device (per-CU occupancy x CUs), cached per device in `cache`.
-template <class K>
-int resident_wgs(K kernel, int (&cache)[64]) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 768;
-  int& v = cache[dev];
-  if (v <= 0) {
-    int cus = 0, per_cu = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, 0) != hipSuccess || per_cu <= 0) per_cu = 2;
-    v = per_cu * cus;
-  }
-  return v;
-}
-
-// Workgroups of the weight-gradient kernel for (taps, wm, wn) resident at
-// once (3 x 256 on MI355X for the 3 x 3 kernel).  One full round of resident
-// workgroups measured fastest: at 512 workgroups on 768 slots some CUs hold
-// 1 and others 3 (54 % of fp32 MFMA for the C5 weight gradients), at 768
-// every CU holds 3 (77 %), at 1024 the last 256 run as a tail (62 %).
-int wgrad_slots(int taps, int wm, int wn) {
-  static int c3[2][64], c1[5][64];
-  if (taps == 9)
-    return wm == 1 ? resident_wgs(conv3_wgrad_kernel<1, 3>, c3[0]) : resident_wgs(conv3_wgrad_kernel<2, 3>, c3[1]);
-  if (wm == 1)
-    return wn == 4 ? resident_wgs(conv1_wgrad_kernel<1, 4, 4>, c1[0])
-                   : (wn == 2 ? resident_wgs(conv1_wgrad_kernel<1, 2, 4>, c1[1])
-                              : resident_wgs(conv1_wgrad_kernel<1, 1, 4>, c1[2]));
-  return wn == 2 ? resident_wgs(conv1_wgrad_kernel<2, 2, 4>, c1[3]) : resident_wgs(conv1_wgrad_kernel<2, 1, 4>, c1[4]);
-}
-
-// Register-direct weight gradient plan: 3 x 3 (stride 1, pad 1, W >= 16)
-// in 128 x 96 tiles of C (64 x 192 when cout <= 64), or 1 x 1 (stride 1,
-// pad 0, cin % 4 == 0, H * W >= 16) in 64 wm x 64 wn tiles (wm = 1 when
-// cout <= 64, else 2; wn the smallest power of two up to 4 / wm whose
-// columns cover cin, the remaining waves sharing the pixels); the pixels
-// split so that tiles x splits fills one round of resident workgroups, each
-// split a whole number of 16-pixel stages and at least 256 pixels.  Returns
-// false when the shape is outside what the kernels assume.
-bool wgrad_plan(const ConvGeom& g, Wgrad3Args& c, int& taps, int& wm, int& wn) {
-  const bool k3 = g.kh == 3 && g.kw == 3 && g.pad == 1 && g.stride == 1 && g.w % 4 == 0 && g.w >= 16;
-  const bool k1 = g.kh == 1 && g.kw == 1 && g.pad == 0 && g.stride == 1 && (g.h * g.w) % 4 == 0 &&
-                  g.h * g.w >= 16 && g.cin % 4 == 0;
-  if (!k3 && !k1) return false;
-  taps = k3 ? 9 : 1;
-  const double hw = (double)g.h * g.w;
-  if ((double)g.n * g.cin * hw * 4.0 >= 2147483647.0 || (double)g.n * g.cout * hw * 4.0 >= 2147483647.0) return false;
-  c = Wgrad3Args{};
-  c.cout = g.cout;
-  c.cin = g.cin;
-  c.h = g.h;
-  c.w = g.w;
-  c.hw = g.h * g.w;
-  c.npix = g.n * c.hw;
-  wm = g.cout <= 64 ? 1 : 2;
-  wn = 4 / wm;
-  if (k1)
-    while (wn > 1 && 64 * (wn / 2) >= g.cin) wn /= 2;
-  c.tiles_m = (g.cout + 64 * wm - 1) / (64 * wm);
-  c.tiles = c.tiles_m * (k3 ? (3 * g.cin + 16 * wn - 1) / (16 * wn) : (g.cin + 64 * wn - 1) / (64 * wn));
-  const int slots = wgrad_slots(taps, wm, wn);
-  int splits = std::max(1, slots / c.tiles);
-  // At least 256 pixels per split: the C5 1 x 1 weight gradient (65536
-  // pixels) ran 25.1 us with 256-pixel splits and 32.6 us with 128 or fewer,
-  // where the partials' reduce grows faster than the kernel shrinks.
-  const int max_splits = (c.npix + 255) / 256;
-  splits = std::max(1, std::min(splits, max_splits));
-  c.chunk = ((c.npix + splits - 1) / splits + 15) / 16 * 16;
-  splits = (c.npix + c.chunk - 1) / c.chunk;
-  c.items = c.tiles * splits;
-  if ((double)splits * g.cout * g.cin * taps * 4.0 >= 2147483647.0) return false;
-  c.x_bytes = (uint32_t)((size_t)g.n * g.cin * c.hw * 4);
-  c.dy_bytes = (uint32_t)((size_t)g.n * g.cout * c.hw * 4);
-  c.out_bytes = (uint32_t)((size_t)splits * g.cout * g.cin * taps * 4);
-  return true;
 }
 
 // K split for wgrad: aim for >= ~512 workgroups, chunks of whole BK slices.
@@ -1493,6 +738,20 @@ int wgrad_splits(const ConvGeom& g, int& kchunk) {
   return splits;
 }
 
+// One convolution's forward and input gradient on whichever kernel takes it.
+void conv_fwd_any(hipStream_t s, const ConvGeom& g, const float* x, const float* w, const float* b, float* y) {
+  if (direct_better(false, g) && conv_direct(s, false, g, x, w, b, y, 0)) return;
+  if (split_fwd(s, g, x, w, b, y)) return;
+  const FwdOps op{x, w, b, y, g, g.cout, g.n * g.oh * g.ow, g.cin * g.kh * g.kw};
+  mle::launch(igemm_kernel<FwdOps, false>, dim3((op.N + BN - 1) / BN, (op.M + BM - 1) / BM, 1), NT, 0, s, op, op.K);
+}
+void conv_dgrad_any(hipStream_t s, const ConvGeom& g, const float* dy, const float* w, float* dx, int acc) {
+  if (direct_better(true, g) && conv_direct(s, true, g, dy, w, nullptr, dx, acc)) return;
+  if (split_dgrad(s, g, dy, w, dx, acc)) return;
+  const DgradOps op{dy, w, dx, g, g.cin, g.n * g.h * g.w, g.cout * g.kh * g.kw, acc};
+  mle::launch(igemm_kernel<DgradOps, false>, dim3((op.N + BN - 1) / BN, (op.M + BM - 1) / BM, 1), NT, 0, s, op, op.K);
+}
+
 }  // namespace
 
 extern "C" {
@@ -1503,20 +762,9 @@ int mle_conv2d_fwd(mle_stream stream, const float* x, const float* w, const floa
   ConvGeom g;
   int rc = geom(n, cin, h, w_in, cout, kh, kw, pad, stride, g);
   if (rc) return rc;
-  FwdOps op{x, w, b, y, g, cout, n * g.oh * g.ow, cin * kh * kw};
   hipStream_t s = as_stream(stream);
-  ProbeScope probe("conv_fwd", s, 2.0 * op.M * (double)op.N * op.K, 0.0);
-  const int ohw = g.oh * g.ow;
-  if (conv_direct(s, false, g, x, w, b, y, 0)) {
-  } else if (fast_filter(g) && ohw % 4 == 0 && op.K % 4 == 0 && a16(y) && fits_2g((double)n * cin * h * w_in) &&
-      fits_2g((double)n * cout * ohw) && fits_2g((double)cout * op.K)) {
-    FastConv c{x, w, b, y, (uint32_t)((size_t)n * cin * h * w_in * 4), (uint32_t)((size_t)cout * op.K * 4),
-               op.M, op.N, op.K, op.K, cin, h, w_in, h * w_in, g.oh, g.ow, ohw, pad, cout, cin, 0};
-    launch_fast<CONV_FWD>(s, c, kh, 1);
-  } else {
-    dim3 grid((op.N + BN - 1) / BN, (op.M + BM - 1) / BM, 1);
-    mle::launch(igemm_kernel<FwdOps, false>, grid, NT, 0, s, op, op.K);
-  }
+  ProbeScope probe("conv_fwd", s, 2.0 * cout * (double)n * g.oh * g.ow * cin * kh * kw, 0.0);
+  conv_fwd_any(s, g, x, w, b, y);
   return check_launch("mle_conv2d_fwd");
 }
 
@@ -1526,32 +774,17 @@ int mle_conv2d_dgrad(mle_stream stream, const float* dy, const float* w, float* 
   ConvGeom g;
   int rc = geom(n, cin, h, w_in, cout, kh, kw, pad, stride, g);
   if (rc) return rc;
-  DgradOps op{dy, w, dx, g, cin, n * h * w_in, cout * kh * kw, accumulate != 0};
   hipStream_t s = as_stream(stream);
-  ProbeScope probe("conv_dgrad", s, 2.0 * op.M * (double)op.N * op.K, 0.0);
-  const int hw = h * w_in;
-  if (conv_direct(s, true, g, dy, w, nullptr, dx, accumulate != 0)) {
-  } else if (fast_filter(g) && hw % 4 == 0 && a16(dx) && fits_2g((double)n * cin * hw) &&
-      fits_2g((double)n * cout * g.oh * g.ow) && fits_2g((double)cout * cin * kh * kw)) {
-    FastConv c{dy, w, nullptr, dx, (uint32_t)((size_t)n * cout * g.oh * g.ow * 4),
-               (uint32_t)((size_t)cout * cin * kh * kw * 4), op.M, op.N, op.K, op.K, cout, g.oh, g.ow, g.oh * g.ow,
-               h, w_in, hw, pad, cout, cin, accumulate != 0};
-    launch_fast<CONV_DGRAD>(s, c, kh, 1);
-  } else {
-    dim3 grid((op.N + BN - 1) / BN, (op.M + BM - 1) / BM, 1);
-    mle::launch(igemm_kernel<DgradOps, false>, grid, NT, 0, s, op, op.K);
-  }
+  ProbeScope probe("conv_dgrad", s, 2.0 * cin * (double)n * h * w_in * cout * kh * kw, 0.0);
+  conv_dgrad_any(s, g, dy, w, dx, accumulate != 0);
   return check_launch("mle_conv2d_dgrad");
 }
 
 size_t mle_conv2d_wgrad_ws_bytes(int n, int cin, int h, int w_in, int cout, int kh, int kw, int pad, int stride) {
   ConvGeom g;
   if (geom(n, cin, h, w_in, cout, kh, kw, pad, stride, g) != MLE_OK) return 0;
-  Wgrad3Args c3;
-  int taps, wm, wn;
-  // Split partials of dW, then (mle_conv2d_wgrad_bias) those of db.
-  if (wgrad_plan(g, c3, taps, wm, wn))
-    return c3.items > c3.tiles ? (size_t)c3.out_bytes + (size_t)(c3.items / c3.tiles) * cout * sizeof(float) : 0;
+  if (const int sp = split_wgrad_splits(g))
+    return sp > 1 ? (size_t)sp * ((size_t)cout * cin * kh * kw + cout) * sizeof(float) : 0;
   int kchunk;
   const int splits = wgrad_splits(g, kchunk);
   return (size_t)splits * cout * cin * kh * kw * sizeof(float);
@@ -1574,37 +807,13 @@ int mle_conv2d_wgrad_bias(mle_stream stream, const float* x, const float* dy, fl
   if (ws_bytes < need || (need > 0 && !ws)) return set_error(MLE_ERR_WORKSPACE, "mle_conv2d_wgrad: workspace too small");
   hipStream_t s = as_stream(stream);
   const double flop = 2.0 * cout * (double)cin * kh * kw * (double)n * g.oh * g.ow;
-  Wgrad3Args c3;
-  int taps, wm, wn;
-  if (wgrad_plan(g, c3, taps, wm, wn)) {
-    const int splits = c3.items / c3.tiles;
-    c3.x = x;
-    c3.dy = dy;
-    c3.out = splits > 1 ? static_cast<float*>(ws) : dw;
-    if (splits == 1) c3.out_bytes = (uint32_t)((size_t)cout * cin * taps * 4);
-    const size_t mn = (size_t)cout * cin * taps;
-    float* bpart = splits > 1 ? static_cast<float*>(ws) + (size_t)splits * mn : nullptr;
-    c3.db = db;
-    c3.bpart = bpart;
-    c3.db_mode = db ? (splits > 1 ? 2 : (accumulate_db ? 1 : 3)) : 0;
-    {
-      ProbeScope probe("conv_wgrad", s, flop, 0.0);
-      if (taps == 9) {
-        if (wm == 1) mle::launch(conv3_wgrad_kernel<1, 3>, c3.items, 256, 0, s, c3);
-        else mle::launch(conv3_wgrad_kernel<2, 3>, c3.items, 256, 0, s, c3);
-      } else if (wm == 1) {
-        if (wn == 4) mle::launch(conv1_wgrad_kernel<1, 4, 4>, c3.items, 256, 0, s, c3);
-        else if (wn == 2) mle::launch(conv1_wgrad_kernel<1, 2, 4>, c3.items, 256, 0, s, c3);
-        else mle::launch(conv1_wgrad_kernel<1, 1, 4>, c3.items, 256, 0, s, c3);
-      } else {
-        if (wn == 2) mle::launch(conv1_wgrad_kernel<2, 2, 4>, c3.items, 256, 0, s, c3);
-        else mle::launch(conv1_wgrad_kernel<2, 1, 4>, c3.items, 256, 0, s, c3);
-      }
-      // The reduce that completes dW and db is part of the probed family.
-      if (splits > 1)
-        launch_split_reduce(s, static_cast<const float*>(ws), splits, mn, dw, bpart, db ? cout : 0, db,
-                            accumulate_db);
-    }
+  if (const int sp = split_wgrad_splits(g)) {
+    const size_t mn = (size_t)cout * cin * kh * kw;
+    float* part = static_cast<float*>(ws);
+    ProbeScope probe("conv_wgrad", s, flop, 0.0);
+    split_wgrad(s, g, x, dy, dw, db, accumulate_db, part, sp);
+    // The reduce that completes dW and db is part of the probed family.
+    if (sp > 1) launch_split_reduce(s, part, sp, mn, dw, part + (size_t)sp * mn, db ? cout : 0, db, accumulate_db);
     return check_launch("mle_conv2d_wgrad");
   }
   int kchunk;
@@ -1612,17 +821,8 @@ int mle_conv2d_wgrad_bias(mle_stream stream, const float* x, const float* dy, fl
   WgradOps op{x, dy, static_cast<float*>(ws), g, cout, cin * kh * kw, n * g.oh * g.ow};
   {
     ProbeScope probe("conv_wgrad", s, 2.0 * op.M * (double)op.N * op.K, 0.0);
-    const int ohw = g.oh * g.ow;
-    if (fast_filter(g) && ohw % 4 == 0 && ohw >= BK && op.N % 4 == 0 && a16(ws) &&
-        fits_2g((double)n * cin * h * w_in) && fits_2g((double)n * cout * ohw)) {
-      FastConv c{x, dy, nullptr, static_cast<float*>(ws), (uint32_t)((size_t)n * cin * h * w_in * 4),
-                 (uint32_t)((size_t)n * cout * ohw * 4), op.M, op.N, op.K, kchunk, cin, h, w_in, h * w_in,
-                 g.oh, g.ow, ohw, pad, cout, cin, 0};
-      launch_fast<CONV_WGRAD>(s, c, kh, splits);
-    } else {
-      dim3 grid((op.N + BN - 1) / BN, (op.M + BM - 1) / BM, splits);
-      mle::launch(igemm_kernel<WgradOps, true>, grid, NT, 0, s, op, kchunk);
-    }
+    dim3 grid((op.N + BN - 1) / BN, (op.M + BM - 1) / BM, splits);
+    mle::launch(igemm_kernel<WgradOps, true>, grid, NT, 0, s, op, kchunk);
     launch_split_reduce(s, static_cast<const float*>(ws), splits, (size_t)op.M * op.N, dw);
   }
   rc = check_launch("mle_conv2d_wgrad");
@@ -1675,8 +875,10 @@ int mle_conv2d_pair_fwd(mle_stream stream, const float* x, int n, int cin, int h
   hipStream_t s = as_stream(stream);
   const double flop = 2.0 * (double)n * h * w * cin * (9.0 * cout3 + cout1);
   ProbeScope probe("conv_fwd", s, flop, 0.0);
-  if (halo) launch_pair_fwd<true>(s, a, wma, b, wmb);
-  else launch_pair_fwd<false>(s, a, wma, b, wmb);
+  ConvGeom g3, g1;
+  pair_geoms(n, cin, h, w, cout3, cout1, g3, g1);
+  conv_fwd_any(s, g3, x, w3, b3, y3);
+  conv_fwd_any(s, g1, x, w1, b1, y1);
   return check_launch("mle_conv2d_pair_fwd");
 }
 
@@ -1692,9 +894,14 @@ int mle_conv2d_pair_dgrad(mle_stream stream, float* dx, int accumulate, int n, i
   hipStream_t s = as_stream(stream);
   const double flop = 2.0 * (double)n * h * w * cin * (9.0 * cout3 + cout1);
   ProbeScope probe("conv_dgrad", s, flop, 0.0);
-  auto k = halo ? (wma == 1 ? conv_pair_dgrad_kernel<true, 1> : conv_pair_dgrad_kernel<true, 2>)
-                : (wma == 1 ? conv_pair_dgrad_kernel<false, 1> : conv_pair_dgrad_kernel<false, 2>);
-  mle::launch(k, (unsigned)a.tiles, 256, 0, s, a, b);
+  if (wma == 1) {  // one launch, dx written once
+    mle::launch(halo ? conv_pair_dgrad_kernel<true> : conv_pair_dgrad_kernel<false>, (unsigned)a.tiles, 256, 0, s, a, b);
+  } else {
+    ConvGeom g3, g1;
+    pair_geoms(n, cin, h, w, cout3, cout1, g3, g1);
+    conv_dgrad_any(s, g3, dy3, w3, dx, accumulate != 0);
+    conv_dgrad_any(s, g1, dy1, w1, dx, 1);
+  }
   return check_launch("mle_conv2d_pair_dgrad");
 }
 

@@ -553,31 +553,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_ksplit_pair_kernel(GemmArgs g0, 
 // of its time in us -- rounds of workgroups times (stages x time of a stage +
 // prologue and epilogue), plus the reduce of the partial products.  A function
 // of the shape only, as mle_gemm_ws_bytes needs.
-//
-// Measured on MI355X under sustained load, us per stage and per tile beside
-// them, a whole round of 256 workgroups: large 2.6 + 8.5 (2.3 in short runs,
-// before the power limit lowers the clock), medium 1.75 + 6, small 0.75 + 4.5
-// alone on a CU and 0.55 + 3 a piece when three share it.
-constexpr double kStageUs[3] = {2.6, 1.75, 0.75}, kTileUs[3] = {8.5, 6.0, 4.5};
-constexpr double kSharedStageUs = 0.55, kSharedTileUs = 3.0;
-constexpr int kChipCus = 256;
-
 struct SplitChoice {
   int tile = kSplitLarge, splits = 1, kchunk = 0;
   double us = 0;
 };
-
-long long tiles_of(int tile, int M, int N) {
-  return (long long)((M + kSplitTm[tile] - 1) / kSplitTm[tile]) * ((N + kSplitTn[tile] - 1) / kSplitTn[tile]);
-}
-
-// Time of n workgroups of `stages` stages each on tile shape `tile`.
-double grid_us(int tile, long long n, int stages) {
-  const long long per = (n + kChipCus - 1) / kChipCus;  // workgroups per CU
-  const double alone = stages * kStageUs[tile] + kTileUs[tile];
-  if (tile != kSplitSmall) return (double)per * alone;
-  return std::max(alone, (double)per * (stages * kSharedStageUs + kSharedTileUs));
-}
 
 SplitChoice choose_split(int M, int N, int K, int batch, bool may_split) {
   SplitChoice best;
@@ -597,8 +576,9 @@ SplitChoice choose_split(int M, int N, int K, int batch, bool may_split) {
       last = sp;
       int depth = (int)((st + sp - 1) / sp);
       sp = (st + depth - 1) / depth;
-      double us = grid_us(tile, tiles * sp, depth);
-      if (sp > 1) us += 5.0 + (double)(sp + 1) * M * N * batch * 4.0 / 4.0e6;
+      double us = split_grid_us(tile, tiles * sp, depth);
+      // the reduce: 5 us and its bytes, element by element where rows are no multiple of 4
+      if (sp > 1) us += 5.0 + (double)(sp + 1) * M * N * batch * 4.0 / (N % 4 == 0 ? 4.0e6 : 1.5e6);
       if (us < best.us) best = {tile, (int)sp, sp > 1 ? depth * 32 : K, us};
     }
   }
@@ -714,7 +694,10 @@ static int gemm_plan(GemmPlan& P, int trans_a, int trans_b, int M, int N, int K,
   // Folded terms end on whole stages unless both operands are k-contiguous
   // (whose last stage is masked).
   const bool fold = K % 32 == 0 || (!trans_a && trans_b);
-  SplitChoice ch = choose_split(M, N, K, batch, ws != nullptr && terms <= 1);
+  const bool simple = simple_shape(M, N, K, batch, inner, terms);
+  const bool ksplit = !simple && ksplit_shape(M, N, K, batch, terms);
+  SplitChoice ch;
+  if (!simple && !ksplit && terms <= 1) ch = choose_split(M, N, K, batch, ws != nullptr);
   if (terms > 1) ch = choose_split(M, N, (int)std::min(2147483000.0, (double)K * terms), batch, false);
   const double items = (double)tiles_of(ch.tile, M, N) * batch * std::max(ch.splits, std::max(terms, 1));
   split = split && items < 1073741824.0;
@@ -743,12 +726,12 @@ static int gemm_plan(GemmPlan& P, int trans_a, int trans_b, int M, int N, int K,
       g.part_cs = g.part + (size_t)ch.splits * batch * M * N;
     }
   }
-  if (simple_shape(M, N, K, batch, inner, terms)) {
+  if (simple) {
     g.splits = 1;
     g.kchunk = K;
     g.part = g.part_cs = nullptr;
     P.simple = true;
-  } else if (ksplit_shape(M, N, K, batch, terms)) {
+  } else if (ksplit) {
     g.splits = 1;
     g.kchunk = K;
     g.part = g.part_cs = nullptr;
@@ -1062,7 +1045,11 @@ extern "C" {
 size_t mle_linear_bwd_ws_bytes(int rows, int in, int out, int layers) {
   const size_t dx = layers > 1 ? mle_gemm_sum_ws_bytes(rows, in, layers) : mle_gemm_ws_bytes(rows, in, out, 1);
   size_t dw = mle_gemm_ws_bytes(in, out, rows, layers);
-  const PairChoice pc = choose_pair(rows, in, out, layers);
+  // (a product on a small-product kernel never shares a launch with a split one)
+  const bool small = simple_shape(rows, in, out, 1, 1, layers > 1 ? layers : 0) || ksplit_shape(rows, in, out, 1, layers > 1 ? layers : 0) ||
+                     simple_shape(in, out, rows, layers, 1, 0) || ksplit_shape(in, out, rows, layers, 0);
+  PairChoice pc;
+  if (!small) pc = choose_pair(rows, in, out, layers);
   if (pc.splits > 1) dw = std::max(dw, (size_t)pc.splits * layers * ((size_t)in * out + out) * sizeof(float));
   return std::max(dx, dw);
 }

@@ -2,6 +2,8 @@
 #pragma once
 #include "common.hpp"
 
+#include <algorithm>
+
 namespace gemm {
 
 struct GemmArgs {
@@ -64,6 +66,28 @@ struct GemmArgs {
 // Tile shapes of the split kernel (split_core.hpp), and a launch of it.
 enum SplitTile { kSplitLarge = 0, kSplitMedium = 1, kSplitSmall = 2 };
 constexpr int kSplitTm[3] = {256, 128, 64}, kSplitTn[3] = {128, 128, 64};
+// Time model of a grid of them.
+// Measured on MI355X over 33 products of 100 .. 8192 rows, columns and depth, us
+// per stage and per tile for a round of at most 256 workgroups: large 2.3 + 8
+// (+ 13 where a round follows another: every workgroup writes its 128 KB of C
+// at once), medium 1.4 + 5.5, small 0.53 + 4.5 (one workgroup per CU, two K
+// groups); 0.53 + 1.7 for each small tile of a CU that several share.
+constexpr double kStageUs[3] = {2.3, 1.4, 0.53}, kTileUs[3] = {8.0, 5.5, 4.5};
+constexpr double kFullTileUs = 13.0, kSharedTileUs = 1.7;
+constexpr int kChipCus = 256;
+
+inline long long tiles_of(int tile, int M, int N) {
+  return (long long)((M + kSplitTm[tile] - 1) / kSplitTm[tile]) * ((N + kSplitTn[tile] - 1) / kSplitTn[tile]);
+}
+
+// Time of n workgroups of `stages` stages each on tile shape `tile`.
+inline double split_grid_us(int tile, long long n, int stages) {
+  const long long per = (n + kChipCus - 1) / kChipCus;  // workgroups per CU
+  if (per == 1) return stages * kStageUs[tile] + kTileUs[tile];
+  const double t = tile == kSplitLarge ? kFullTileUs : tile == kSplitMedium ? kTileUs[tile] : kSharedTileUs;
+  return (double)per * (stages * kStageUs[tile] + t) + (tile == kSplitSmall ? 3.0 : 0.0);
+}
+
 // trans: 2 * trans_a + trans_b.  tail: K % 4 != 0 beside a k-contiguous operand
 // (kEpiPlain only).  epi: kEpi*.
 void launch_split(hipStream_t s, int trans, const GemmArgs& g, int tile, bool tail, bool colsum, int epi, int gx, int gy,

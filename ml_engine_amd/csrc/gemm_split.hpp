@@ -1,27 +1,13 @@
 // The split-bf16 GEMM (split_core.hpp): C = alpha op(A) op(B) + beta C with the
 // epilogues of gemm_args.hpp.  Included by gemm_split_*.hip, which
 // instantiate the layouts.
-//
-// Tiles (workgroup of C, waves, LDS): large 256 x 128, 8 waves of 64 x 64,
-// 147 KB; medium 128 x 128, 8 waves of 32 x 64, 98 KB; small 64 x 64, 4 waves
-// of 32 x 32, 49 KB (three workgroups per CU).  What bounds the large tile on
-// full grids is power: 1.3 PFLOP/s of bf16 MFMA at a clock of about 1.75 GHz,
-// of whose cycles the matrix cores are busy three quarters.
 #pragma once
 #include "activation.hpp"
-#include "gemm_args.hpp"
-#include "split_core.hpp"
+#include "gemm_tiles.hpp"
 
 #include <float.h>
 
 namespace gemm {
-
-using LargeTile = split::Shape<4, 4, 4, 2>;
-using MediumTile = split::Shape<2, 4, 4, 2>;
-using SmallTile = split::Shape<2, 2, 2, 2>;
-static_assert(LargeTile::TM == kSplitTm[0] && LargeTile::TN == kSplitTn[0] && MediumTile::TM == kSplitTm[1] &&
-                  MediumTile::TN == kSplitTn[1] && SmallTile::TM == kSplitTm[2] && SmallTile::TN == kSplitTn[2],
-              "tile table");
 
 // One tile (tm, tn) of batch item / K split bz.
 template <class S, int TA, int TB, bool TAIL, bool COLSUM, int EPI>
@@ -38,15 +24,18 @@ __device__ __forceinline__ void split_tile(const GemmArgs& g, int tm, int tn, in
   float* C = g.C + batch_off(z, g, g.sc, g.sc2);
   const int kbeg = g.grouped ? 0 : part * g.kchunk;
   const int klen = (g.grouped ? g.K : min(g.K, kbeg + g.kchunk)) - kbeg;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, group = split::k_group<S>(), t = tid % S::NTH;
   f32x4 v[BI][BN], lo[BI][BN];
   split::Tiny tiny;
   {
     LA la;
     LB lb;
-    la.init(A, g.lda, g.M, g.K, m0, kbeg, klen, g.kterms, g.gsa, tid);
-    lb.init(B, g.ldb, g.N, g.K, n0, kbeg, klen, g.kterms, g.gsb, tid);
-    split::mma_loop<S>(lds, la, lb, g.kterms * ((klen + split::KS - 1) / split::KS), v, lo, tiny);
+    // With two K groups (kterms == 1) each takes half of the stages.
+    const int nk = ((klen + split::KS - 1) / split::KS + S::KG - 1) / S::KG;
+    const int k0 = group * nk * split::KS, kl = S::KG == 1 ? klen : min(klen - k0, nk * split::KS);
+    la.init(A, g.lda, g.M, g.K, m0, kbeg + k0, kl, g.kterms, g.gsa, t);
+    lb.init(B, g.ldb, g.N, g.K, n0, kbeg + k0, kl, g.kterms, g.gsb, t);
+    split::mma_loop<S>(lds + group * S::LDS, la, lb, g.kterms * nk, v, lo, tiny);
     if (COLSUM && tm == 0) {
       // the lane groups' sums of each column, added in order
       float* red = reinterpret_cast<float*>(lds);
@@ -54,18 +43,23 @@ __device__ __forceinline__ void split_tile(const GemmArgs& g, int tm, int tn, in
 #pragma unroll
       for (int c = 0; c < LB::NC; ++c) {
         int r, q;
-        LB::unit(tid, c, r, q);
-        red[q * S::TN + r] = lb.sum[c];
+        LB::unit(t, c, r, q);
+        red[(4 * group + q) * S::TN + r] = lb.sum[c];
       }
       __syncthreads();
       if (tid < S::TN && n0 + tid < g.N) {
-        const float cs = ((red[tid] + red[S::TN + tid]) + red[2 * S::TN + tid]) + red[3 * S::TN + tid];
+        float cs = red[tid];
+#pragma unroll
+        for (int q = 1; q < 4 * S::KG; ++q) cs += red[q * S::TN + tid];
         if (g.splits > 1) g.part_cs[(int64_t)bz * g.N + n0 + tid] = cs;
         else put_colsum(g, z * g.scs + n0 + tid, cs);
       }
     }
   }
-  if (__syncthreads_or(split::needs_fp32<S>(v, lo, tiny))) {
+  const bool redo = __syncthreads_or(split::needs_fp32<S>(v, lo, tiny));
+  split::join_groups<S>(lds, v, lo);
+  if (group != 0) return;  // (no barrier follows)
+  if (redo) {
 #pragma unroll
     for (int i = 0; i < BI; ++i)
 #pragma unroll
@@ -203,8 +197,8 @@ __device__ __forceinline__ void split_tile(const GemmArgs& g, int tm, int tn, in
 }
 
 template <class S, int TA, int TB, bool TAIL, bool COLSUM, int EPI>
-__global__ __launch_bounds__(S::NTH, 2) void gemm_split_kernel(GemmArgs g, int gx, int gy, int items) {
-  __shared__ __attribute__((aligned(16))) char lds[S::LDS];
+__global__ __launch_bounds__(S::NTH * S::KG, 2) void gemm_split_kernel(GemmArgs g, int gx, int gy, int items) {
+  __shared__ __attribute__((aligned(16))) char lds[S::LDS * S::KG];
   int tm, tn, z;
   item_tile(blockIdx.x, items, gx, gy, tm, tn, z);
   split_tile<S, TA, TB, TAIL, COLSUM, EPI>(g, tm, tn, z, lds);
@@ -216,8 +210,12 @@ void launch_split_tile(hipStream_t s, const GemmArgs& g, int tile, int gx, int g
     mle::launch(gemm_split_kernel<LargeTile, TA, TB, TAIL, COLSUM, EPI>, dim3((unsigned)items), LargeTile::NTH, 0, s, g, gx, gy, items);
   else if (tile == kSplitMedium)
     mle::launch(gemm_split_kernel<MediumTile, TA, TB, TAIL, COLSUM, EPI>, dim3((unsigned)items), MediumTile::NTH, 0, s, g, gx, gy, items);
-  else if constexpr (EPI == kEpiPlain)
-    mle::launch(gemm_split_kernel<SmallTile, TA, TB, TAIL, COLSUM, EPI>, dim3((unsigned)items), SmallTile::NTH, 0, s, g, gx, gy, items);
+  else if constexpr (EPI == kEpiPlain) {
+    if (items <= kChipCus && g.kterms == 1)
+      mle::launch(gemm_split_kernel<PairedTile, TA, TB, TAIL, COLSUM, EPI>, dim3((unsigned)items), PairedTile::NTH * PairedTile::KG, 0, s, g, gx, gy, items);
+    else
+      mle::launch(gemm_split_kernel<SmallTile, TA, TB, TAIL, COLSUM, EPI>, dim3((unsigned)items), SmallTile::NTH, 0, s, g, gx, gy, items);
+  }
 }
 
 }  // namespace gemm

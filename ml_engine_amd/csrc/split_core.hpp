@@ -27,8 +27,8 @@
 // Tile engine: a workgroup of CM x CN waves, each (16 BI) x (16 BN) of C.
 // 32-deep K stages, double-buffered in LDS as three bf16 planes per operand.
 // While the MFMAs of stage t run, every thread splits its share of stage
-// t + 1 (raw fp32 in registers, loaded a stage earlier) and writes it to the
-// other buffer, then issues the loads of stage t + 2.  The barrier sits
+// t + 1 (raw fp32 in registers, loaded DEPTH stages earlier) and writes it to
+// the other buffer, then issues the loads of stage t + 1 + DEPTH.  The barrier sits
 // before the last row block's MFMAs, so the first fragments of the next
 // stage arrive under them.
 //
@@ -112,9 +112,12 @@ __device__ __forceinline__ uint32_t slot(int r, int q) {
   return (uint32_t)((r >> 6) * 4096 + b * 1024 + q * 256 + ((p ^ (q + 4 * b)) * 16));
 }
 
-template <int BI_, int BN_, int CM_, int CN_>
+// DEPTH: raw register sets, i.e. how many stages ahead of the splitting the
+// loads run.  KG: groups of CM x CN waves that share the tile's K, each with
+// its own buffers (NTH and LDS are a group's); join_groups adds their sums.
+template <int BI_, int BN_, int CM_, int CN_, int DEPTH_ = 1, int KG_ = 1>
 struct Shape {
-  static constexpr int BI = BI_, BN = BN_, CM = CM_, CN = CN_;
+  static constexpr int BI = BI_, BN = BN_, CM = CM_, CN = CN_, DEPTH = DEPTH_, KG = KG_;
   static constexpr int TM = 16 * BI * CM, TN = 16 * BN * CN, NTH = 64 * CM * CN;
   static constexpr int PA = TM * 64, PB = TN * 64;  // bytes of one plane
   static constexpr int STAGE = 3 * (PA + PB), LDS = 2 * STAGE;
@@ -129,7 +132,7 @@ struct WaveMap {
   int lane, lr, q, wm, wn;
   __device__ __forceinline__ WaveMap() {
     const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) % (S::CM * S::CN);
     lane = tid & 63;
     lr = lane & 15;
     q = lane >> 4;
@@ -147,9 +150,10 @@ struct WaveMap {
 };
 
 // hi + lo = A B^T over nk stages.  The loaders la / lb give CA / CB chunks of
-// 8 k values per thread and stage: load() fetches the next stage's raw values
-// (zeros outside the operand), put(lds, c, tiny) splits chunk c into the
-// planes.  nk >= 0; stages past nk are loaded but never multiplied.
+// 8 k values per thread and stage: load(x) fetches the next stage's raw values
+// (zeros outside the operand) into a register set, put(lds, x[c], c, tiny)
+// splits chunk c into the planes.  nk >= 0; stages past nk are loaded but
+// never multiplied.
 template <class S, class LA, class LB>
 __device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x4 (&hi)[S::BI][S::BN],
                                          f32x4 (&lo)[S::BI][S::BN], Tiny& tiny) {
@@ -169,14 +173,23 @@ __device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x
     bo[n] = 3 * PA + (int)slot((blk >> 2) * 64 + 4 * w.lr + (blk & 3), w.q);
   }
   auto frag = [&](const char* p) { return *reinterpret_cast<const u32x4*>(p); };
-  la.load();
-  lb.load();
+  constexpr int D = S::DEPTH;
+  float xa[D][CA][8], xb[D][CB][8];  // stage kt + 1 + u waits in set (kt + u) % D
+  la.pre();
+  lb.pre();
+  la.load(xa[0]);
+  lb.load(xb[0]);
 #pragma unroll
-  for (int c = 0; c < CA; ++c) la.template put<PA>(lds, c, tiny);
+  for (int c = 0; c < CA; ++c) la.template put<PA>(lds, xa[0][c], c, tiny);
 #pragma unroll
-  for (int c = 0; c < CB; ++c) lb.template put<PB>(lds + 3 * PA, c, tiny);
-  la.load();
-  lb.load();
+  for (int c = 0; c < CB; ++c) lb.template put<PB>(lds + 3 * PA, xb[0][c], c, tiny);
+#pragma unroll
+  for (int u = 0; u < D; ++u) {
+    la.pre();
+    lb.pre();
+    la.load(xa[u]);
+    lb.load(xb[u]);
+  }
   __syncthreads();
   u32x4 b[BN][3], a0[2], a1, a2;
 #pragma unroll
@@ -186,7 +199,7 @@ __device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x
   a0[0] = frag(lds + ao[0]);
   a1 = frag(lds + ao[0] + PA);
   a2 = frag(lds + ao[0] + 2 * PA);
-  for (int kt = 0; kt < nk; ++kt) {
+  auto stage = [&](int kt, float(&sa)[CA][8], float(&sb)[CB][8]) {
     char* cur = lds + (kt & 1) * STG;
     char* nxt = lds + ((kt & 1) ^ 1) * STG;
 #pragma unroll
@@ -196,6 +209,10 @@ __device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x
       const int in = last ? 0 : i + 1;
       if (last) __syncthreads();  // stage kt fully read, stage kt + 1 fully written
       a0[(i + 1) & 1] = frag(src + ao[in]);
+      if (i + 2 == BI) {
+        la.pre();
+        lb.pre();
+      }
       const u32x4 x0 = a0[i & 1];
       // x0 y2, x1 y1, x0 y1, x2 y0, x1 y0 into lo, x0 y0 into hi; a plane's
       // registers take the next fragments after its last use
@@ -226,12 +243,12 @@ __device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x
 #pragma unroll
         for (int c = 0; c < CT; ++c)
           if (c * (BI - 1) / CT == i) {
-            if (c < CA) la.template put<PA>(nxt, c, tiny);
-            else lb.template put<PB>(nxt + 3 * PA, c - CA, tiny);
+            if (c < CA) la.template put<PA>(nxt, sa[c], c, tiny);
+            else lb.template put<PB>(nxt + 3 * PA, sb[c < CA ? 0 : c - CA], c - CA, tiny);
           }
         if (i + 2 == BI && !LA::kBranch && !LB::kBranch) {
-          la.load();
-          lb.load();
+          la.load(sa);
+          lb.load(sb);
         }
       }
       // the splitting's vector instructions and the LDS traffic between the MFMAs
@@ -247,10 +264,46 @@ __device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x
       }
       __builtin_amdgcn_sched_barrier(0);
       if (i + 2 == BI && (LA::kBranch || LB::kBranch)) {
-        la.load();
-        lb.load();
+        la.load(sa);
+        lb.load(sb);
       }
     }
+  };
+  for (int kt = 0; kt < nk; kt += D) {
+#pragma unroll
+    for (int u = 0; u < D; ++u)
+      if (kt + u < nk) stage(kt + u, xa[u], xb[u]);
+  }
+}
+
+// This thread's K group.
+template <class S>
+__device__ __forceinline__ int k_group() {
+  return S::KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) / (S::CM * S::CN);
+}
+
+// Group 0's hi += lo + the other groups' sums, in group order; lo = 0.
+template <class S>
+__device__ __forceinline__ void join_groups(char* lds, f32x4 (&hi)[S::BI][S::BN], f32x4 (&lo)[S::BI][S::BN]) {
+  if (S::KG == 1) return;
+  static_assert(S::KG <= 2 && S::NTH * S::BI * S::BN * 16 <= S::LDS * S::KG, "exchange buffer");
+  f32x4* x = reinterpret_cast<f32x4*>(lds) + threadIdx.x % S::NTH;
+  __syncthreads();
+  if (k_group<S>() == 1) {
+#pragma unroll
+    for (int i = 0; i < S::BI; ++i)
+#pragma unroll
+      for (int n = 0; n < S::BN; ++n) x[(i * S::BN + n) * S::NTH] = hi[i][n] + lo[i][n];
+  }
+  __syncthreads();
+  if (k_group<S>() == 0) {
+#pragma unroll
+    for (int i = 0; i < S::BI; ++i)
+#pragma unroll
+      for (int n = 0; n < S::BN; ++n) {
+        hi[i][n] = (hi[i][n] + lo[i][n]) + x[(i * S::BN + n) * S::NTH];
+        lo[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
   }
 }
 
@@ -295,6 +348,43 @@ __device__ __forceinline__ void fp32_tile(FA a, FB b, int klen, f32x4 (&acc)[S::
   }
 }
 
+// The slots of a thread's chunks: the part every loader shares.
+// kBranch: load() has a branch, and is kept out of the interleaved schedule;
+// pre() may read ahead what load() needs.
+template <int NC_, bool SUM>
+struct Chunks {
+  static constexpr int NC = NC_;
+  static constexpr bool kBranch = false;
+  uint32_t dst[NC];
+  float sum[SUM ? NC : 1];  // SUM: each chunk's sum over k
+  __device__ __forceinline__ void place(int c, int r, int q) {
+    dst[c] = slot(r, q);
+    if (SUM) sum[c] = 0.f;
+  }
+  __device__ __forceinline__ void pre() {}
+  template <int PL>
+  __device__ __forceinline__ void put(char* lds, const float (&x)[8], int c, Tiny& tiny) {
+    u32x4 p0, p1, p2;
+    split8(x, p0, p1, p2, tiny);
+    if (SUM)
+      sum[c] += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+    char* d = lds + dst[c];
+    *reinterpret_cast<u32x4*>(d) = p0;
+    *reinterpret_cast<u32x4*>(d + PL) = p1;
+    *reinterpret_cast<u32x4*>(d + 2 * PL) = p2;
+  }
+};
+// Tile row and lane group of chunk c of thread t: rows along a wave (a lane
+// group per wave), or four lane groups of a row beside each other.
+template <bool ROWS, int NTH>
+__device__ __forceinline__ void chunk_at(int t, int c, int& r, int& q) {
+  const int e = t + c * NTH;
+  q = ROWS ? (e >> 6) & 3 : e & 3;
+  r = ROWS ? (e & 63) + 64 * (e >> 8) : e >> 2;
+}
+// k (within a stage) of element j of a chunk of lane group 0.
+__device__ __forceinline__ constexpr int chunk_k(int j) { return (j & 3) + 16 * (j >> 2); }
+
 // ------------------------------------------------------------- matrix operand
 // A tile of R rows of a strided matrix, by NTH threads; a thread's chunks are
 // 8 k values of one row each.  MC: row-contiguous (element (row, k) at
@@ -305,17 +395,16 @@ __device__ __forceinline__ void fp32_tile(FA a, FB b, int klen, f32x4 (&acc)[S::
 // K % 4 != 0, so the last stage of a k-contiguous operand is read element by
 // element.  SUM: also keeps each chunk's sum over k (the bias gradient).
 template <bool MC, int R, int NTH, bool TAIL, bool SUM = false>
-struct MatLoad {
-  static constexpr int NC = R * 4 / NTH;
-  static constexpr bool kBranch = !MC && TAIL;  // load() has a branch
+struct MatLoad : Chunks<R * 4 / NTH, SUM> {
+  using Base = Chunks<R * 4 / NTH, SUM>;
+  using Base::NC;
+  static constexpr bool kBranch = !MC && TAIL;
   static_assert(NC * NTH == R * 4, "chunks per thread");
   __amdgpu_buffer_rsrc_t rs;
-  uint32_t off[NC], dst[NC];
+  uint32_t off[NC];
   uint32_t ld4b, step, so, jump;  // bytes: one row of ld, one stage, the cursor, the extra step past a term's end
   int left, stages, terms;        // stages left of this term, stages per term, terms left
   int kq, kfull;                  // k of this lane group in the stage; K % 32 bound of the last stage (32: full)
-  float x[NC][8];
-  float sum[SUM ? NC : 1];
 
   // Rows [r0, r0 + R) of `rows`, k in [k0, k0 + klen); `nterms` copies
   // term_stride elements apart, one after another.  base's extent, 64 more rows
@@ -331,6 +420,7 @@ struct MatLoad {
     stages = left = (klen + KS - 1) / KS;
     jump = (uint32_t)(term_stride * 4) - (uint32_t)stages * step;
     kfull = klen - (stages - 1) * KS;
+    if (klen <= 0) so = kOOB, step = jump = 0, left = stages = 1 << 30;  // nothing: every load gives zeros
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       int r, q;
@@ -338,28 +428,22 @@ struct MatLoad {
       kq = 4 * q;  // the same for every chunk
       const int64_t o = MC ? (int64_t)kq * ld + r0 + r : (int64_t)(r0 + r) * ld + kq;
       off[c] = r0 + r < rows ? (uint32_t)(o * 4) : kOOB;
-      dst[c] = slot(r, q);
-      if (SUM) sum[c] = 0.f;
+      this->place(c, r, q);
     }
   }
-  // Tile row and lane group of a thread's chunk c.
-  __device__ __forceinline__ static void unit(int t, int c, int& r, int& q) {
-    const int e = t + c * NTH;
-    q = MC ? (e >> 6) & 3 : e & 3;
-    r = MC ? (e & 63) + 64 * (e >> 8) : e >> 2;
-  }
+  __device__ __forceinline__ static void unit(int t, int c, int& r, int& q) { chunk_at<MC, NTH>(t, c, r, q); }
   // A row-contiguous operand ends at its extent (reads past it give zeros; a
   // term or split that ends before it ends on a whole stage, see the host's
   // rule); along k of a k-contiguous one the last stage masks what lies past
   // it.  Past the last term every load gives zeros.
-  __device__ __forceinline__ void load() {
+  __device__ __forceinline__ void load(float (&x)[NC][8]) {
     const int kmax = left == 1 ? kfull : KS;
     if (!MC && TAIL && kmax < KS) {
 #pragma unroll
       for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const int k = (j & 3) + 16 * (j >> 2);
+          const int k = chunk_k(j);
           x[c][j] = ld1(rs, kq + k < kmax ? off[c] + so + 4u * k : kOOB);
         }
     } else {
@@ -378,7 +462,7 @@ struct MatLoad {
         } else {
 #pragma unroll
           for (int j = 0; j < 8; ++j)
-            x[c][j] = ld1(rs, off[c] + (so + (uint32_t)((j & 3) + 16 * (j >> 2)) * ld4b));
+            x[c][j] = ld1(rs, off[c] + (so + (uint32_t)chunk_k(j) * ld4b));
         }
       }
     }
@@ -388,17 +472,6 @@ struct MatLoad {
       so += jump;
       if (--terms == 0) so = kOOB, step = jump = 0;
     }
-  }
-  template <int PL>
-  __device__ __forceinline__ void put(char* lds, int c, Tiny& tiny) {
-    u32x4 p0, p1, p2;
-    split8(x[c], p0, p1, p2, tiny);
-    if (SUM)
-      sum[c] += ((x[c][0] + x[c][1]) + (x[c][2] + x[c][3])) + ((x[c][4] + x[c][5]) + (x[c][6] + x[c][7]));
-    char* d = lds + dst[c];
-    *reinterpret_cast<u32x4*>(d) = p0;
-    *reinterpret_cast<u32x4*>(d + PL) = p1;
-    *reinterpret_cast<u32x4*>(d + 2 * PL) = p2;
   }
 };
 

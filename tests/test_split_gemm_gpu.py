@@ -108,3 +108,89 @@ def test_split_gemm_identity_exact(hip):
     a = (r.standard_normal((M, N)) * np.exp2(r.integers(-60, 60, (M, N)))).astype(np.float32)
     C, _ = run(hip, 0, 0, M, N, N, a, np.eye(N, dtype=np.float32))
     np.testing.assert_array_equal(C, a)
+
+
+# Convolutions at the edges of the split kernels' tiles and of their tap
+# table's period (32 channels): maps of odd size (one-element loads), strides,
+# depths of one, whole and part periods, a 25-tap filter, one pixel, few and
+# many tiles (K groups), against float64 sums of the same products.
+CONVS = [(3, 33, 7, 7, 70, 3, 1, 1), (2, 65, 9, 11, 130, 3, 1, 2), (1, 97, 5, 5, 66, 3, 0, 1), (2, 64, 14, 14, 129, 3, 1, 1),
+         (1, 20, 13, 10, 67, 5, 2, 1), (4, 31, 3, 3, 257, 1, 0, 1), (1, 130, 1, 1, 72, 3, 1, 1), (5, 160, 28, 28, 72, 1, 0, 2),
+         (33, 66, 32, 32, 67, 3, 1, 1)]
+
+
+@pytest.mark.parametrize("n,cin,h,w,cout,k,pad,stride", CONVS)
+def test_split_conv_edges(hip, n, cin, h, w, cout, k, pad, stride):
+    r = rng(n + cin + h + w + cout + k + stride)
+    oh, ow = (h + 2 * pad - k) // stride + 1, (w + 2 * pad - k) // stride + 1
+    x = r.standard_normal((n, cin, h, w), dtype=np.float32)
+    wt = r.standard_normal((cout, cin, k, k), dtype=np.float32)
+    b = r.standard_normal(cout, dtype=np.float32)
+    dy = r.standard_normal((n, cout, oh, ow), dtype=np.float32)
+    xp = np.zeros((n, cin, h + 2 * pad, w + 2 * pad))
+    xp[:, :, pad:pad + h, pad:pad + w] = x
+    span = lambda o, s: slice(s, s + (o - 1) * stride + 1, stride)  # noqa: E731
+    y, ya = np.zeros((n, cout, oh, ow)), np.zeros((n, cout, oh, ow))
+    dxp, dxa = np.zeros_like(xp), np.zeros_like(xp)
+    dw, dwa = np.zeros(wt.shape), np.zeros(wt.shape)
+    for i in range(k):
+        for j in range(k):
+            xs, wij = xp[:, :, span(oh, i), span(ow, j)], wt[:, :, i, j].astype(np.float64)
+            d = dy.astype(np.float64)
+            y += np.einsum("oc,ncyx->noyx", wij, xs, optimize=True)
+            ya += np.einsum("oc,ncyx->noyx", np.abs(wij), np.abs(xs), optimize=True)
+            dxp[:, :, span(oh, i), span(ow, j)] += np.einsum("oc,noyx->ncyx", wij, d, optimize=True)
+            dxa[:, :, span(oh, i), span(ow, j)] += np.einsum("oc,noyx->ncyx", np.abs(wij), np.abs(d), optimize=True)
+            dw[:, :, i, j] = np.einsum("noyx,ncyx->oc", d, xs, optimize=True)
+            dwa[:, :, i, j] = np.einsum("noyx,ncyx->oc", np.abs(d), np.abs(xs), optimize=True)
+    y += b[:, None, None]
+    dx, dxa = dxp[:, :, pad:pad + h, pad:pad + w], dxa[:, :, pad:pad + h, pad:pad + w]
+    B = hip.Buffer.from_array
+    dims = (n, cin, h, w, cout, k, k, pad, stride)
+    gx, gw, gb, gdy = B(x), B(wt), B(b), B(dy)
+    gy, gdx, gdw = B(np.full(y.shape, np.nan, np.float32)), B(np.full(x.shape, np.nan, np.float32)), B(np.full(wt.shape, np.nan, np.float32))
+    gdb = B(np.full(cout, np.nan, np.float32))
+    # the fp32 MFMA kernels, where they run, round once per 4 products
+    lim = lambda K: max(bound(K), (K / 4 + 8) * 2.0 ** -24)  # noqa: E731
+    hip.call("mle_conv2d_fwd", None, gx.ptr, gw.ptr, gb.ptr, gy.ptr, *dims)
+    assert np.all(np.abs(gy.numpy(y.shape) - y) <= lim(cin * k * k) * (ya + np.abs(b)[:, None, None]))
+    hip.call("mle_conv2d_dgrad", None, gdy.ptr, gw.ptr, gdx.ptr, *dims, 0)
+    assert np.all(np.abs(gdx.numpy(x.shape) - dx) <= lim(cout * k * k) * dxa)
+    hip.call("mle_conv2d_dgrad", None, gdy.ptr, gw.ptr, gdx.ptr, *dims, 1)
+    assert np.all(np.abs(gdx.numpy(x.shape) - 2 * dx) <= 2 * lim(cout * k * k) * dxa + 2.0 ** -22 * np.abs(dx))
+    nb = hip.lib().mle_conv2d_wgrad_ws_bytes(*dims)
+    ws = hip.Buffer(nb)
+    hip.call("mle_conv2d_wgrad_bias", None, gx.ptr, gdy.ptr, gdw.ptr, gdb.ptr, 0, *dims, ws.ptr, nb)
+    K = n * oh * ow
+    assert np.all(np.abs(gdw.numpy(wt.shape) - dw) <= lim(K) * dwa)
+    db, dba = dy.astype(np.float64).sum((0, 2, 3)), np.abs(dy).sum((0, 2, 3))
+    assert np.all(np.abs(gdb.numpy() - db) <= (K / 4 + 8) * 2.0 ** -24 * dba)
+
+
+def test_split_conv_special_values(hip):
+    """An infinity, a NaN and the largest value in x and dy: the same
+    positions as fp32 products give them, everything else finite and right."""
+    n, cin, h, cout = 2, 96, 20, 80
+    r = rng(9)
+    x = r.standard_normal((n, cin, h, h), dtype=np.float32)
+    wt = (r.random((cout, cin, 3, 3)) * 0.5 + 0.1).astype(np.float32)
+    x[0, 3, 4, 5], x[1, 90, 19, 19], x[0, 50, 10, 10] = np.inf, np.nan, np.finfo(np.float32).max
+    xp = np.zeros((n, cin, h + 2, h + 2))
+    xp[:, :, 1:-1, 1:-1] = x
+    y = np.zeros((n, cout, h, h))
+    ya = np.zeros_like(y)
+    with np.errstate(invalid="ignore", over="ignore"):
+        for i in range(3):
+            for j in range(3):
+                xs, wij = xp[:, :, i:i + h, j:j + h], wt[:, :, i, j].astype(np.float64)
+                y += np.einsum("oc,ncyx->noyx", wij, xs)
+                ya += np.einsum("oc,ncyx->noyx", wij, np.abs(xs))
+        y32 = y.astype(np.float32)
+    B = hip.Buffer.from_array
+    gx, gw, gy = B(x), B(wt), B(np.zeros(y.shape, np.float32))
+    hip.call("mle_conv2d_fwd", None, gx.ptr, gw.ptr, None, gy.ptr, n, cin, h, h, cout, 3, 3, 1, 1)
+    got = gy.numpy(y.shape)
+    assert np.array_equal(np.isnan(got), np.isnan(y32))
+    assert np.array_equal(got[np.isinf(y32)], y32[np.isinf(y32)])
+    ok = np.isfinite(y32)
+    assert np.all(np.abs(got[ok] - y[ok]) <= bound(cin * 9) * ya[ok])
