@@ -20,13 +20,17 @@
 // registers.  Because P is normalised over the rows, D_c = <dV_c, V_c>: the
 // key-block kernel finishes dV first and gets D from it.
 //
-//   attn_stats_kernel  (key blocks)   : m_c, 1 / l_c
-//   attn_fwd_kernel    (query blocks) : O = P V
-//   attn_bwd_kv_kernel (key blocks)   : dV, D (and dK = scale dS^T Q)
-//   attn_bwd_q_kernel  (query blocks) : dQ = scale dS K (or the reference's dK)
+//   statistics (key blocks)   : m_c, 1 / l_c
+//   forward    (query blocks) : O = P V
+//   bwd kv     (key blocks)   : dV, D (and dK = scale dS^T Q)
+//   bwd q      (query blocks) : dQ = scale dS K (or the reference's dK)
 //
-// All products are v_mfma_f32_16x16x4f32 with operands loaded from memory in
-// the MFMA lane layout.  Lane (lr, q) = (lane % 16, lane / 16).  A score tile
+// Up to 256 positions a workgroup runs a whole slice on the fp32 matrix cores;
+// past that the passes are kernels of their own on the bf16 matrix cores, and
+// the fp32 tile functions are what they fall back to.
+//
+// The fp32 products are v_mfma_f32_16x16x4f32 with operands loaded from memory
+// in the MFMA lane layout.  Lane (lr, q) = (lane % 16, lane / 16).  A score tile
 // in the accumulator layout holds, in lane (lr, q), rows 4q + r (r = 0..3) of
 // column lr -- which is exactly the B operand layout of the next product when
 // the tile's rows are that product's contraction index (step r feeds rows
@@ -35,6 +39,7 @@
 // dimension, and the result's block (i, n) row 4q + r is element
 // 16 q + 4 r + i of the head dimension: four blocks give one float4 store.
 #include "common.hpp"
+#include "split_core.hpp"
 
 #include <float.h>
 
@@ -83,9 +88,8 @@ __device__ __forceinline__ f32x4 bld4s(__amdgpu_buffer_rsrc_t r, uint32_t elem, 
 __device__ __forceinline__ float bld1(__amdgpu_buffer_rsrc_t r, uint32_t elem) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)(elem * 4u), 0, 0));
 }
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void bst4(__amdgpu_buffer_rsrc_t r, uint32_t elem, f32x4 v) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, (int)(elem * 4u), 0, 0);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(split::u32x4, v), r, (int)(elem * 4u), 0, 0);
 }
 __device__ __forceinline__ void bst1(__amdgpu_buffer_rsrc_t r, uint32_t elem, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)(elem * 4u), 0, 0);
@@ -1084,26 +1088,571 @@ __device__ __forceinline__ void bwd_q_kept(const AttnArgs& a, const Slice& sl, i
 // One wave per 32-row tile, two tiles (j and nb - 1 - j) per workgroup,
 // workgroups spread over the XCDs by slice (slice_of).
 template <bool CAUSAL>
-__global__ __launch_bounds__(128, 2) void attn_stats_kernel(AttnArgs a) {
-  const Slice sl = slice_of(a);
-  stats_tile<CAUSAL>(a, sl, tile_of(a, sl, threadIdx.x >> 6) * TW);
-}
-template <bool CAUSAL>
-__global__ __launch_bounds__(128, 2) void attn_fwd_kernel(AttnArgs a) {
-  const Slice sl = slice_of(a);
-  fwd_tile<CAUSAL>(a, sl, tile_of(a, sl, threadIdx.x >> 6) * TW);
-}
-template <bool CAUSAL, bool DK>
 __global__ __launch_bounds__(128, 2) void attn_bwd_kv_kernel(AttnArgs a) {
   const Slice sl = slice_of(a);
-  bwd_kv_tile<CAUSAL, DK>(a, sl, tile_of(a, sl, threadIdx.x >> 6) * TW);
+  bwd_kv_tile<CAUSAL, true>(a, sl, tile_of(a, sl, threadIdx.x >> 6) * TW);
 }
+// ---------------------------------------------------------------------------
+// The passes on the bf16 matrix cores (split_core.hpp: exact three-way splits,
+// six bf16 MFMAs per product, fp32 accuracy), a kernel per pass.  A workgroup
+// is four waves of 32 columns each (keys of the statistics and dV, queries of O
+// and dQ); together they stage 32 rows of the other side at a time in LDS,
+// split once for all four.  A score block leaves the accumulators as the next
+// product's B operand without another exchange: lane (lr, q) holds rows
+// 4 q + r and 16 + 4 q + r of column lr, the 8 contraction values that lane
+// group q feeds.
+//
+// Staged tiles, three planes of 4 KB each:
+//   rows  [32 positions][64 of the head] as two 32-deep stages: the A operand
+//         of a contraction over the head (scores, dP); 16-byte slot lr of lane
+//         group q of (stage s, block i): (2 s + i) KB + 256 q + 16 lr
+//   cols  [64 of the head][32 positions]: the A operand of a contraction over
+//         the positions; row d = 4 lr + b of block b: b KB + 256 q + 16 (lr ^ 4 b)
+// both written and read without bank conflicts.
+//
+// A workgroup whose sums show an infinity or NaN, or whose operands hold a
+// value the split cannot represent, runs its columns again on the fp32 tile
+// functions above.  What bounds the passes is the vector unit and its overlap
+// with the matrix cores at one to two waves per SIMD: splitting and
+// exponentials take about as many cycles as the products.  32 heads of 1024
+// unmasked positions, us: statistics 41, O 79, dV 76, dQ and dK 136; the whole
+// forward and backward 597 on the fp32 matrix cores, 286 here.
+constexpr int CW = 128;             // columns of a workgroup
+constexpr int kTile = 12288;        // bytes of a staged tile
+using split::u32x4;
+using Frag = u32x4[3];
+
+// One staged 8-value chunk per thread and tile.
+struct Raw {
+  float x[8];
+};
+__device__ __forceinline__ void load_rows(__amdgpu_buffer_rsrc_t r, uint32_t base, int ld, int pos, Raw& o) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const uint32_t e = base + (uint32_t)(pos + 16 * (w & 1) + (lane & 15)) * ld + 32 * (w >> 1) + 4 * (lane >> 4);
+  const f32x4 a = bld4(r, e), b = bld4(r, e + 16);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    o.x[j] = a[j];
+    o.x[4 + j] = b[j];
+  }
+}
+__device__ __forceinline__ void load_cols(__amdgpu_buffer_rsrc_t r, uint32_t base, int ld, int pos, Raw& o) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) o.x[j] = bld1(r, base + (uint32_t)(pos + 4 * w + split::chunk_k(j)) * ld + lane);
+}
+__device__ __forceinline__ int rows_slot() {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  return ((w >> 1) * 2 + (w & 1)) * 1024 + lane * 16;
+}
+__device__ __forceinline__ int cols_slot() {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, b = lane & 3;
+  return b * 1024 + w * 256 + (((lane >> 2) ^ (4 * b)) * 16);
+}
+__device__ __forceinline__ void put(char* tile, int slot, const Raw& o, split::Tiny& tiny) {
+  u32x4 p0, p1, p2;
+  split::split8(o.x, p0, p1, p2, tiny);
+  *reinterpret_cast<u32x4*>(tile + slot) = p0;
+  *reinterpret_cast<u32x4*>(tile + slot + 4096) = p1;
+  *reinterpret_cast<u32x4*>(tile + slot + 8192) = p2;
+}
+__device__ __forceinline__ void frag(const char* p, Frag& f) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i) f[i] = *reinterpret_cast<const u32x4*>(p + 4096 * i);
+}
+// hi += a0 b0; lo += the five corrections.
+__device__ __forceinline__ void mma6(const Frag& a, const Frag& b, f32x4& hi, f32x4& lo) {
+  lo = split::mma(a[0], b[2], lo);
+  hi = split::mma(a[0], b[0], hi);
+  lo = split::mma(a[1], b[1], lo);
+  lo = split::mma(a[0], b[1], lo);
+  lo = split::mma(a[2], b[0], lo);
+  lo = split::mma(a[1], b[0], lo);
+}
+// The wave's columns c0 + 16 n + lr of a [seq][64] operand, as B fragments of
+// the two head stages.
+template <int NB>
+__device__ __forceinline__ void load_b(__amdgpu_buffer_rsrc_t r, uint32_t base, int ld, int c0, Frag (&b)[NB][2],
+                                       split::Tiny& tiny) {
+  const int lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
+#pragma unroll
+  for (int n = 0; n < NB; ++n)
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const uint32_t e = base + (uint32_t)(c0 + 16 * n + lr) * ld + 32 * s + 4 * q;
+      const f32x4 u = bld4(r, e), v = bld4(r, e + 16);
+      const float x[8] = {u[0], u[1], u[2], u[3], v[0], v[1], v[2], v[3]};
+      split::split8(x, b[n][s][0], b[n][s][1], b[n][s][2], tiny);
+    }
+}
+// out[i][n] = rows tile (32 positions) times the columns, over the head.
+template <int NB>
+__device__ __forceinline__ void score(const char* tile, const Frag (&b)[NB][2], f32x4 (&out)[2][NB]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    f32x4 hi[NB], lo[NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) hi[n] = lo[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      Frag a;
+      frag(tile + (2 * s + i) * 1024 + lane * 16, a);
+#pragma unroll
+      for (int n = 0; n < NB; ++n) mma6(a, b[n][s], hi[n], lo[n]);
+    }
+#pragma unroll
+    for (int n = 0; n < NB; ++n) out[i][n] = hi[n] + lo[n];
+  }
+}
+// A score block's 8 values per lane and column block, as B fragments.
+template <int NB>
+__device__ __forceinline__ void to_frag(const f32x4 (&v)[2][NB], Frag (&f)[NB]) {
+  split::Tiny ignore;  // single small values are ordinary: below 2^-110 they lose bits, 2^-134 at most (see Peak)
+#pragma unroll
+  for (int n = 0; n < NB; ++n) {
+    const float x[8] = {v[0][n][0], v[0][n][1], v[0][n][2], v[0][n][3], v[1][n][0], v[1][n][1], v[1][n][2], v[1][n][3]};
+    split::split8(x, f[n][0], f[n][1], f[n][2], ignore);
+  }
+}
+// hi + lo += cols tile times the fragments, over 32 positions.
+template <int NB>
+__device__ __forceinline__ void accumulate(const char* tile, const Frag (&f)[NB], f32x4 (&hi)[4][NB], f32x4 (&lo)[4][NB]) {
+  const int lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    Frag a;
+    frag(tile + b * 1024 + q * 256 + ((lr ^ (4 * b)) * 16), a);
+#pragma unroll
+    for (int n = 0; n < NB; ++n) mma6(a, f[n], hi[b][n], lo[b][n]);
+  }
+}
+template <int NB>
+__device__ __forceinline__ void clear(f32x4 (&a)[4][NB], f32x4 (&b)[4][NB]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int n = 0; n < NB; ++n) a[i][n] = b[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+// 0 when every element is finite, else NaN.
+template <int I, int NB>
+__device__ __forceinline__ float finite_mark(const f32x4 (&a)[I][NB]) {
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t = fmaf(0.f, a[i][n][r], t);
+  return t;
+}
+
+// Largest |value| of a column over everything its fragments held.  The split
+// drops at most 2^-134 of a value; a column whose largest is under 2^-80 (and
+// not 0) would notice and goes to the fp32 tile.
+struct Peak {
+  float v[2] = {0.f, 0.f};
+  __device__ __forceinline__ void add(const f32x4 (&s)[2][2]) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[n] = fmaxf(v[n], fabsf(s[i][n][r]));
+  }
+  __device__ __forceinline__ bool low() {
+    bool any = false;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      v[n] = fmaxf(v[n], __shfl_xor(v[n], 16, 64));
+      v[n] = fmaxf(v[n], __shfl_xor(v[n], 32, 64));
+      any |= v[n] > 0.f && v[n] < 0x1p-80f;
+    }
+    return any;
+  }
+};
+
+// Workgroup's slice and first column; the slices of an XCD are neighbours.
+__device__ __forceinline__ Slice column_block(const AttnArgs& a) {
+  const int L = blockIdx.x, total = gridDim.x, blocks = (a.seq + CW - 1) / CW;
+  const int x = L % kXcds, j = L / kXcds, per = total / kXcds, rem = total % kXcds;
+  const int t = x * per + min(x, rem) + j;
+  const int z = t / blocks, b = z / a.heads, h = z - b * a.heads;
+  return {z, (uint32_t)b * a.seq * a.ld + (uint32_t)h * HD, t - z * blocks};
+}
+
+// Stages chunks [c0, c1) of 32 positions, double-buffered: fetch(c) loads a
+// chunk's raw values, store(buffer) splits them into it, compute(c, buffer)
+// multiplies.  Every wave of the workgroup runs it with the same bounds.
+template <int BYTES, class Fetch, class Store, class Compute>
+__device__ __forceinline__ void staged_loop(char* lds, int c0, int c1, Fetch fetch, Store store, Compute compute) {
+  if (c0 >= c1) return;
+  fetch(c0);
+  store(lds);
+  fetch(min(c0 + 1, c1 - 1));
+  __syncthreads();
+  for (int c = c0; c < c1; ++c) {
+    char* cur = lds + ((c - c0) & 1) * BYTES;
+    char* nxt = lds + (((c - c0) & 1) ^ 1) * BYTES;
+    store(nxt);
+    fetch(min(c + 2, c1 - 1));
+    compute(c, cur);
+    __syncthreads();
+  }
+}
+
+// Column statistics m_c, 1 / l_c of 128 keys: S = Q K^T in chunks of 32
+// queries, a running maximum and masked sum per lane and key, merged over the
+// lane groups at the end.
+template <bool CAUSAL>
+__global__ __launch_bounds__(256, 2) void attn_stats_split_kernel(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[2 * kTile];
+  const Slice sl = column_block(a);
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
+  const int k0 = sl.pair * CW + w * TW;
+  const bool live = k0 < a.seq;
+  const __amdgpu_buffer_rsrc_t Q = rsrc(a.q, a.bytes), K = rsrc(a.k, a.bytes);
+  split::Tiny tiny;
+  Frag kb[2][2];
+  load_b<2>(K, sl.base, a.ld, min(k0, a.seq - TW), kb, tiny);
+  float m[2] = {-FLT_MAX, -FLT_MAX}, l[2] = {0.f, 0.f}, mark = 0.f;
+  Raw raw;
+  const int slot = rows_slot();
+  staged_loop<kTile>(
+      lds, 0, a.seq / TW, [&](int c) { load_rows(Q, sl.base, a.ld, TW * c, raw); },
+      [&](char* t) { put(t, slot, raw, tiny); },
+      [&](int c, const char* t) {
+        if (!live) return;
+        f32x4 s[2][2];
+        score<2>(t, kb, s);
+        const bool masked = CAUSAL && TW * c < k0 + TW - 1, above = CAUSAL && TW * c + TW - 1 < k0;
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          const int key = k0 + 16 * n + lr;
+          float v[8], mx = m[n];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            v[j] = a.scale * s[j >> 2][n][j & 3];
+            mark = fmaf(0.f, v[j], mark);
+            mx = fmaxf(mx, v[j]);
+          }
+          if (!above) {  // wholly masked chunks only raise the maximum
+            float add = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const float e = __expf(v[j] - mx);
+              add += !masked || TW * c + split::chunk_k(j) + 4 * q >= key ? e : 0.f;
+            }
+            l[n] = l[n] * __expf(m[n] - mx) + add;
+          }
+          // (an unmasked chunk follows every wholly masked one: its update rescales a sum of 0)
+          m[n] = mx;
+        }
+      });
+  const bool bad = tiny.found() || (live && !(mark == 0.f));
+  if (__syncthreads_or(bad)) {
+    if (live) stats_tile<CAUSAL>(a, sl, k0);
+    return;
+  }
+  if (!live) return;
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+#pragma unroll
+    for (int off = 16; off < 64; off <<= 1) {
+      const float mo = __shfl_xor(m[n], off, 64), lo = __shfl_xor(l[n], off, 64);
+      const float M = fmaxf(m[n], mo);
+      l[n] = l[n] * __expf(m[n] - M) + lo * __expf(mo - M);
+      m[n] = M;
+    }
+    const float il = 1.0f / (l[n] < 1e-45f ? 1.0f : l[n]);
+    if (q == 0)
+      *reinterpret_cast<float2*>(a.stats + ((size_t)sl.z * a.seq + k0 + 16 * n + lr) * 2) = make_float2(m[n], il);
+  }
+}
+
+// O = P V of 128 queries: S^T = K Q^T and O^T += V^T P^T per 32 keys.
+template <bool CAUSAL>
+__global__ __launch_bounds__(256, 2) void attn_fwd_split_kernel(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[4 * kTile];
+  const Slice sl = column_block(a);
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
+  // heaviest blocks first under the mask
+  const int blk = CAUSAL ? (a.seq + CW - 1) / CW - 1 - sl.pair : sl.pair;
+  const int q0 = blk * CW + w * TW;
+  const bool live = q0 < a.seq;
+  const __amdgpu_buffer_rsrc_t Q = rsrc(a.q, a.bytes), K = rsrc(a.k, a.bytes), V = rsrc(a.v, a.bytes);
+  const float* ST = a.stats + (size_t)sl.z * a.seq * 2;
+  split::Tiny tiny;
+  Peak peak;
+  Frag qb[2][2];
+  load_b<2>(Q, sl.base, a.ld, min(q0, a.seq - TW), qb, tiny);
+  f32x4 hi[4][2], lo[4][2];
+  clear(hi, lo);
+  Raw rk, rv;
+  const int rs = rows_slot(), cs = cols_slot();
+  staged_loop<2 * kTile>(
+      lds, 0, CAUSAL ? min(a.seq, (blk + 1) * CW) / TW : a.seq / TW,
+      [&](int c) {
+        load_rows(K, sl.base, a.ld, TW * c, rk);
+        load_cols(V, sl.base, a.ld, TW * c, rv);
+      },
+      [&](char* t) {
+        put(t, rs, rk, tiny);
+        put(t + kTile, cs, rv, tiny);
+      },
+      [&](int c, const char* t) {
+        if (!live || (CAUSAL && TW * c > q0)) return;
+        f32x4 st[2][2];  // (m, 1 / l) pairs of this lane's keys
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) st[i][h] = ld4(ST + (size_t)(TW * c + 16 * i + 4 * q) * 2 + 4 * h);
+        f32x4 s[2][2];
+        score<2>(t, qb, s);
+        const bool masked = CAUSAL && TW * c == q0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const bool keep = !masked || q0 + 16 * n + lr >= TW * c + 16 * i + 4 * q + r;
+              s[i][n][r] = keep ? __expf(a.scale * s[i][n][r] - st[i][r >> 1][2 * (r & 1)]) * st[i][r >> 1][2 * (r & 1) + 1] : 0.f;
+            }
+        peak.add(s);
+        Frag p[2];
+        to_frag<2>(s, p);
+        accumulate<2>(t + kTile, p, hi, lo);
+      });
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int n = 0; n < 2; ++n) hi[b][n] += lo[b][n];
+  const bool bad = tiny.found() || (live && (peak.low() || !(finite_mark(hi) == 0.f)));
+  if (__syncthreads_or(bad)) {
+    if (live) fwd_tile<CAUSAL>(a, sl, q0);
+    return;
+  }
+  if (!live) return;
+  const __amdgpu_buffer_rsrc_t O = rsrc(a.out, a.bytes);
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      bst4(O, sl.base + (uint32_t)(q0 + 16 * n + lr) * a.ld + 16 * q + 4 * r,
+           f32x4{hi[0][n][r], hi[1][n][r], hi[2][n][r], hi[3][n][r]});
+}
+
+// dV and D of 128 keys: S = Q K^T and dV^T += dO^T P per 32 queries.
+template <bool CAUSAL>
+__global__ __launch_bounds__(256, 2) void attn_bwd_kv_split_kernel(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[4 * kTile];
+  const Slice sl = column_block(a);
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
+  const int k0 = sl.pair * CW + w * TW;
+  const bool live = k0 < a.seq;
+  const __amdgpu_buffer_rsrc_t Q = rsrc(a.q, a.bytes), K = rsrc(a.k, a.bytes), V = rsrc(a.v, a.bytes), dO = rsrc(a.dout, a.bytes);
+  split::Tiny tiny;
+  Peak peak;
+  Frag kb[2][2];
+  load_b<2>(K, sl.base, a.ld, min(k0, a.seq - TW), kb, tiny);
+  float m[2] = {0.f, 0.f}, il[2] = {0.f, 0.f};
+  if (live) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const float2 t = *reinterpret_cast<const float2*>(a.stats + ((size_t)sl.z * a.seq + k0 + 16 * n + lr) * 2);
+      m[n] = t.x;
+      il[n] = t.y;
+    }
+  }
+  f32x4 hi[4][2], lo[4][2];
+  clear(hi, lo);
+  Raw rq, ro;
+  const int rs = rows_slot(), cs = cols_slot();
+  staged_loop<2 * kTile>(
+      lds, CAUSAL ? sl.pair * CW / TW : 0, a.seq / TW,
+      [&](int c) {
+        load_rows(Q, sl.base, a.ld, TW * c, rq);
+        load_cols(dO, sl.base, a.ld, TW * c, ro);
+      },
+      [&](char* t) {
+        put(t, rs, rq, tiny);
+        put(t + kTile, cs, ro, tiny);
+      },
+      [&](int c, const char* t) {
+        if (!live || (CAUSAL && TW * c < k0)) return;
+        f32x4 s[2][2];
+        score<2>(t, kb, s);
+        const bool masked = CAUSAL && TW * c == k0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const bool keep = !masked || TW * c + 16 * i + 4 * q + r >= k0 + 16 * n + lr;
+              s[i][n][r] = keep ? __expf(a.scale * s[i][n][r] - m[n]) * il[n] : 0.f;
+            }
+        peak.add(s);
+        Frag p[2];
+        to_frag<2>(s, p);
+        accumulate<2>(t + kTile, p, hi, lo);
+      });
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int n = 0; n < 2; ++n) hi[b][n] += lo[b][n];
+  const bool bad = tiny.found() || (live && (peak.low() || !(finite_mark(hi) == 0.f)));
+  if (__syncthreads_or(bad)) {
+    if (live) bwd_kv_tile<CAUSAL, false>(a, sl, k0);
+    return;
+  }
+  if (!live) return;
+  const __amdgpu_buffer_rsrc_t dVr = rsrc(a.dv, a.bytes);
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    const uint32_t row = sl.base + (uint32_t)(k0 + 16 * n + lr) * a.ld;
+    f32x4 vv[4], old[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      vv[r] = bld4(V, row + 16 * q + 4 * r);
+      old[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (a.acc_v) old[r] = bld4(dVr, row + 16 * q + 4 * r);
+    }
+    float part = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const f32x4 g = {hi[0][n][r], hi[1][n][r], hi[2][n][r], hi[3][n][r]};
+      part += g[0] * vv[r][0] + g[1] * vv[r][1] + g[2] * vv[r][2] + g[3] * vv[r][3];
+      bst4(dVr, row + 16 * q + 4 * r, a.acc_v ? g + old[r] : g);
+    }
+    part += __shfl_xor(part, 16, 64);
+    part += __shfl_xor(part, 32, 64);
+    if (q == 0) a.dcol[(size_t)sl.z * a.seq + k0 + 16 * n + lr] = part;
+  }
+}
+
+// dQ (and with KREF the reference's K gradient) of 128 queries: S^T = K Q^T,
+// dP^T = V dO^T, dS^T = P^T (dP^T - D), then dQ^T += K^T dS^T and X^T += Q^T
+// dS^T (Q's rows at the key positions) per 32 keys.  Twice the accumulators
+// and operands of the other passes: one wave per SIMD with up to 512 registers.
 template <bool CAUSAL, bool KREF>
-__global__ __launch_bounds__(128, 2) void attn_bwd_q_kernel(AttnArgs a) {
-  __shared__ __attribute__((aligned(16))) float lds[2][2][TW * LQ];  // [wave][Q, dO][row * LQ + col]
-  const Slice sl = slice_of(a);
-  const int w = threadIdx.x >> 6;
-  bwd_q_tile<CAUSAL, KREF>(a, sl, tile_of(a, sl, w) * TW, lds[w][0], lds[w][1]);
+__global__ __launch_bounds__(256, 1) void attn_bwd_q_split_kernel(AttnArgs a) {
+  constexpr int NT = KREF ? 4 : 3;
+  constexpr int kLds = 2 * NT * kTile > 8 * TW * LQ * 4 ? 2 * NT * kTile : 8 * TW * LQ * 4;
+  __shared__ __attribute__((aligned(16))) char lds[kLds];
+  const Slice sl = column_block(a);
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
+  const int blk = CAUSAL ? (a.seq + CW - 1) / CW - 1 - sl.pair : sl.pair;
+  const int q0 = blk * CW + w * TW;
+  const bool live = q0 < a.seq;
+  const __amdgpu_buffer_rsrc_t Q = rsrc(a.q, a.bytes), K = rsrc(a.k, a.bytes), V = rsrc(a.v, a.bytes), dO = rsrc(a.dout, a.bytes);
+  const float* ST = a.stats + (size_t)sl.z * a.seq * 2;
+  const float* DC = a.dcol + (size_t)sl.z * a.seq;
+  split::Tiny tiny;
+  Peak peak;
+  Frag qb[2][2], ob[2][2];
+  load_b<2>(Q, sl.base, a.ld, min(q0, a.seq - TW), qb, tiny);
+  load_b<2>(dO, sl.base, a.ld, min(q0, a.seq - TW), ob, tiny);
+  f32x4 hi[4][2], lo[4][2], xh[4][2], xl[4][2];
+  clear(hi, lo);
+  clear(xh, xl);
+  Raw rk, rv, ck, cq;
+  const int rs = rows_slot(), cs = cols_slot();
+  staged_loop<NT * kTile>(
+      lds, 0, CAUSAL ? min(a.seq, (blk + 1) * CW) / TW : a.seq / TW,
+      [&](int c) {
+        load_rows(K, sl.base, a.ld, TW * c, rk);
+        load_rows(V, sl.base, a.ld, TW * c, rv);
+        load_cols(K, sl.base, a.ld, TW * c, ck);
+        if (KREF) load_cols(Q, sl.base, a.ld, TW * c, cq);
+      },
+      [&](char* t) {
+        put(t, rs, rk, tiny);
+        put(t + kTile, rs, rv, tiny);
+        put(t + 2 * kTile, cs, ck, tiny);
+        if (KREF) put(t + 3 * kTile, cs, cq, tiny);
+      },
+      [&](int c, const char* t) {
+        if (!live || (CAUSAL && TW * c > q0)) return;
+        f32x4 st[2][2], dc[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) st[i][h] = ld4(ST + (size_t)(TW * c + 16 * i + 4 * q) * 2 + 4 * h);
+          dc[i] = ld4(DC + TW * c + 16 * i + 4 * q);
+        }
+        f32x4 s[2][2], dp[2][2];
+        score<2>(t, qb, s);
+        score<2>(t + kTile, ob, dp);
+        const bool masked = CAUSAL && TW * c == q0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const bool keep = !masked || q0 + 16 * n + lr >= TW * c + 16 * i + 4 * q + r;
+              const float p = __expf(a.scale * s[i][n][r] - st[i][r >> 1][2 * (r & 1)]) * st[i][r >> 1][2 * (r & 1) + 1];
+              s[i][n][r] = keep ? p * (dp[i][n][r] - dc[i][r]) : 0.f;
+            }
+        peak.add(s);
+        Frag f[2];
+        to_frag<2>(s, f);
+        accumulate<2>(t + 2 * kTile, f, hi, lo);
+        if (KREF) accumulate<2>(t + 3 * kTile, f, xh, xl);
+      });
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      hi[b][n] += lo[b][n];
+      xh[b][n] += xl[b][n];
+    }
+  const bool bad = tiny.found() || (live && (peak.low() || !(finite_mark(hi) + finite_mark(xh) == 0.f)));
+  if (__syncthreads_or(bad)) {
+    float* own = reinterpret_cast<float*>(lds) + w * 2 * TW * LQ;
+    if (live) bwd_q_tile<CAUSAL, KREF>(a, sl, q0, own, own + TW * LQ);
+    return;
+  }
+  if (!live) return;
+  const __amdgpu_buffer_rsrc_t dQr = rsrc(a.dq, a.bytes);
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    f32x4 old[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      old[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (a.acc_q) old[r] = bld4(dQr, sl.base + (uint32_t)(q0 + 16 * n + lr) * a.ld + 16 * q + 4 * r);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const f32x4 g = a.scale * f32x4{hi[0][n][r], hi[1][n][r], hi[2][n][r], hi[3][n][r]};
+      bst4(dQr, sl.base + (uint32_t)(q0 + 16 * n + lr) * a.ld + 16 * q + 4 * r, a.acc_q ? g + old[r] : g);
+    }
+  }
+  if (KREF) {
+    // C[d][j] lands at flat d * seq + j of the head's [seq x 64] block.
+    const __amdgpu_buffer_rsrc_t dKr = rsrc(a.dk, a.bytes);
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        uint32_t e[4];
+        float old[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const uint32_t f = (uint32_t)(16 * q + 4 * r + b) * (uint32_t)a.seq + q0 + 16 * n + lr;
+          e[r] = sl.base + (f / HD) * a.ld + f % HD;
+          old[r] = a.acc_k ? bld1(dKr, e[r]) : 0.f;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float g = a.scale * xh[b][n][r];
+          bst1(dKr, e[r], a.acc_k ? g + old[r] : g);
+        }
+      }
+  }
 }
 
 // Whole-slice kernels for seq <= 256: workgroup z runs every tile of slice z
@@ -1211,7 +1760,7 @@ int mle_attention_fwd(mle_stream stream, const float* q, const float* k, const f
   a.bytes = (uint32_t)((size_t)batch * seq * ld * sizeof(float));
   a.scale = scale;
   hipStream_t s = as_stream(stream);
-  const dim3 grid((unsigned)(seq / (2 * TW) * batch * heads));  // two 32-row tiles per workgroup
+  const dim3 blocks((unsigned)((seq + CW - 1) / CW * batch * heads));
   const double flop = 4.0 * batch * heads * (double)seq * seq * HD;  // S and P V, as the reference computes them
   ProbeScope probe("attn_fwd", s, flop, 0.0);
   if (seq <= SW * TW) {
@@ -1219,11 +1768,11 @@ int mle_attention_fwd(mle_stream stream, const float* q, const float* k, const f
     if (causal) mle::launch(attn_fwd_slice_kernel<true>, slices, SW * 64, 0, s, a);
     else mle::launch(attn_fwd_slice_kernel<false>, slices, SW * 64, 0, s, a);
   } else if (causal) {
-    mle::launch(attn_stats_kernel<true>, grid, 128, 0, s, a);
-    mle::launch(attn_fwd_kernel<true>, grid, 128, 0, s, a);
+    mle::launch(attn_stats_split_kernel<true>, blocks, 256, 0, s, a);
+    mle::launch(attn_fwd_split_kernel<true>, blocks, 256, 0, s, a);
   } else {
-    mle::launch(attn_stats_kernel<false>, grid, 128, 0, s, a);
-    mle::launch(attn_fwd_kernel<false>, grid, 128, 0, s, a);
+    mle::launch(attn_stats_split_kernel<false>, blocks, 256, 0, s, a);
+    mle::launch(attn_fwd_split_kernel<false>, blocks, 256, 0, s, a);
   }
   return check_launch("mle_attention_fwd");
 }
@@ -1260,6 +1809,7 @@ int mle_attention_bwd(mle_stream stream, const float* q, const float* k, const f
   a.acc_v = acc_v != 0;
   hipStream_t s = as_stream(stream);
   const dim3 grid((unsigned)(seq / (2 * TW) * batch * heads));  // two 32-row tiles per workgroup
+  const dim3 blocks((unsigned)((seq + CW - 1) / CW * batch * heads));
   const double flop = 8.0 * batch * heads * (double)seq * seq * HD;  // dP, dV, dQ, dK
   ProbeScope probe("attn_bwd", s, flop, 0.0);
   const bool kref = k_reference_grad != 0;
@@ -1274,19 +1824,19 @@ int mle_attention_bwd(mle_stream stream, const float* q, const float* k, const f
     }
   } else if (causal) {
     if (kref) {
-      mle::launch(attn_bwd_kv_kernel<true, false>, grid, 128, 0, s, a);
-      mle::launch(attn_bwd_q_kernel<true, true>, grid, 128, 0, s, a);
-    } else {
-      mle::launch(attn_bwd_kv_kernel<true, true>, grid, 128, 0, s, a);
-      mle::launch(attn_bwd_q_kernel<true, false>, grid, 128, 0, s, a);
+      mle::launch(attn_bwd_kv_split_kernel<true>, blocks, 256, 0, s, a);
+      mle::launch(attn_bwd_q_split_kernel<true, true>, blocks, 256, 0, s, a);
+    } else {  // dK needs a second pass over the finished D: the fp32 kernel
+      mle::launch(attn_bwd_kv_kernel<true>, grid, 128, 0, s, a);
+      mle::launch(attn_bwd_q_split_kernel<true, false>, blocks, 256, 0, s, a);
     }
   } else {
     if (kref) {
-      mle::launch(attn_bwd_kv_kernel<false, false>, grid, 128, 0, s, a);
-      mle::launch(attn_bwd_q_kernel<false, true>, grid, 128, 0, s, a);
+      mle::launch(attn_bwd_kv_split_kernel<false>, blocks, 256, 0, s, a);
+      mle::launch(attn_bwd_q_split_kernel<false, true>, blocks, 256, 0, s, a);
     } else {
-      mle::launch(attn_bwd_kv_kernel<false, true>, grid, 128, 0, s, a);
-      mle::launch(attn_bwd_q_kernel<false, false>, grid, 128, 0, s, a);
+      mle::launch(attn_bwd_kv_kernel<false>, grid, 128, 0, s, a);
+      mle::launch(attn_bwd_q_split_kernel<false, false>, blocks, 256, 0, s, a);
     }
   }
   return check_launch("mle_attention_bwd");
