@@ -192,7 +192,7 @@ int mle_act_fwd(mle_stream stream, int kind, const float* x, float* y, size_t n)
 int mle_act_bwd(mle_stream stream, int kind, const float* x, const float* dy, float* dx, size_t n, int accumulate);
 
 /* ------------------------------------------------------------------------- */
-/* GEMM (fp32 MFMA)                                                          */
+/* GEMM (fp32 accuracy: split bf16 MFMA, or fp32 MFMA for small products)    */
 /* ------------------------------------------------------------------------- */
 
 /* C[b] = alpha * op(A[b]) * op(B[b]) + beta * C[b],  b < batch, row-major.
@@ -241,7 +241,7 @@ int mle_gemm_batched_ex(mle_stream stream, int trans_a, int trans_b, int M, int 
                         void* ws, size_t ws_bytes);
 
 /* C = alpha * sum_{t < terms} op(A + t*stride_a_term) op(B + t*stride_b_term) + beta * C,
- * the terms summed in order (deterministic: on the register-direct kernel
+ * the terms summed in order (deterministic: on the split-bf16 kernel
  * they extend one K loop; otherwise each term is a split whose partial
  * products are reduced in term order).  The input gradient of several
  * Linear layers that share an input, dX = sum_t dY_t W_t^T, in one launch
@@ -309,7 +309,7 @@ int mle_gemm_act_bwd(mle_stream stream, int trans_a, int trans_b, int M, int N, 
  *   db_l     += sum_rows dY_l          (db may be NULL)
  * Layer l's dY, W (and dW), db sit at l * stride_dy, l * stride_w, l * stride_db
  * floats (strides unused when layers == 1).  When both products run on the
- * register-direct GEMM at most one workgroup per CU each, or both on one of
+ * split-bf16 GEMM at most one workgroup per CU each, or both on one of
  * the small-product kernels, they share one launch; otherwise dX then dW (a
  * weight gradient of one round of tiles beside a larger dX runs as two K
  * splits).  Needs mle_linear_bwd_ws_bytes(rows, in, out, layers) bytes of
@@ -623,7 +623,7 @@ int mle_copy_crop_bwd(mle_stream stream, const float* dy, float* dx1, float* dx2
 int mle_weight_swap(mle_stream stream, const float* src, float* dst, int o, int i, int khw, int accumulate);
 
 /* ------------------------------------------------------------------------- */
-/* Convolution (NCHW input, OIHW weights), implicit GEMM on fp32 MFMA        */
+/* Convolution (NCHW input, OIHW weights), implicit GEMM, fp32 accuracy      */
 /* ------------------------------------------------------------------------- */
 
 /* y = conv(x, w) + b (b may be NULL).  CV2D (Engine/kernels.cu:985-1019). */

@@ -42,8 +42,8 @@ import sys
 from collections import defaultdict
 
 FAMILIES = {"gemm_nn": (0, 0), "gemm_nt": (0, 1), "gemm_tn": (1, 0), "gemm_tt": (1, 1)}
-GEMM_KERNEL = re.compile(r"gemm_(?:direct_|stream_)?kernel<(\d), (\d)")
-PAIR_KERNEL = re.compile(r"gemm_pair_kernel<")
+GEMM_KERNEL = re.compile(r"gemm_(?:split_kernel<split::Shape<[^>]*>, |kernel<)(\d), (\d)")
+PAIR_KERNEL = re.compile(r"gemm_split_pair_kernel<")
 COPY_KERNEL = "ScaleWriteOp"
 CUS, SIMDS = 256, 4
 NAME_WIDTH = 100
@@ -73,12 +73,12 @@ def instances(db: str, counter: str) -> dict[int, int]:
     return {d: n for d, n in rows}
 
 
-CONV_DIRECT = re.compile(r"conv[13]_direct_kernel<(\w+)")
-OTHER_FAMILIES = [("conv_wgrad", re.compile(r"conv[13]_wgrad_kernel<")),
+CONV_GATHER = re.compile(r"conv(?:[13]_direct_kernel<|_split_kernel<split::Shape<[^>]*>, )(\w+)")
+OTHER_FAMILIES = [("conv_wgrad", re.compile(r"wgrad_split_kernel<")),
                   ("adam_update", re.compile(r"adam(_vec)?_kernel<")),
                   ("sqnorm", re.compile(r"sqnorm_partial<")),
-                  ("attn_fwd", re.compile(r"attn_(stats|fwd)_kernel<")),
-                  ("attn_bwd", re.compile(r"attn_bwd_(kv|q)_kernel<"))]
+                  ("attn_fwd", re.compile(r"attn_(stats|fwd)(_slice|_split)?_kernel<")),
+                  ("attn_bwd", re.compile(r"attn_bwd_(kv|q|slice)(_split)?_kernel<"))]
 
 
 def family_of(name: str) -> str | None:
@@ -89,7 +89,7 @@ def family_of(name: str) -> str | None:
     if m:
         key = (int(m.group(1)), int(m.group(2)))
         return next((f for f, v in FAMILIES.items() if v == key), None)
-    m = CONV_DIRECT.search(name)
+    m = CONV_GATHER.search(name)
     if m:
         return "conv_dgrad" if m.group(1) in ("true", "1") else "conv_fwd"
     return next((f for f, rx in OTHER_FAMILIES if rx.search(name)), None)
