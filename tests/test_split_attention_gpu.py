@@ -1,4 +1,5 @@
-"""The attention passes on split bf16 products (seq > 256) against float64.
+"""The attention passes on split bf16 products (seq > 256, unmasked seq > 128)
+against float64.
 
 Tolerance: a score is a 64-term product, |error| <= 8 * 2^-24 of its terms'
 magnitudes; it enters exp() as an absolute error of the exponent, next to
@@ -49,9 +50,13 @@ def run(hip, q, k, v, do, b, h, s, ld, scale, causal, kref):
     return [x.numpy((b, s, ld)) for x in out]
 
 
-# whole and half column blocks (128), several heads and batch items, a wider ld
+# whole and half column blocks (128), several heads and batch items, a wider ld;
+# unmasked up to 256 positions: both directions split (up to 128 slices, or
+# whole blocks), the forward alone (more slices), neither (128 positions)
 @pytest.mark.parametrize("b,h,s,extra,causal,kref", [
-    (2, 3, 320, 0, 1, 1), (1, 2, 448, 64, 0, 1), (2, 1, 512, 0, 1, 0), (1, 9, 576, 0, 0, 0), (1, 1, 1088, 128, 1, 1)])
+    (2, 3, 320, 0, 1, 1), (1, 2, 448, 64, 0, 1), (2, 1, 512, 0, 1, 0), (1, 9, 576, 0, 0, 0), (1, 1, 1088, 128, 1, 1),
+    (1, 2, 192, 64, 0, 1), (1, 2, 256, 0, 0, 0), (2, 64, 192, 0, 0, 1), (3, 43, 192, 0, 0, 1), (3, 43, 192, 0, 0, 0),
+    (3, 43, 256, 0, 0, 1), (3, 43, 256, 0, 0, 0), (1, 2, 128, 0, 0, 1), (1, 2, 256, 0, 1, 1)])
 def test_split_attention(hip, b, h, s, extra, causal, kref):
     r = rng(b + h + s + causal)
     ld = h * HD + extra
