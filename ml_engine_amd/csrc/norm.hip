@@ -13,6 +13,8 @@
 //   pass 2: each chunk's workgroup combines its group's chunk partials in a
 //           fixed order (Chan et al. pairwise update) and normalises.
 // The backward uses the same split for sum(dy) and sum(dy*y).
+// Groups of at most 4 chunks run both passes in one kernel, a workgroup per
+// group (norm_fwd_group, norm_bwd_group).
 #include "activation.hpp"
 #include "common.hpp"
 
@@ -52,7 +54,8 @@ __device__ __forceinline__ size_t at(const NormShape& sh, int g, size_t e) {
 // t + i NT.
 template <bool VEC>
 __device__ __forceinline__ size_t elem(size_t c0, int i) {
-  return VEC ? c0 + 4 * (threadIdx.x + (size_t)(i / 4) * NT) + (i % 4) : c0 + threadIdx.x + (size_t)i * NT;
+  const unsigned t = threadIdx.x % NT;  // a workgroup may hold several chunks
+  return VEC ? c0 + 4 * (t + (size_t)(i / 4) * NT) + (i % 4) : c0 + t + (size_t)i * NT;
 }
 
 template <bool SEG, bool VEC>
@@ -240,7 +243,9 @@ __device__ __forceinline__ PartPre part_pre(const double* __restrict__ part, con
 // The group's (mean, M2) from its chunk partials, computed by every wave of
 // the workgroup with the same fixed order: lane l first merges chunks l,
 // l + 64, ... in turn, then lanes merge pairwise in a tree (lower lane first).
-// `pre` holds chunk l's partial (part_pre).
+// `pre` holds chunk l's partial (part_pre).  LANES: at least nchunk or 64 (the
+// lanes past the chunks merge nothing).
+template <int LANES = 64>
 __device__ __forceinline__ void group_stats_from(const PartPre& pre, const double* __restrict__ part,
                                                  const NormShape& sh, int g, double& mean, double& m2) {
   const int lane = threadIdx.x & 63;
@@ -249,7 +254,7 @@ __device__ __forceinline__ void group_stats_from(const PartPre& pre, const doubl
   if (lane < sh.nchunk) chan_merge(n, mu, M, chunk_n(sh, lane), pre.a, pre.b);
   for (int c = lane + 64; c < sh.nchunk; c += 64) chan_merge(n, mu, M, chunk_n(sh, c), p[2 * c], p[2 * c + 1]);
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
+  for (int off = 1; off < LANES; off <<= 1) {
     const double nb = __shfl_down(n, off, 64), mub = __shfl_down(mu, off, 64), Mb = __shfl_down(M, off, 64);
     if ((lane & (2 * off - 1)) == 0 && lane + off < 64) chan_merge(n, mu, M, nb, mub, Mb);
   }
@@ -258,6 +263,7 @@ __device__ __forceinline__ void group_stats_from(const PartPre& pre, const doubl
 }
 
 // The group's sum(dy) and sum(dy * y), same fixed order.
+template <int LANES = 64>
 __device__ __forceinline__ void group_sums_from(const PartPre& pre, const double* __restrict__ part,
                                                 const NormShape& sh, int g, double& a, double& b) {
   const int lane = threadIdx.x & 63;
@@ -273,7 +279,7 @@ __device__ __forceinline__ void group_sums_from(const PartPre& pre, const double
     b += p[2 * c + 1];
   }
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
+  for (int off = 1; off < LANES; off <<= 1) {
     const double ab = __shfl_down(a, off, 64), bb = __shfl_down(b, off, 64);
     if ((lane & (2 * off - 1)) == 0 && lane + off < 64) {
       a += ab;
@@ -419,6 +425,13 @@ __global__ __launch_bounds__(NT) void norm_bwd_partial(const float* __restrict__
   }
 }
 
+// A gradient's old value plus v, v rounded first (no fma): every backward
+// kernel, whatever the compiler makes of its branches, adds the same bits.
+__device__ __forceinline__ float add_rounded(float old, float v) {
+#pragma clang fp contract(off)
+  return old + v;
+}
+
 // Per group, once (the LayerNorm layout quirk reads other groups' sums per
 // element): fin[2g] = sum(dy), fin[2g+1] = sum(dy * y), same order as group_sums.
 __global__ __launch_bounds__(64) void norm_bwd_final(const double* __restrict__ part, NormShape sh,
@@ -500,7 +513,7 @@ __global__ __launch_bounds__(NT) void norm_bwd_apply(const float* __restrict__ y
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           const float v = r * (gv[u][k] - (sg / fN) - yv[u][k] * (sgy / fN));
-          d[u][k] = acc ? d[u][k] + v : v;
+          d[u][k] = acc ? add_rounded(d[u][k], v) : v;
           d2[u][k] = acc2 ? d2[u][k] + d[u][k] : d[u][k];
           d3[u][k] = acc3 ? d3[u][k] + d[u][k] : d[u][k];
         }
@@ -530,7 +543,7 @@ __global__ __launch_bounds__(NT) void norm_bwd_apply(const float* __restrict__ y
       terms((int)(idx / quirk_hw), sg, sgy, r);
     }
     const float v = r * (dy[idx] - (sg / fN) - y[idx] * (sgy / fN));
-    const float nv = acc ? dx_in[idx] + v : v;
+    const float nv = acc ? add_rounded(dx_in[idx], v) : v;
     dx[idx] = nv;
     if (EXTRA) dx2[idx] = acc2 ? dx2[idx] + nv : nv;
     if (EXTRA && dx3) dx3[idx] = acc3 ? dx3[idx] + nv : nv;
@@ -563,13 +576,199 @@ void with_act(int kind, F f) {
   }
 }
 
+// ------------------------------------------------------------- whole groups
+// A group of at most 4 chunks fits a workgroup's registers, so each direction
+// reads its operands once and is one launch: SUB sub-blocks of NT threads hold
+// CPS chunks each, the chunk partials meet in LDS, and the results follow from
+// registers.  Every sum and merge has the order of the two-pass kernels, so
+// the bits are the same.  Bound by memory; forward / backward us, two
+// passes against one kernel: 512 groups of 16384 with SiLU 22.9 / 39.0 and
+// 21.9 / 28.8; 1024 of 3069 17.7 / 22.3 and 11.5 / 17.0; 16 of 1568 9.2 / 10.3
+// and 6.2 / 6.5.
+constexpr int kGroupChunks = 4;
+
+// block_sum over each sub-block of NT threads (the same order); red: NT / 64
+// values per sub-block.
+template <int SUB>
+__device__ __forceinline__ double sub_sum(double v, double* red) {
+  if (SUB == 1) return block_sum<NT>(v, red);
+  v = wave_sum(v);
+  const int wid = threadIdx.x >> 6;
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[wid] = v;
+  __syncthreads();
+  double t = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) t += red[wid / (NT / 64) * (NT / 64) + w];
+  return t;
+}
+
+// Forward: statistics, y, and with ACT >= 0 act_out as norm_apply writes them.
+template <bool VEC, int ACT, int SUB, int CPS>
+__global__ __launch_bounds__(NT * SUB, 4) void norm_fwd_group(const float* __restrict__ x, float* __restrict__ y,
+                                                           float* __restrict__ stats, NormShape sh, float eps,
+                                                           float* __restrict__ act_out, const float* __restrict__ cbias,
+                                                           uint32_t cb_hw, uint32_t cb_ch) {
+  __shared__ double red[SUB * NT / 64], part[2 * SUB * CPS];
+  const int g = blockIdx.x, sub = threadIdx.x / NT;
+  float v[CPS][VPT];
+#pragma unroll
+  for (int j = 0; j < CPS; ++j) load_chunk<false, VEC>(x, sh, g, (size_t)(sub + j * SUB) * CH, v[j]);
+#pragma unroll
+  for (int j = 0; j < CPS; ++j) {
+    const int ck = sub + j * SUB;
+    const size_t c0 = (size_t)ck * CH;
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) s += v[j][i];
+    s = sub_sum<SUB>(s, red);
+    const double mean = ck < sh.nchunk ? s / chunk_n(sh, ck) : 0.0;
+    double m2 = 0.0;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const double d = (double)v[j][i] - mean;
+      if (elem<VEC>(c0, i) < sh.N) m2 += d * d;
+    }
+    m2 = sub_sum<SUB>(m2, red);
+    if (threadIdx.x % NT == 0) {
+      part[2 * ck] = mean;
+      part[2 * ck + 1] = m2;
+    }
+  }
+  __syncthreads();
+  double mean_d, m2_d;
+  group_stats_from<kGroupChunks>(part_pre(part, sh, 0), part, sh, 0, mean_d, m2_d);
+  const float mean = (float)mean_d, ssd = (float)m2_d;
+  const float r = rsqrtf((1.0f / (float)sh.N) * ssd + eps);
+  if (threadIdx.x == 0) {
+    stats[2 * g] = mean;
+    stats[2 * g + 1] = ssd;
+  }
+#pragma unroll
+  for (int j = 0; j < CPS; ++j) {
+    const size_t c0 = (size_t)(sub + j * SUB) * CH;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) v[j][i] = (v[j][i] - mean) * r;
+    store_chunk<false, VEC>(y, sh, g, c0, v[j]);
+    if (ACT >= 0) {
+#pragma unroll
+      for (int i = 0; i < VPT; ++i) v[j][i] = act_f<ACT < 0 ? 0 : ACT>(v[j][i]);
+      if (cbias) {
+#pragma unroll
+        for (int i = 0; i < VPT; i += VEC ? 4 : 1) {  // a float4 never straddles a channel (the host checks cb_hw % 4 == 0)
+          const size_t e = elem<VEC>(c0, i);
+          const float cb = e < sh.N ? cbias[(at<false>(sh, g, e) / cb_hw) % cb_ch] : 0.f;
+#pragma unroll
+          for (int k = 0; k < (VEC ? 4 : 1); ++k) v[j][i + k] = v[j][i + k] + cb;
+        }
+      }
+      store_chunk<false, VEC>(act_out, sh, g, c0, v[j]);
+    }
+  }
+}
+
+// Backward: dy (formed and stored as norm_bwd_partial does with ACT >= 0), its
+// sums, and dx as norm_bwd_apply writes it.
+template <bool VEC, int ACT, int SUB, int CPS>
+__global__ __launch_bounds__(NT * SUB, 4) void norm_bwd_group(const float* __restrict__ y, const float* dy,
+                                                           const float* da, float* dy_out, int acc_dy, float* dx,
+                                                           int acc, const float* __restrict__ stats, NormShape sh,
+                                                           float eps) {
+  __shared__ double red[SUB * NT / 64], part[2 * SUB * CPS];
+  const int g = blockIdx.x, sub = threadIdx.x / NT;
+  const float ssd = stats[2 * g + 1], fN = (float)(int)sh.N;
+  float yv[CPS][VPT], gv[CPS][VPT];
+#pragma unroll
+  for (int j = 0; j < CPS; ++j) {
+    const size_t c0 = (size_t)(sub + j * SUB) * CH;
+    load_chunk<false, VEC>(y, sh, g, c0, yv[j]);
+    load_chunk<false, VEC>(ACT >= 0 ? da : dy, sh, g, c0, gv[j]);
+  }
+#pragma unroll
+  for (int j = 0; j < CPS; ++j) {
+    const int ck = sub + j * SUB;
+    const size_t c0 = (size_t)ck * CH;
+    if (ACT >= 0) {
+      float old[VPT];
+      if (acc_dy) load_chunk<false, VEC>(dy_out, sh, g, c0, old);
+#pragma unroll
+      for (int i = 0; i < VPT; ++i) {
+        // product rounded, then the add (no fma): the activation kernel's steps
+#pragma clang fp contract(off)
+        const float t = act_df<ACT < 0 ? 0 : ACT>(yv[j][i]) * gv[j][i];
+        gv[j][i] = acc_dy ? old[i] + t : t;
+      }
+      store_chunk<false, VEC>(dy_out, sh, g, c0, gv[j]);
+      // past the group's end the loads gave zeros: they add nothing
+    }
+    double sg = 0.0, sgy = 0.0;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      sg += gv[j][i];
+      sgy += (double)(gv[j][i] * yv[j][i]);
+    }
+    sg = sub_sum<SUB>(sg, red);
+    sgy = sub_sum<SUB>(sgy, red);
+    if (threadIdx.x % NT == 0) {
+      part[2 * ck] = sg;
+      part[2 * ck + 1] = sgy;
+    }
+  }
+  __syncthreads();
+  double a, b;
+  group_sums_from<kGroupChunks>(part_pre(part, sh, 0), part, sh, 0, a, b);
+  const float sg = (float)a, sgy = (float)b, r = rsqrtf(ssd / fN + eps);
+#pragma unroll
+  for (int j = 0; j < CPS; ++j) {
+    const size_t c0 = (size_t)(sub + j * SUB) * CH;
+    float d[VPT];
+    if (acc) load_chunk<false, VEC>(dx, sh, g, c0, d);
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const float v = r * (gv[j][i] - (sg / fN) - yv[j][i] * (sgy / fN));
+      d[i] = acc ? add_rounded(d[i], v) : v;
+    }
+    store_chunk<false, VEC>(dx, sh, g, c0, d);
+  }
+}
+
+// f(SUB, CPS) for the groups of sh: a chunk per sub-block, except that with
+// more groups of 3 or 4 chunks than CUs two workgroups of half the threads share a
+// CU, one loading while the other reduces (512 groups of 16384, forward /
+// backward: 25 / 33 us with four sub-blocks, 22 / 29 so; not the backward of
+// GELU, which needs more registers than that leaves: 1024 groups, 52 against 61).
+template <class F>
+void with_group(const NormShape& sh, bool heavy, F f) {
+  using std::integral_constant;
+  if (sh.nchunk == 1) f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+  else if (sh.nchunk == 2) f(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+  else if (heavy || sh.groups_tot <= 256) f(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+  else f(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+}
+
+// Contiguous groups of at most 16384 elements.  Larger ones would make one
+// workgroup walk what a chunk per workgroup spreads (64 groups of 32768,
+// forward / backward: 11 / 13 us in two passes, 17 / 23 in one).
+bool whole_group(const NormShape& sh) { return !sh.seg && sh.nchunk <= kGroupChunks; }
+
 // act >= 0: the normalisation also writes act_out = act(y) (+ cbias[channel]).
 void launch_fwd(hipStream_t s, const NormShape& sh, const float* x, float* y, float* stats, void* ws, float eps,
                 bool stats_ready = false, int act = -1, float* act_out = nullptr, const float* cbias = nullptr,
                 uint32_t cb_hw = 1, uint32_t cb_ch = 1) {
   dim3 grid(sh.nchunk, sh.groups_tot);
   double* part = static_cast<double*>(ws);
-  const bool v = vec_ok(sh, {x, y}) && (act < 0 || aligned16(act_out));
+  const bool v = vec_ok(sh, {x, y}) && (act < 0 || aligned16(act_out)) && (!cbias || cb_hw % 4 == 0);
+  if (!stats_ready && whole_group(sh)) {
+    with_act(act, [&](auto K) {
+      with_group(sh, false, [&](auto SUB, auto CPS) {
+        constexpr int A = decltype(K)::value, B = decltype(SUB)::value, C = decltype(CPS)::value;
+        const dim3 one(sh.groups_tot);
+        if (v) norm_fwd_group<true, A, B, C><<<one, NT * B, 0, s>>>(x, y, stats, sh, eps, act_out, cbias, cb_hw, cb_ch);
+        else norm_fwd_group<false, A, B, C><<<one, NT * B, 0, s>>>(x, y, stats, sh, eps, act_out, cbias, cb_hw, cb_ch);
+      });
+    });
+    return;
+  }
   if (!stats_ready || sh.seg) {  // otherwise pass 1 ran in the producer of x
     if (sh.seg) {
       if (v) norm_stats_partial<true, true><<<grid, NT, 0, s>>>(x, sh, part);
@@ -638,6 +837,19 @@ void launch_bwd_apply(hipStream_t s, const NormShape& sh, const float* y, const 
 void launch_bwd(hipStream_t s, const NormShape& sh, const float* y, const float* dy, float* dx, const float* stats,
                 void* ws, float eps, size_t quirk, int accumulate, int act = -1, const float* da = nullptr,
                 int acc_dy = 0) {
+  if (!quirk && whole_group(sh)) {
+    const bool v = vec_ok(sh, {y, dy, dx}) && (act < 0 || aligned16(da));
+    float* dyw = const_cast<float*>(dy);  // written only with act >= 0
+    with_act(act, [&](auto K) {
+      with_group(sh, act == MLE_GELU, [&](auto SUB, auto CPS) {
+        constexpr int A = decltype(K)::value, B = decltype(SUB)::value, C = decltype(CPS)::value;
+        const dim3 one(sh.groups_tot);
+        if (v) norm_bwd_group<true, A, B, C><<<one, NT * B, 0, s>>>(y, dy, da, dyw, acc_dy, dx, accumulate, stats, sh, eps);
+        else norm_bwd_group<false, A, B, C><<<one, NT * B, 0, s>>>(y, dy, da, dyw, acc_dy, dx, accumulate, stats, sh, eps);
+      });
+    });
+    return;
+  }
   launch_bwd_partials(s, sh, y, dy, ws, quirk, act, da, acc_dy);
   launch_bwd_apply(s, sh, y, dy, dx, accumulate, stats, ws, eps, quirk);
 }
