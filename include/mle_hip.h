@@ -640,8 +640,8 @@ int mle_conv2d_wgrad(mle_stream stream, const float* x, const float* dy, float* 
 /* mle_conv2d_wgrad, and db[c] (+)= sum_{n,oh,ow} dy[n][c] (db may be NULL;
  * accumulate_db 1 adds, 0 assigns): the bias gradient of Convolute2D's
  * backward (GV2D then Channel_Squeeze1D over dy, Engine/engine.cu:3768-3769)
- * taken from the dy rows the weight-gradient kernel already reads (3x3 pad 1
- * and 1x1 stride 1; other filters run the channel sum after the weight
+ * taken from the dy values the weight-gradient kernel already reads (the
+ * split-bf16 kernel; beyond its limits the channel sum runs after the weight
  * gradient).  Same workspace as mle_conv2d_wgrad. */
 int mle_conv2d_wgrad_bias(mle_stream stream, const float* x, const float* dy, float* dw, float* db,
                           int accumulate_db, int n, int cin, int h, int w_in, int cout, int kh, int kw, int pad,
@@ -649,9 +649,10 @@ int mle_conv2d_wgrad_bias(mle_stream stream, const float* x, const float* dy, fl
 
 /* A 3 x 3 (pad 1) and a 1 x 1 (pad 0) convolution of the same input, both
  * stride 1 (ResidualBlock's conv1 and skip convolution, Engine/diffusion.cu:
- * 129-137): the two CV2D forwards (Engine/kernels.cu:985-1019) in one launch,
- * and the two CV2D_GradInput passes (Engine/kernels.cu:1052-1089) adding into
- * the one dx in one launch, dx (+)= dgrad3(dy3) + dgrad1(dy1).  _supported
+ * 129-137): the two CV2D forwards (Engine/kernels.cu:985-1019), each on
+ * its own kernel, and the two CV2D_GradInput passes (Engine/kernels.cu:1052-1089)
+ * adding into the one dx, dx (+)= dgrad3(dy3) + dgrad1(dy1), in one launch for
+ * at most 64 input channels.  _supported
  * says whether the shapes run on these kernels (otherwise the per-convolution
  * calls do; the paired calls return MLE_ERR_UNSUPPORTED). */
 int mle_conv2d_pair_supported(int n, int cin, int h, int w, int cout3, int cout1);

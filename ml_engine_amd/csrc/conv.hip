@@ -836,7 +836,7 @@ int mle_conv2d_wgrad_bias(mle_stream stream, const float* x, const float* dy, fl
 }
 
 
-// ---- a 3 x 3 and a 1 x 1 convolution of one input, in one launch ----------
+// ---- a 3 x 3 and a 1 x 1 convolution of one input -------------------------
 // (a residual block's first convolution and its skip; both stride 1)
 
 // Arguments of both products for the paired forward (dg = 0) or input

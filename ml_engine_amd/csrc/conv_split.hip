@@ -184,8 +184,8 @@ struct WeightLoad : Chunks<R * 4 / NTH, false> {
 // True on every thread when some thread of the workgroup saw a value the split
 // cannot represent; then v (+ lo) is cleared for fp32_tile.
 template <class S>
-__device__ __forceinline__ bool redo(f32x4 (&v)[S::BI][S::BN], f32x4 (&lo)[S::BI][S::BN], const Tiny& tiny) {
-  if (!__syncthreads_or(needs_fp32<S>(v, lo, tiny))) return false;
+__device__ __forceinline__ bool redo(f32x4 (&v)[S::BI][S::BN], f32x4 (&lo)[S::BI][S::BN]) {
+  if (!__syncthreads_or(needs_fp32<S>(v, lo))) return false;
 #pragma unroll
   for (int i = 0; i < S::BI; ++i)
 #pragma unroll
@@ -206,7 +206,6 @@ __global__ __launch_bounds__(S::NTH * S::KG, 2) void conv_split_kernel(GatherArg
   fill_table<DG>(a, tab, tid, S::NTH * S::KG);
   __syncthreads();
   f32x4 v[BI][BN], lo[BI][BN];
-  Tiny tiny;
   {
     // With two K groups each takes half of the stages.
     const int group = k_group<S>(), t = tid % S::NTH;
@@ -217,14 +216,14 @@ __global__ __launch_bounds__(S::NTH * S::KG, 2) void conv_split_kernel(GatherArg
     if constexpr (DG) {
       WeightLoad<S::TM, S::NTH> la;
       la.init(a, tab.wt, k0, m0, t);
-      mma_loop<S>(buf, la, lb, nk, v, lo, tiny);
+      mma_loop<S>(buf, la, lb, nk, v, lo);
     } else {
       MatLoad<false, S::TM, S::NTH, TAIL> la;
       la.init(a.wt, a.K, a.M, a.K, m0, k0, S::KG == 1 ? a.K : min(a.K - k0, nk * KS), 1, 0, t);
-      mma_loop<S>(buf, la, lb, nk, v, lo, tiny);
+      mma_loop<S>(buf, la, lb, nk, v, lo);
     }
   }
-  const bool again = redo<S>(v, lo, tiny);
+  const bool again = redo<S>(v, lo);
   join_groups<S>(lds, v, lo);
   if (k_group<S>() != 0) return;  // (no barrier follows)
   if (again) {
@@ -445,7 +444,6 @@ __global__ __launch_bounds__(S::NTH * S::KG, 2) void wgrad_split_kernel(WgradArg
   tab.fill(a, kbeg, klen, tid, S::NTH * S::KG);
   __syncthreads();
   f32x4 v[BI][BN], lo[BI][BN];
-  Tiny tiny;
   {
     using LA = RowLoad<S::TM, S::NTH, V4, true>;
     LA la;
@@ -456,11 +454,11 @@ __global__ __launch_bounds__(S::NTH * S::KG, 2) void wgrad_split_kernel(WgradArg
     if constexpr (ONE) {
       RowLoad<S::TN, S::NTH, V4, false> lb;
       lb.init(a.x, a.x_bytes, a.N, a.g.h * a.g.w, tab.src, k0, nk, n0, t);
-      mma_loop<S>(lds + group * S::LDS, la, lb, nk, v, lo, tiny);
+      mma_loop<S>(lds + group * S::LDS, la, lb, nk, v, lo);
     } else {
       XLoad<S::TN, S::NTH, T> lb;
       lb.init(a, &tab, k0, n0, t);
-      mma_loop<S>(lds + group * S::LDS, la, lb, nk, v, lo, tiny);
+      mma_loop<S>(lds + group * S::LDS, la, lb, nk, v, lo);
     }
     if (a.db && tn == 0) {  // the lane groups' sums of each dY row, added in order
       float* red = reinterpret_cast<float*>(lds);
@@ -481,7 +479,7 @@ __global__ __launch_bounds__(S::NTH * S::KG, 2) void wgrad_split_kernel(WgradArg
       }
     }
   }
-  const bool again = redo<S>(v, lo, tiny);
+  const bool again = redo<S>(v, lo);
   join_groups<S>(lds, v, lo);
   if (k_group<S>() != 0) return;  // (no barrier follows)
   if (again) {

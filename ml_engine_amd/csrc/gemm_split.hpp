@@ -26,7 +26,6 @@ __device__ __forceinline__ void split_tile(const GemmArgs& g, int tm, int tn, in
   const int klen = (g.grouped ? g.K : min(g.K, kbeg + g.kchunk)) - kbeg;
   const int tid = threadIdx.x, group = split::k_group<S>(), t = tid % S::NTH;
   f32x4 v[BI][BN], lo[BI][BN];
-  split::Tiny tiny;
   {
     LA la;
     LB lb;
@@ -35,7 +34,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs& g, int tm, int tn, in
     const int k0 = group * nk * split::KS, kl = S::KG == 1 ? klen : min(klen - k0, nk * split::KS);
     la.init(A, g.lda, g.M, g.K, m0, kbeg + k0, kl, g.kterms, g.gsa, t);
     lb.init(B, g.ldb, g.N, g.K, n0, kbeg + k0, kl, g.kterms, g.gsb, t);
-    split::mma_loop<S>(lds + group * S::LDS, la, lb, g.kterms * nk, v, lo, tiny);
+    split::mma_loop<S>(lds + group * S::LDS, la, lb, g.kterms * nk, v, lo);
     if (COLSUM && tm == 0) {
       // the lane groups' sums of each column, added in order
       float* red = reinterpret_cast<float*>(lds);
@@ -56,7 +55,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs& g, int tm, int tn, in
       }
     }
   }
-  const bool redo = __syncthreads_or(split::needs_fp32<S>(v, lo, tiny));
+  const bool redo = __syncthreads_or(split::needs_fp32<S>(v, lo));
   split::join_groups<S>(lds, v, lo);
   if (group != 0) return;  // (no barrier follows)
   if (redo) {

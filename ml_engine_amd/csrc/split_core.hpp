@@ -17,12 +17,17 @@
 // (all six in one accumulator is biased by the MFMA's truncation and loses to
 // the fp32 MFMA on one-sided operands: 9.2e-7 against 8.0e-7 at K 4096.)
 //
+// The tile engine splits 2^24 x: the last bit of any fp32 value is then at least
+// 2^-125, so every part of every value, the smallest included, is exact and
+// normal; the sums are scaled back by 2^-48.  (Without the scale values
+// under 2^-110 lose bits.  They are ordinary: a softmax gradient far from its
+// target holds some in most tiles.  Sending those tiles to fp32_tile made a
+// training step three times slower as soon as they appeared.)
+//
 // What the split cannot represent goes to the fp32 MFMA instead, tile by
-// tile: an infinity or NaN, or a value that rounds to infinity in bf16, makes
-// its products NaN, which the accumulators show at the end; a nonzero value
-// below 2^-110, whose third part would fall under bf16's smallest step, is
-// noted while splitting.  Such a tile is multiplied again by
-// fp32_tile (the same results as before the split).
+// tile: an infinity or NaN, a value of 2^104 or more, or a sum of 2^80 or more
+// makes its accumulators infinite or NaN.  Such a tile is multiplied again by
+// fp32_tile (fp32 products).
 //
 // Tile engine: a workgroup of CM x CN waves, each (16 BI) x (16 BN) of C.
 // 32-deep K stages, double-buffered in LDS as three bf16 planes per operand.
@@ -73,8 +78,8 @@ __device__ __forceinline__ unsigned pack_bf16(float a, float b) {
 __device__ __forceinline__ float low_f(unsigned h) { return __builtin_bit_cast(float, h << 16); }
 __device__ __forceinline__ float high_f(unsigned h) { return __builtin_bit_cast(float, h & 0xffff0000u); }
 
-// Smallest (bits << 1) - 1 of the nonzero leading parts seen (zero wraps to
-// the largest value).
+// For splits without the scale: smallest (bits << 1) - 1 of the nonzero leading
+// parts seen (zero wraps to the largest value).
 struct Tiny {
   u16x2 m = {0xffff, 0xffff};
   __device__ __forceinline__ void see(unsigned h) {
@@ -87,8 +92,10 @@ struct Tiny {
   }
 };
 
+constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f;  // of an operand, of a sum of products
+
 // Eight fp32 values to their three bf16 parts.
-__device__ __forceinline__ void split8(const float (&x)[8], u32x4& p0, u32x4& p1, u32x4& p2, Tiny& tiny) {
+__device__ __forceinline__ void split8(const float (&x)[8], u32x4& p0, u32x4& p1, u32x4& p2) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const float a = x[2 * j], b = x[2 * j + 1];
@@ -98,8 +105,13 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4& p0, u32x4& p1
     p0[j] = h;
     p1[j] = m;
     p2[j] = pack_bf16(ra - low_f(m), rb - high_f(m));
-    tiny.see(h);
   }
+}
+// Noting values too small for it.
+__device__ __forceinline__ void split8(const float (&x)[8], u32x4& p0, u32x4& p1, u32x4& p2, Tiny& tiny) {
+  split8(x, p0, p1, p2);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) tiny.see(p0[j]);
 }
 
 __device__ __forceinline__ f32x4 mma(const u32x4& a, const u32x4& b, const f32x4& c) {
@@ -151,12 +163,12 @@ struct WaveMap {
 
 // hi + lo = A B^T over nk stages.  The loaders la / lb give CA / CB chunks of
 // 8 k values per thread and stage: load(x) fetches the next stage's raw values
-// (zeros outside the operand) into a register set, put(lds, x[c], c, tiny)
+// (zeros outside the operand) into a register set, put(lds, x[c], c)
 // splits chunk c into the planes.  nk >= 0; stages past nk are loaded but
 // never multiplied.
 template <class S, class LA, class LB>
 __device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x4 (&hi)[S::BI][S::BN],
-                                         f32x4 (&lo)[S::BI][S::BN], Tiny& tiny) {
+                                         f32x4 (&lo)[S::BI][S::BN]) {
   constexpr int BI = S::BI, BN = S::BN, PA = S::PA, PB = S::PB, STG = S::STAGE;
   constexpr int CA = LA::NC, CB = LB::NC, CT = CA + CB;
   const WaveMap<S> w;
@@ -180,9 +192,9 @@ __device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x
   la.load(xa[0]);
   lb.load(xb[0]);
 #pragma unroll
-  for (int c = 0; c < CA; ++c) la.template put<PA>(lds, xa[0][c], c, tiny);
+  for (int c = 0; c < CA; ++c) la.template put<PA>(lds, xa[0][c], c);
 #pragma unroll
-  for (int c = 0; c < CB; ++c) lb.template put<PB>(lds + 3 * PA, xb[0][c], c, tiny);
+  for (int c = 0; c < CB; ++c) lb.template put<PB>(lds + 3 * PA, xb[0][c], c);
 #pragma unroll
   for (int u = 0; u < D; ++u) {
     la.pre();
@@ -243,8 +255,8 @@ __device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x
 #pragma unroll
         for (int c = 0; c < CT; ++c)
           if (c * (BI - 1) / CT == i) {
-            if (c < CA) la.template put<PA>(nxt, sa[c], c, tiny);
-            else lb.template put<PB>(nxt + 3 * PA, sb[c < CA ? 0 : c - CA], c - CA, tiny);
+            if (c < CA) la.template put<PA>(nxt, sa[c], c);
+            else lb.template put<PB>(nxt + 3 * PA, sb[c < CA ? 0 : c - CA], c - CA);
           }
         if (i + 2 == BI && !LA::kBranch && !LB::kBranch) {
           la.load(sa);
@@ -274,6 +286,13 @@ __device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x
     for (int u = 0; u < D; ++u)
       if (kt + u < nk) stage(kt + u, xa[u], xb[u]);
   }
+#pragma unroll
+  for (int i = 0; i < BI; ++i)
+#pragma unroll
+    for (int n = 0; n < BN; ++n) {
+      hi[i][n] *= kUnscale;
+      lo[i][n] *= kUnscale;
+    }
 }
 
 // This thread's K group.
@@ -307,10 +326,9 @@ __device__ __forceinline__ void join_groups(char* lds, f32x4 (&hi)[S::BI][S::BN]
   }
 }
 
-// Whether this thread saw something the split cannot represent.
+// Whether this thread's sums show something the split cannot represent.
 template <class S>
-__device__ __forceinline__ bool needs_fp32(const f32x4 (&hi)[S::BI][S::BN], const f32x4 (&lo)[S::BI][S::BN],
-                                           const Tiny& tiny) {
+__device__ __forceinline__ bool needs_fp32(const f32x4 (&hi)[S::BI][S::BN], const f32x4 (&lo)[S::BI][S::BN]) {
   float t = 0.f;  // 0 * finite is 0, 0 * infinity and 0 * NaN are NaN
 #pragma unroll
   for (int i = 0; i < S::BI; ++i)
@@ -318,7 +336,7 @@ __device__ __forceinline__ bool needs_fp32(const f32x4 (&hi)[S::BI][S::BN], cons
     for (int n = 0; n < S::BN; ++n)
 #pragma unroll
       for (int r = 0; r < 4; ++r) t = fmaf(0.f, hi[i][n][r] + lo[i][n][r], t);
-  return tiny.found() || !(t == 0.f);
+  return !(t == 0.f);
 }
 
 // The tile on the fp32 MFMA: a(row, k) and b(col, k) read the operands (0
@@ -363,9 +381,12 @@ struct Chunks {
   }
   __device__ __forceinline__ void pre() {}
   template <int PL>
-  __device__ __forceinline__ void put(char* lds, const float (&x)[8], int c, Tiny& tiny) {
+  __device__ __forceinline__ void put(char* lds, const float (&x)[8], int c) {
     u32x4 p0, p1, p2;
-    split8(x, p0, p1, p2, tiny);
+    float s[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s[j] = x[j] * kScale;
+    split8(s, p0, p1, p2);
     if (SUM)
       sum[c] += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
     char* d = lds + dst[c];

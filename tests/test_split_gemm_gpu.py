@@ -64,11 +64,12 @@ def test_split_gemm_edges(hip, ta, tb, M, N, K):
     assert np.all(np.abs(C - (a64 @ b64 + C0)) <= bound(K) * (terms + np.abs(C0)))
 
 
-@pytest.mark.parametrize("what", ["inf", "nan", "max", "tiny", "overflow"])
+@pytest.mark.parametrize("what", ["inf", "nan", "max", "tiny", "denormal", "overflow"])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
 def test_split_gemm_special_values(hip, ta, tb, what):
     """Infinities, NaN, the largest values (which round to infinity in bf16)
-    and values too small for three bf16 parts: as fp32 products give them."""
+    and the smallest (whole rows near and below the end of the normal range,
+    single values among ordinary ones): as fp32 products give them."""
     M, N, K = 700, 600, 200
     r = rng(77 + ta + 2 * tb)
     a, b = r.standard_normal((M, K), dtype=np.float32), r.standard_normal((K, N), dtype=np.float32)
@@ -83,6 +84,10 @@ def test_split_gemm_special_values(hip, ta, tb, what):
     elif what == "tiny":
         a[400:, :] *= np.float32(2.0 ** -112)
         b[:, 100:200] *= np.float32(2.0 ** 40)
+    elif what == "denormal":
+        a[400:, :] *= np.float32(2.0 ** -130)
+        a[:400, ::7] *= np.float32(2.0 ** -120)
+        b *= np.float32(2.0 ** 40)
     else:
         a[50, :], b[:, 60] = np.float32(1e30), np.float32(1e30)
     A, Bm = np.ascontiguousarray(a.T if ta else a), np.ascontiguousarray(b.T if tb else b)
