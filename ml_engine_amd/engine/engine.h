@@ -481,11 +481,11 @@ class Convolute2D {
 // input (a residual block's first convolution and its skip).  `y3` and `y1`
 // are their forward nodes.  When the shapes run on the paired kernels the
 // nodes' lambdas are rewired:
-//  * forward: whichever runs first in a pass computes both outputs in one
-//    launch (mle_conv2d_pair_fwd; the same bits as two launches);
+//  * forward: whichever runs first in a pass computes both outputs
+//    (mle_conv2d_pair_fwd; the same bits as the separate calls);
 //  * backward: each keeps its own weight and bias gradients; the second to
 //    run computes the input gradient of both, dx (+)= dgrad3(dY3) +
-//    dgrad1(dY1), in one launch (mle_conv2d_pair_dgrad).
+//    dgrad1(dY1), in one call (mle_conv2d_pair_dgrad).
 // Both nodes must be evaluated in every pass, as the residual block's are.
 // Returns false (and changes nothing) otherwise.
 namespace mle {
