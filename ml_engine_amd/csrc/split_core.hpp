@@ -20,9 +20,9 @@
 // The tile engine splits 2^24 x: the last bit of any fp32 value is then at least
 // 2^-125, so every part of every value, the smallest included, is exact and
 // normal; the sums are scaled back by 2^-48.  (Without the scale values
-// under 2^-110 lose bits.  They are ordinary: a softmax gradient far from its
-// target holds some in most tiles.  Sending those tiles to fp32_tile made a
-// training step three times slower as soon as they appeared.)
+// under 2^-110 lose bits.  They are ordinary: after some 60 steps a transformer
+// block's gradients hold them in many tiles, and sending those to fp32_tile
+// took its step from 2.3 to 6.5 ms.)
 //
 // What the split cannot represent goes to the fp32 MFMA instead, tile by
 // tile: an infinity or NaN, a value of 2^104 or more, or a sum of 2^80 or more
