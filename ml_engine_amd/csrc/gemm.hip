@@ -560,6 +560,7 @@ struct SplitChoice {
 
 SplitChoice choose_split(int M, int N, int K, int batch, bool may_split) {
   SplitChoice best;
+  if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return best;  // nothing to multiply, nothing to divide
   best.us = 1e30;
   const int st = (K + 31) / 32;
   for (int tile = 0; tile < 3; ++tile) {
@@ -861,7 +862,7 @@ size_t mle_gemm_ws_bytes(int M, int N, int K, int batch) {
   int splits = choose_splits(M, N, K, batch, kchunk);
   // A product of at most 4096 outputs runs on the simple kernel, which leaves
   // the workspace unused; its size stays that of one split per 32 deep stage.
-  if ((double)M * N * batch <= 4096.0) splits = std::max(splits, (K + 31) / 32);
+  if ((double)M * N * batch <= 4096.0 && (double)M * N * batch > 0.0) splits = std::max(splits, (K + 31) / 32);
   if (splits <= 1) return 0;
   return ((size_t)splits * batch * M * N + (size_t)splits * batch * N) * sizeof(float);
 }

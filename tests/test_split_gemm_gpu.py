@@ -199,3 +199,18 @@ def test_split_conv_special_values(hip):
     assert np.array_equal(got[np.isinf(y32)], y32[np.isinf(y32)])
     ok = np.isfinite(y32)
     assert np.all(np.abs(got[ok] - y[ok]) <= bound(cin * 9) * ya[ok])
+
+
+@pytest.mark.parametrize("M,N", [(2300, 2000), (3, 5)])
+def test_empty_depth(hip, M, N):
+    """K = 0: C = beta C + bias, whatever the size of C (more than 4 Mi values
+    go past the small-product kernels); a Linear of no rows has zero gradients."""
+    r = rng(M)
+    C0, bias = r.standard_normal((M, N), dtype=np.float32), r.standard_normal(N, dtype=np.float32)
+    gC, gb = hip.Buffer.from_array(C0), hip.Buffer.from_array(bias)
+    hip.call("mle_gemm_ex", None, 0, 0, M, N, 0, 1.0, None, 0, 0, None, N, 0, 0.5, gC.ptr, N, 0, 1, None, gb.ptr, None, 0)
+    np.testing.assert_array_equal(gC.numpy((M, N)), np.float32(0.5) * C0 + bias)
+    gX, gW = hip.Buffer.from_array(np.zeros(4, np.float32)), hip.Buffer.from_array(C0)
+    dW, db = hip.Buffer.from_array(C0), hip.Buffer.from_array(bias)
+    hip.call("mle_linear_bwd_ex", None, 0, M, N, 1, gX.ptr, gX.ptr, 0, gW.ptr, 0, gX.ptr, 0, dW.ptr, db.ptr, 0, 0, None, 0)
+    assert not dW.numpy().any() and not db.numpy().any()

@@ -1,0 +1,16 @@
+"""CPU checks of the workspace queries: pure functions of the sizes, which any
+program may ask before it has data, sizes of zero included."""
+import pytest
+
+from ml_engine_amd import hip
+
+
+@pytest.mark.parametrize("zero", range(4))
+def test_queries_take_empty_products(zero):
+    sizes = [300, 520, 700, 2]
+    sizes[zero] = 0
+    assert hip.lib().mle_gemm_ws_bytes(*sizes) == 0
+    if zero < 3:  # rows, in, out; a layer there is always
+        for layers in (1, 3):
+            dx = hip.lib().mle_gemm_sum_ws_bytes(sizes[0], sizes[1], layers)
+            assert hip.lib().mle_linear_bwd_ws_bytes(*sizes[:3], layers) == dx
