@@ -1111,13 +1111,16 @@ __global__ __launch_bounds__(128, 2) void attn_bwd_kv_kernel(AttnArgs a) {
 //         the positions; row d = 4 lr + b of block b: b KB + 256 q + 16 (lr ^ 4 b)
 // both written and read without bank conflicts.
 //
-// A workgroup whose sums show an infinity or NaN, or whose operands hold a
-// value the split cannot represent, runs its columns again on the fp32 tile
-// functions above.  What bounds the passes is the vector unit and its overlap
+// Operands, P and dS are split as 2^24 x, as in the tile engine, so every fp32
+// value keeps its bits; scores and sums are scaled back by 2^-48.  A workgroup
+// whose scores or sums show an infinity or NaN (2^80 and more among them)
+// runs its columns again on the fp32 tile functions above.  What bounds the passes is the vector unit and its overlap
 // with the matrix cores at one to two waves per SIMD: splitting and
 // exponentials take about as many cycles as the products.  32 heads of 1024
-// unmasked positions, us: statistics 41, O 79, dV 76, dQ and dK 136; the whole
-// forward and backward 597 on the fp32 matrix cores, 286 here.
+// unmasked positions, us: statistics 37, O 76, dV 71, dQ and dK 129; the whole
+// forward and backward 596 on the fp32 matrix cores, 282 here, and the same
+// with values of 2^-120 in dO (483 when such a value sent its workgroups to
+// the fp32 tiles).
 constexpr int CW = 128;             // columns of a workgroup
 constexpr int kTile = 12288;        // bytes of a staged tile
 using split::u32x4;
@@ -1150,9 +1153,12 @@ __device__ __forceinline__ int cols_slot() {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, b = lane & 3;
   return b * 1024 + w * 256 + (((lane >> 2) ^ (4 * b)) * 16);
 }
-__device__ __forceinline__ void put(char* tile, int slot, const Raw& o, split::Tiny& tiny) {
+__device__ __forceinline__ void put(char* tile, int slot, const Raw& o) {
   u32x4 p0, p1, p2;
-  split::split8(o.x, p0, p1, p2, tiny);
+  float x[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) x[j] = o.x[j] * split::kScale;
+  split::split8(x, p0, p1, p2);
   *reinterpret_cast<u32x4*>(tile + slot) = p0;
   *reinterpret_cast<u32x4*>(tile + slot + 4096) = p1;
   *reinterpret_cast<u32x4*>(tile + slot + 8192) = p2;
@@ -1173,20 +1179,19 @@ __device__ __forceinline__ void mma6(const Frag& a, const Frag& b, f32x4& hi, f3
 // The wave's columns c0 + 16 n + lr of a [seq][64] operand, as B fragments of
 // the two head stages.
 template <int NB>
-__device__ __forceinline__ void load_b(__amdgpu_buffer_rsrc_t r, uint32_t base, int ld, int c0, Frag (&b)[NB][2],
-                                       split::Tiny& tiny) {
+__device__ __forceinline__ void load_b(__amdgpu_buffer_rsrc_t r, uint32_t base, int ld, int c0, Frag (&b)[NB][2]) {
   const int lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
 #pragma unroll
   for (int n = 0; n < NB; ++n)
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const uint32_t e = base + (uint32_t)(c0 + 16 * n + lr) * ld + 32 * s + 4 * q;
-      const f32x4 u = bld4(r, e), v = bld4(r, e + 16);
+      const f32x4 u = bld4(r, e) * split::kScale, v = bld4(r, e + 16) * split::kScale;
       const float x[8] = {u[0], u[1], u[2], u[3], v[0], v[1], v[2], v[3]};
-      split::split8(x, b[n][s][0], b[n][s][1], b[n][s][2], tiny);
+      split::split8(x, b[n][s][0], b[n][s][1], b[n][s][2]);
     }
 }
-// out[i][n] = rows tile (32 positions) times the columns, over the head.
+// out[i][n] = rows tile (32 positions) times the columns, over the head (scaled by 2^48).
 template <int NB>
 __device__ __forceinline__ void score(const char* tile, const Frag (&b)[NB][2], f32x4 (&out)[2][NB]) {
   const int lane = threadIdx.x & 63;
@@ -1206,17 +1211,16 @@ __device__ __forceinline__ void score(const char* tile, const Frag (&b)[NB][2], 
     for (int n = 0; n < NB; ++n) out[i][n] = hi[n] + lo[n];
   }
 }
-// A score block's 8 values per lane and column block, as B fragments.
+// A score block's 8 values per lane and column block (scaled by 2^24), as B fragments.
 template <int NB>
 __device__ __forceinline__ void to_frag(const f32x4 (&v)[2][NB], Frag (&f)[NB]) {
-  split::Tiny ignore;  // single small values are ordinary: below 2^-110 they lose bits, 2^-134 at most (see Peak)
 #pragma unroll
   for (int n = 0; n < NB; ++n) {
     const float x[8] = {v[0][n][0], v[0][n][1], v[0][n][2], v[0][n][3], v[1][n][0], v[1][n][1], v[1][n][2], v[1][n][3]};
-    split::split8(x, f[n][0], f[n][1], f[n][2], ignore);
+    split::split8(x, f[n][0], f[n][1], f[n][2]);
   }
 }
-// hi + lo += cols tile times the fragments, over 32 positions.
+// hi + lo += cols tile times the fragments, over 32 positions (scaled by 2^48).
 template <int NB>
 __device__ __forceinline__ void accumulate(const char* tile, const Frag (&f)[NB], f32x4 (&hi)[4][NB], f32x4 (&lo)[4][NB]) {
   const int lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
@@ -1248,30 +1252,17 @@ __device__ __forceinline__ float finite_mark(const f32x4 (&a)[I][NB]) {
   return t;
 }
 
-// Largest |value| of a column over everything its fragments held.  The split
-// drops at most 2^-134 of a value; a column whose largest is under 2^-80 (and
-// not 0) would notice and goes to the fp32 tile.
-struct Peak {
-  float v[2] = {0.f, 0.f};
-  __device__ __forceinline__ void add(const f32x4 (&s)[2][2]) {
+// The score scale on such sums.  It keeps its bits down to 2^-78; smaller scales
+// (and not 0) take the fp32 tiles.
+__device__ __forceinline__ float score_scale(const AttnArgs& a) { return a.scale * split::kUnscale; }
+__device__ __forceinline__ bool scale_lost(const AttnArgs& a) { return fabsf(a.scale) < 0x1p-78f && a.scale != 0.f; }
+// The finished sums: hi = (hi + lo) 2^-48.
+__device__ __forceinline__ void finish(f32x4 (&hi)[4][2], const f32x4 (&lo)[4][2]) {
 #pragma unroll
-    for (int n = 0; n < 2; ++n)
+  for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[n] = fmaxf(v[n], fabsf(s[i][n][r]));
-  }
-  __device__ __forceinline__ bool low() {
-    bool any = false;
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      v[n] = fmaxf(v[n], __shfl_xor(v[n], 16, 64));
-      v[n] = fmaxf(v[n], __shfl_xor(v[n], 32, 64));
-      any |= v[n] > 0.f && v[n] < 0x1p-80f;
-    }
-    return any;
-  }
-};
+    for (int n = 0; n < 2; ++n) hi[b][n] = (hi[b][n] + lo[b][n]) * split::kUnscale;
+}
 
 // Workgroup's slice and first column; the slices of an XCD are neighbours.
 __device__ __forceinline__ Slice column_block(const AttnArgs& a) {
@@ -1313,15 +1304,15 @@ __global__ __launch_bounds__(256, 2) void attn_stats_split_kernel(AttnArgs a) {
   const int k0 = sl.pair * CW + w * TW;
   const bool live = k0 < a.seq;
   const __amdgpu_buffer_rsrc_t Q = rsrc(a.q, a.bytes), K = rsrc(a.k, a.bytes);
-  split::Tiny tiny;
   Frag kb[2][2];
-  load_b<2>(K, sl.base, a.ld, min(k0, a.seq - TW), kb, tiny);
+  load_b<2>(K, sl.base, a.ld, min(k0, a.seq - TW), kb);
+  const float ss = score_scale(a);
   float m[2] = {-FLT_MAX, -FLT_MAX}, l[2] = {0.f, 0.f}, mark = 0.f;
   Raw raw;
   const int slot = rows_slot();
   staged_loop<kTile>(
       lds, 0, a.seq / TW, [&](int c) { load_rows(Q, sl.base, a.ld, TW * c, raw); },
-      [&](char* t) { put(t, slot, raw, tiny); },
+      [&](char* t) { put(t, slot, raw); },
       [&](int c, const char* t) {
         if (!live) return;
         f32x4 s[2][2];
@@ -1333,7 +1324,7 @@ __global__ __launch_bounds__(256, 2) void attn_stats_split_kernel(AttnArgs a) {
           float v[8], mx = m[n];
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            v[j] = a.scale * s[j >> 2][n][j & 3];
+            v[j] = ss * s[j >> 2][n][j & 3];
             mark = fmaf(0.f, v[j], mark);
             mx = fmaxf(mx, v[j]);
           }
@@ -1350,7 +1341,7 @@ __global__ __launch_bounds__(256, 2) void attn_stats_split_kernel(AttnArgs a) {
           m[n] = mx;
         }
       });
-  const bool bad = tiny.found() || (live && !(mark == 0.f));
+  const bool bad = scale_lost(a) || (live && !(mark == 0.f));
   if (__syncthreads_or(bad)) {
     if (live) stats_tile<CAUSAL>(a, sl, k0);
     return;
@@ -1383,10 +1374,10 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_split_kernel(AttnArgs a) {
   const bool live = q0 < a.seq;
   const __amdgpu_buffer_rsrc_t Q = rsrc(a.q, a.bytes), K = rsrc(a.k, a.bytes), V = rsrc(a.v, a.bytes);
   const float* ST = a.stats + (size_t)sl.z * a.seq * 2;
-  split::Tiny tiny;
-  Peak peak;
+  const float ss = score_scale(a);
+  float mark = 0.f;  // NaN once a score is not finite (minus infinity would leave a P of 0)
   Frag qb[2][2];
-  load_b<2>(Q, sl.base, a.ld, min(q0, a.seq - TW), qb, tiny);
+  load_b<2>(Q, sl.base, a.ld, min(q0, a.seq - TW), qb);
   f32x4 hi[4][2], lo[4][2];
   clear(hi, lo);
   Raw rk, rv;
@@ -1398,8 +1389,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_split_kernel(AttnArgs a) {
         load_cols(V, sl.base, a.ld, TW * c, rv);
       },
       [&](char* t) {
-        put(t, rs, rk, tiny);
-        put(t + kTile, cs, rv, tiny);
+        put(t, rs, rk);
+        put(t + kTile, cs, rv);
       },
       [&](int c, const char* t) {
         if (!live || (CAUSAL && TW * c > q0)) return;
@@ -1408,8 +1399,11 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_split_kernel(AttnArgs a) {
         for (int i = 0; i < 2; ++i)
 #pragma unroll
           for (int h = 0; h < 2; ++h) st[i][h] = ld4(ST + (size_t)(TW * c + 16 * i + 4 * q) * 2 + 4 * h);
-        f32x4 s[2][2];
+        f32x4 s[2][2], il[2];
         score<2>(t, qb, s);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)  // 2^24 / l (after the scores, which hide the loads)
+          il[i] = split::kScale * f32x4{st[i][0][1], st[i][0][3], st[i][1][1], st[i][1][3]};
         const bool masked = CAUSAL && TW * c == q0;
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -1418,18 +1412,15 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_split_kernel(AttnArgs a) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const bool keep = !masked || q0 + 16 * n + lr >= TW * c + 16 * i + 4 * q + r;
-              s[i][n][r] = keep ? __expf(a.scale * s[i][n][r] - st[i][r >> 1][2 * (r & 1)]) * st[i][r >> 1][2 * (r & 1) + 1] : 0.f;
+              mark = fmaf(0.f, s[i][n][r], mark);
+              s[i][n][r] = keep ? __expf(ss * s[i][n][r] - st[i][r >> 1][2 * (r & 1)]) * il[i][r] : 0.f;
             }
-        peak.add(s);
         Frag p[2];
         to_frag<2>(s, p);
         accumulate<2>(t + kTile, p, hi, lo);
       });
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-#pragma unroll
-    for (int n = 0; n < 2; ++n) hi[b][n] += lo[b][n];
-  const bool bad = tiny.found() || (live && (peak.low() || !(finite_mark(hi) == 0.f)));
+  finish(hi, lo);
+  const bool bad = scale_lost(a) || (live && !(mark + finite_mark(hi) == 0.f));
   if (__syncthreads_or(bad)) {
     if (live) fwd_tile<CAUSAL>(a, sl, q0);
     return;
@@ -1453,17 +1444,17 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kv_split_kernel(AttnArgs a) {
   const int k0 = sl.pair * CW + w * TW;
   const bool live = k0 < a.seq;
   const __amdgpu_buffer_rsrc_t Q = rsrc(a.q, a.bytes), K = rsrc(a.k, a.bytes), V = rsrc(a.v, a.bytes), dO = rsrc(a.dout, a.bytes);
-  split::Tiny tiny;
-  Peak peak;
+  const float ss = score_scale(a);
+  float mark = 0.f;  // NaN once a score is not finite (minus infinity would leave a P of 0)
   Frag kb[2][2];
-  load_b<2>(K, sl.base, a.ld, min(k0, a.seq - TW), kb, tiny);
+  load_b<2>(K, sl.base, a.ld, min(k0, a.seq - TW), kb);
   float m[2] = {0.f, 0.f}, il[2] = {0.f, 0.f};
   if (live) {
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
       const float2 t = *reinterpret_cast<const float2*>(a.stats + ((size_t)sl.z * a.seq + k0 + 16 * n + lr) * 2);
       m[n] = t.x;
-      il[n] = t.y;
+      il[n] = split::kScale * t.y;
     }
   }
   f32x4 hi[4][2], lo[4][2];
@@ -1477,8 +1468,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kv_split_kernel(AttnArgs a) {
         load_cols(dO, sl.base, a.ld, TW * c, ro);
       },
       [&](char* t) {
-        put(t, rs, rq, tiny);
-        put(t + kTile, cs, ro, tiny);
+        put(t, rs, rq);
+        put(t + kTile, cs, ro);
       },
       [&](int c, const char* t) {
         if (!live || (CAUSAL && TW * c < k0)) return;
@@ -1492,18 +1483,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kv_split_kernel(AttnArgs a) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const bool keep = !masked || TW * c + 16 * i + 4 * q + r >= k0 + 16 * n + lr;
-              s[i][n][r] = keep ? __expf(a.scale * s[i][n][r] - m[n]) * il[n] : 0.f;
+              mark = fmaf(0.f, s[i][n][r], mark);
+              s[i][n][r] = keep ? __expf(ss * s[i][n][r] - m[n]) * il[n] : 0.f;
             }
-        peak.add(s);
         Frag p[2];
         to_frag<2>(s, p);
         accumulate<2>(t + kTile, p, hi, lo);
       });
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-#pragma unroll
-    for (int n = 0; n < 2; ++n) hi[b][n] += lo[b][n];
-  const bool bad = tiny.found() || (live && (peak.low() || !(finite_mark(hi) == 0.f)));
+  finish(hi, lo);
+  const bool bad = scale_lost(a) || (live && !(mark + finite_mark(hi) == 0.f));
   if (__syncthreads_or(bad)) {
     if (live) bwd_kv_tile<CAUSAL, false>(a, sl, k0);
     return;
@@ -1550,11 +1538,11 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_q_split_kernel(AttnArgs a) {
   const __amdgpu_buffer_rsrc_t Q = rsrc(a.q, a.bytes), K = rsrc(a.k, a.bytes), V = rsrc(a.v, a.bytes), dO = rsrc(a.dout, a.bytes);
   const float* ST = a.stats + (size_t)sl.z * a.seq * 2;
   const float* DC = a.dcol + (size_t)sl.z * a.seq;
-  split::Tiny tiny;
-  Peak peak;
+  const float ss = score_scale(a);
+  float mark = 0.f;  // NaN once a score is not finite (minus infinity would leave a P of 0)
   Frag qb[2][2], ob[2][2];
-  load_b<2>(Q, sl.base, a.ld, min(q0, a.seq - TW), qb, tiny);
-  load_b<2>(dO, sl.base, a.ld, min(q0, a.seq - TW), ob, tiny);
+  load_b<2>(Q, sl.base, a.ld, min(q0, a.seq - TW), qb);
+  load_b<2>(dO, sl.base, a.ld, min(q0, a.seq - TW), ob);
   f32x4 hi[4][2], lo[4][2], xh[4][2], xl[4][2];
   clear(hi, lo);
   clear(xh, xl);
@@ -1569,10 +1557,10 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_q_split_kernel(AttnArgs a) {
         if (KREF) load_cols(Q, sl.base, a.ld, TW * c, cq);
       },
       [&](char* t) {
-        put(t, rs, rk, tiny);
-        put(t + kTile, rs, rv, tiny);
-        put(t + 2 * kTile, cs, ck, tiny);
-        if (KREF) put(t + 3 * kTile, cs, cq, tiny);
+        put(t, rs, rk);
+        put(t + kTile, rs, rv);
+        put(t + 2 * kTile, cs, ck);
+        if (KREF) put(t + 3 * kTile, cs, cq);
       },
       [&](int c, const char* t) {
         if (!live || (CAUSAL && TW * c > q0)) return;
@@ -1583,9 +1571,11 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_q_split_kernel(AttnArgs a) {
           for (int h = 0; h < 2; ++h) st[i][h] = ld4(ST + (size_t)(TW * c + 16 * i + 4 * q) * 2 + 4 * h);
           dc[i] = ld4(DC + TW * c + 16 * i + 4 * q);
         }
-        f32x4 s[2][2], dp[2][2];
+        f32x4 s[2][2], dp[2][2], il[2];
         score<2>(t, qb, s);
         score<2>(t + kTile, ob, dp);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) il[i] = split::kScale * f32x4{st[i][0][1], st[i][0][3], st[i][1][1], st[i][1][3]};
         const bool masked = CAUSAL && TW * c == q0;
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -1594,23 +1584,18 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_q_split_kernel(AttnArgs a) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const bool keep = !masked || q0 + 16 * n + lr >= TW * c + 16 * i + 4 * q + r;
-              const float p = __expf(a.scale * s[i][n][r] - st[i][r >> 1][2 * (r & 1)]) * st[i][r >> 1][2 * (r & 1) + 1];
-              s[i][n][r] = keep ? p * (dp[i][n][r] - dc[i][r]) : 0.f;
+              mark = fmaf(0.f, s[i][n][r], mark);
+              const float p = __expf(ss * s[i][n][r] - st[i][r >> 1][2 * (r & 1)]) * il[i][r];
+              s[i][n][r] = keep ? p * (dp[i][n][r] * split::kUnscale - dc[i][r]) : 0.f;
             }
-        peak.add(s);
         Frag f[2];
         to_frag<2>(s, f);
         accumulate<2>(t + 2 * kTile, f, hi, lo);
         if (KREF) accumulate<2>(t + 3 * kTile, f, xh, xl);
       });
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      hi[b][n] += lo[b][n];
-      xh[b][n] += xl[b][n];
-    }
-  const bool bad = tiny.found() || (live && (peak.low() || !(finite_mark(hi) + finite_mark(xh) == 0.f)));
+  finish(hi, lo);
+  if (KREF) finish(xh, xl);
+  const bool bad = scale_lost(a) || (live && !(mark + finite_mark(hi) + finite_mark(xh) == 0.f));
   if (__syncthreads_or(bad)) {
     float* own = reinterpret_cast<float*>(lds) + w * 2 * TW * LQ;
     if (live) bwd_q_tile<CAUSAL, KREF>(a, sl, q0, own, own + TW * LQ);

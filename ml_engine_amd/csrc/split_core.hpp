@@ -17,7 +17,7 @@
 // (all six in one accumulator is biased by the MFMA's truncation and loses to
 // the fp32 MFMA on one-sided operands: 9.2e-7 against 8.0e-7 at K 4096.)
 //
-// The tile engine splits 2^24 x: the last bit of any fp32 value is then at least
+// What is split is 2^24 x: the last bit of any fp32 value is then at least
 // 2^-125, so every part of every value, the smallest included, is exact and
 // normal; the sums are scaled back by 2^-48.  (Without the scale values
 // under 2^-110 lose bits.  They are ordinary: after some 60 steps a transformer
@@ -53,7 +53,6 @@ namespace split {
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int KS = 32;                      // K depth of a stage
 constexpr uint32_t kOOB = 0x80000000u;      // byte offset past every buffer: reads 0
@@ -78,20 +77,6 @@ __device__ __forceinline__ unsigned pack_bf16(float a, float b) {
 __device__ __forceinline__ float low_f(unsigned h) { return __builtin_bit_cast(float, h << 16); }
 __device__ __forceinline__ float high_f(unsigned h) { return __builtin_bit_cast(float, h & 0xffff0000u); }
 
-// For splits without the scale: smallest (bits << 1) - 1 of the nonzero leading
-// parts seen (zero wraps to the largest value).
-struct Tiny {
-  u16x2 m = {0xffff, 0xffff};
-  __device__ __forceinline__ void see(unsigned h) {
-    const u16x2 t = __builtin_bit_cast(u16x2, h) * (unsigned short)2 + (unsigned short)0xffff;
-    m = __builtin_elementwise_min(m, t);
-  }
-  __device__ __forceinline__ bool found() const {
-    constexpr unsigned short kLimit = 17u << 8;  // exponent field 17: 2^-110
-    return m[0] < kLimit || m[1] < kLimit;
-  }
-};
-
 constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f;  // of an operand, of a sum of products
 
 // Eight fp32 values to their three bf16 parts.
@@ -107,13 +92,6 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4& p0, u32x4& p1
     p2[j] = pack_bf16(ra - low_f(m), rb - high_f(m));
   }
 }
-// Noting values too small for it.
-__device__ __forceinline__ void split8(const float (&x)[8], u32x4& p0, u32x4& p1, u32x4& p2, Tiny& tiny) {
-  split8(x, p0, p1, p2);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) tiny.see(p0[j]);
-}
-
 __device__ __forceinline__ f32x4 mma(const u32x4& a, const u32x4& b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }

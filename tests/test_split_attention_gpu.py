@@ -100,3 +100,21 @@ def test_split_attention_special_values(hip, causal):
         tol = 1e-4 if j == 2 else 1e-5
         for name, g, w, m in zip(("out", "dq", "dk", "dv"), got, want, mag):
             assert np.all(np.abs(g[0, :, c] - w) <= tol * m + 2.0 ** -140), (j, name)
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+@pytest.mark.parametrize("exp", [-112, -125, -136])
+def test_split_attention_small_operands(hip, causal, exp):
+    """V and dO near and below the end of the normal range: the outputs that are
+    linear in them keep every bit that fp32 products give (steps of 2^-149)."""
+    s, h = 320, 2
+    r = rng(5 - exp + causal)
+    q, k, v, do = (r.standard_normal((1, s, h * HD), dtype=np.float32) for _ in range(4))
+    v[0, :, :HD] *= np.float32(2.0 ** exp)   # head 0: all of V
+    do[0, :, HD:] *= np.float32(2.0 ** exp)  # head 1: all of dO
+    out, _, _, dv = run(hip, q, k, v, do, 1, h, s, h * HD, 0.125, causal, 1)
+    for j, i in ((0, 0), (1, 3)):
+        c = slice(j * HD, (j + 1) * HD)
+        want, mag = reference(q[0, :, c], k[0, :, c], v[0, :, c], do[0, :, c], 0.125, causal, 1)
+        got = (out if i == 0 else dv)[0, :, c]
+        assert np.all(np.abs(got - want[i]) <= 1e-5 * mag[i] + 2.0 ** -148)
