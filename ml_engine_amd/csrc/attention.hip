@@ -1264,11 +1264,30 @@ __device__ __forceinline__ void finish(f32x4 (&hi)[4][2], const f32x4 (&lo)[4][2
     for (int n = 0; n < 2; ++n) hi[b][n] = (hi[b][n] + lo[b][n]) * split::kUnscale;
 }
 
-// Workgroup's slice and first column; the slices of an XCD are neighbours.
+// Workgroup's slice and column block; the slices of an XCD are neighbours.
+// BY_BLOCK: an XCD's workgroups run block 0 of every slice first, then block 1
+// and so on.  The causal passes give block 0 the most work: slice after slice,
+// the last slices' longest blocks would begin when the chip is nearly done.
+// (Backward, causal, 96 heads of 512 / 115 of 384 / 256 of 1024, us: 184 / 128
+// / 1163 slice after slice, 117 / 95 / 859 so; paired fp32 tiles took 122 / 108 / 1111.)
+template <bool BY_BLOCK>
 __device__ __forceinline__ Slice column_block(const AttnArgs& a) {
   const int L = blockIdx.x, total = gridDim.x, blocks = (a.seq + CW - 1) / CW;
-  const int x = L % kXcds, j = L / kXcds, per = total / kXcds, rem = total % kXcds;
-  const int t = x * per + min(x, rem) + j;
+  const int x = L % kXcds, per = total / kXcds, rem = total % kXcds;
+  const int begin = x * per + min(x, rem), end = begin + per + (x < rem);  // this XCD's items, slice-major
+  int t = begin + L / kXcds;
+  if (BY_BLOCK) {
+    int j = L / kXcds;
+    for (int p = 0; p < blocks; ++p) {
+      const int first = begin + (p + blocks - begin % blocks) % blocks;  // the first item of block p
+      const int n = first < end ? (end - 1 - first) / blocks + 1 : 0;
+      if (j < n) {
+        t = first + j * blocks;
+        break;
+      }
+      j -= n;
+    }
+  }
   const int z = t / blocks, b = z / a.heads, h = z - b * a.heads;
   return {z, (uint32_t)b * a.seq * a.ld + (uint32_t)h * HD, t - z * blocks};
 }
@@ -1299,7 +1318,7 @@ __device__ __forceinline__ void staged_loop(char* lds, int c0, int c1, Fetch fet
 template <bool CAUSAL>
 __global__ __launch_bounds__(256, 2) void attn_stats_split_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) char lds[2 * kTile];
-  const Slice sl = column_block(a);
+  const Slice sl = column_block<false>(a);
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
   const int k0 = sl.pair * CW + w * TW;
   const bool live = k0 < a.seq;
@@ -1366,7 +1385,7 @@ __global__ __launch_bounds__(256, 2) void attn_stats_split_kernel(AttnArgs a) {
 template <bool CAUSAL>
 __global__ __launch_bounds__(256, 2) void attn_fwd_split_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) char lds[4 * kTile];
-  const Slice sl = column_block(a);
+  const Slice sl = column_block<CAUSAL>(a);
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
   // heaviest blocks first under the mask
   const int blk = CAUSAL ? (a.seq + CW - 1) / CW - 1 - sl.pair : sl.pair;
@@ -1439,7 +1458,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_split_kernel(AttnArgs a) {
 template <bool CAUSAL>
 __global__ __launch_bounds__(256, 2) void attn_bwd_kv_split_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) char lds[4 * kTile];
-  const Slice sl = column_block(a);
+  const Slice sl = column_block<CAUSAL>(a);
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
   const int k0 = sl.pair * CW + w * TW;
   const bool live = k0 < a.seq;
@@ -1530,7 +1549,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_q_split_kernel(AttnArgs a) {
   constexpr int NT = KREF ? 4 : 3;
   constexpr int kLds = 2 * NT * kTile > 8 * TW * LQ * 4 ? 2 * NT * kTile : 8 * TW * LQ * 4;
   __shared__ __attribute__((aligned(16))) char lds[kLds];
-  const Slice sl = column_block(a);
+  const Slice sl = column_block<CAUSAL>(a);
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
   const int blk = CAUSAL ? (a.seq + CW - 1) / CW - 1 - sl.pair : sl.pair;
   const int q0 = blk * CW + w * TW;

@@ -118,3 +118,18 @@ def test_split_attention_small_operands(hip, causal, exp):
         want, mag = reference(q[0, :, c], k[0, :, c], v[0, :, c], do[0, :, c], 0.125, causal, 1)
         got = (out if i == 0 else dv)[0, :, c]
         assert np.all(np.abs(got - want[i]) <= 1e-5 * mag[i] + 2.0 ** -148)
+
+
+# the causal passes hand out blocks of one kind after another on each XCD: grids
+# of no multiple of 8, XCDs that share a slice, fewer blocks than XCDs
+@pytest.mark.parametrize("b,h,s,kref", [(3, 23, 320, 1), (1, 13, 576, 1), (1, 3, 384, 1), (5, 7, 448, 0)])
+def test_causal_block_order(hip, b, h, s, kref):
+    r = rng(b * h + s)
+    q, k, v, do = (r.standard_normal((b, s, h * HD), dtype=np.float32) for _ in range(4))
+    got = run(hip, q, k, v, do, b, h, s, h * HD, 0.125, 1, kref)
+    for i in range(b):
+        for j in range(h):
+            c = slice(j * HD, (j + 1) * HD)
+            want, mag = reference(q[i, :, c], k[i, :, c], v[i, :, c], do[i, :, c], 0.125, 1, kref)
+            for name, g, w, m in zip(("out", "dq", "dk", "dv"), got, want, mag):
+                assert np.all(np.abs(g[i, :, c] - w) <= 1e-5 * m + 1e-30), (name, i, j)
