@@ -22,8 +22,9 @@
 //
 //   statistics (key blocks)   : m_c, 1 / l_c
 //   forward    (query blocks) : O = P V
-//   bwd kv     (key blocks)   : dV, D (and dK = scale dS^T Q)
-//   bwd q      (query blocks) : dQ = scale dS K (or the reference's dK)
+//   bwd kv     (key blocks)   : dV, D
+//   bwd k      (key blocks)   : dK = scale dS^T Q (or, with dQ, the reference's)
+//   bwd q      (query blocks) : dQ = scale dS K (and the reference's dK)
 //
 // Up to 256 positions a workgroup runs a whole slice on the fp32 matrix cores;
 // past that, and without the mask past 128 (split_fwd, split_bwd), the passes
@@ -106,41 +107,26 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
 struct Slice {
   int z;
   uint32_t base;  // element offset of (batch item, head) in the [batch][seq][ld] tensors
-  int pair;       // this workgroup's tile pair within the slice
+  int pair;       // this workgroup's column block within the slice
 };
 // Slice z's kept probabilities, kept_blocks(seq) blocks of 256 floats.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t kept_rsrc(const AttnArgs& a, const Slice& sl) {
   const size_t n = kept_blocks(a.seq) * 256;
   return rsrc(a.kept + (size_t)sl.z * n, (uint32_t)(n * sizeof(float)));
 }
-// The grid is one-dimensional: workgroup L runs on XCD L % 8 (workgroups are
+// The grids are one-dimensional: workgroup L runs on XCD L % 8 (workgroups are
 // dispatched round-robin over the XCDs).  XCD x takes a contiguous range of
-// the (slice, tile pair) items, slice-major, so every workgroup of a slice
-// runs on one XCD and shares its L2 copy of the slice's Q, K, V and dO rows.
-// A bijection on [0, gridDim.x) for any grid size.
+// the (slice, column block) items, slice-major, so the workgroups of a slice
+// run on one XCD and share its L2 copy of the slice's Q, K, V and dO rows.
 constexpr int kXcds = 8;
-__device__ __forceinline__ Slice slice_of(const AttnArgs& a) {
-  const int L = blockIdx.x, total = gridDim.x, pairs = a.seq / 64;
-  const int x = L % kXcds, j = L / kXcds, per = total / kXcds, rem = total % kXcds;
-  const int t = x * per + min(x, rem) + j;
-  const int z = t / pairs, b = z / a.heads, h = z - b * a.heads;
-  return {z, (uint32_t)b * a.seq * a.ld + (uint32_t)h * HD, t - z * pairs};
-}
 
-// Work split: every wave owns a 32-row tile of one output (32 keys of the
-// statistics, 32 queries of O or dQ, 32 keys of dV / dK) and walks the whole
-// contraction range for it, so no partial sums cross waves.  A workgroup is
-// two waves of the same (batch item, head) slice taking tiles j and
-// nb - 1 - j (nb = seq / 32): under the causal mask a query tile's work grows
-// with j and a key tile's shrinks, so each workgroup gets the same total.  A
-// loop over 16-row chunks keeps two register sets of chunk operands and
-// fetches chunk c + 1 into one while chunk c computes from the other.
+// The fp32 tile functions: a wave owns a 32-row tile of one output (32 keys of
+// the statistics, 32 queries of O or dQ, 32 keys of dV / dK) and walks the whole
+// contraction range for it, so no partial sums cross waves.  A loop over 16-row
+// chunks keeps two register sets of chunk operands and fetches chunk c + 1 into
+// one while chunk c computes from the other.
 constexpr int TW = 32;      // rows of a wave's tile
 constexpr int LQ = HD + 4;  // padded LDS row: the 16 rows a b128 read touches sit on distinct banks
-
-__device__ __forceinline__ int tile_of(const AttnArgs& a, const Slice& sl, int w) {
-  return w == 0 ? sl.pair : a.seq / TW - 1 - sl.pair;
-}
 
 // Chunk loop with two alternating register sets (no copies between them,
 // so a chunk's loads are waited for only when that chunk is computed).  The
@@ -428,7 +414,8 @@ __device__ __forceinline__ void fwd_tile(const AttnArgs& a, const Slice& sl, int
 // KEEP_P (causal): pass 1's P blocks on or below the diagonal (16-row query
 // block qb >= key block kb) are also written to sst, 1 KB per block at index
 // qb (qb + 1) / 2 + kb, row = query and column = key within the block.
-template <bool CAUSAL, bool DK, bool KEEP_P = false>
+// DV false: dV and D are there already.
+template <bool CAUSAL, bool DK, bool KEEP_P = false, bool DV = true>
 __device__ __forceinline__ void bwd_kv_tile(const AttnArgs& a, const Slice& sl, int k0, float* sst = nullptr) {
   const int lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
   const __amdgpu_buffer_rsrc_t Q = rsrc(a.q, a.bytes);
@@ -512,11 +499,15 @@ __device__ __forceinline__ void bwd_kv_tile(const AttnArgs& a, const Slice& sl, 
     };
     chunk_loop<Chunk>(CAUSAL ? k0 / 16 : 0, a.seq / 16, fetch, compute);
   };
-  run(std::false_type{});
+  if (DV) run(std::false_type{});
   // acc[i][n][r] = dV[k0 + 16n + lr][16q + 4r + i]
   const __amdgpu_buffer_rsrc_t dVr = rsrc(a.dv, a.bytes);
 #pragma unroll
   for (int n = 0; n < 2; ++n) {
+    if (!DV) {
+      D[n] = a.dcol[(size_t)sl.z * a.seq + k0 + 16 * n + lr];
+      continue;
+    }
     const uint32_t row = sl.base + (uint32_t)(k0 + 16 * n + lr) * a.ld;
     float part = 0.f;
 #pragma unroll
@@ -1086,13 +1077,6 @@ __device__ __forceinline__ void bwd_q_kept(const AttnArgs& a, const Slice& sl, i
   }
 }
 
-// One wave per 32-row tile, two tiles (j and nb - 1 - j) per workgroup,
-// workgroups spread over the XCDs by slice (slice_of).
-template <bool CAUSAL>
-__global__ __launch_bounds__(128, 2) void attn_bwd_kv_kernel(AttnArgs a) {
-  const Slice sl = slice_of(a);
-  bwd_kv_tile<CAUSAL, true>(a, sl, tile_of(a, sl, threadIdx.x >> 6) * TW);
-}
 // ---------------------------------------------------------------------------
 // The passes on the bf16 matrix cores (split_core.hpp: exact three-way splits,
 // six bf16 MFMAs per product, fp32 accuracy), a kernel per pass.  A workgroup
@@ -1540,6 +1524,94 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kv_split_kernel(AttnArgs a) {
   }
 }
 
+// The mathematical K gradient of 128 keys, after their dV and D: S = Q K^T,
+// dP = dO V^T, dS = P (dP - D), dK^T += Q^T dS per 32 queries.
+template <bool CAUSAL>
+__global__ __launch_bounds__(256, 1) void attn_bwd_k_split_kernel(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[6 * kTile];
+  const Slice sl = column_block<CAUSAL>(a);
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, q = lane >> 4;
+  const int k0 = sl.pair * CW + w * TW;
+  const bool live = k0 < a.seq;
+  const __amdgpu_buffer_rsrc_t Q = rsrc(a.q, a.bytes), K = rsrc(a.k, a.bytes), V = rsrc(a.v, a.bytes), dO = rsrc(a.dout, a.bytes);
+  const float ss = score_scale(a);
+  float mark = 0.f;
+  Frag kb[2][2], vb[2][2];
+  load_b<2>(K, sl.base, a.ld, min(k0, a.seq - TW), kb);
+  load_b<2>(V, sl.base, a.ld, min(k0, a.seq - TW), vb);
+  float m[2] = {0.f, 0.f}, il[2] = {0.f, 0.f}, D[2] = {0.f, 0.f};
+  if (live) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const size_t key = (size_t)sl.z * a.seq + k0 + 16 * n + lr;
+      const float2 t = *reinterpret_cast<const float2*>(a.stats + key * 2);
+      m[n] = t.x;
+      il[n] = split::kScale * t.y;
+      D[n] = a.dcol[key];
+    }
+  }
+  f32x4 hi[4][2], lo[4][2];
+  clear(hi, lo);
+  Raw rq, ro, cq;
+  const int rs = rows_slot(), cs = cols_slot();
+  staged_loop<3 * kTile>(
+      lds, CAUSAL ? sl.pair * CW / TW : 0, a.seq / TW,
+      [&](int c) {
+        load_rows(Q, sl.base, a.ld, TW * c, rq);
+        load_rows(dO, sl.base, a.ld, TW * c, ro);
+        load_cols(Q, sl.base, a.ld, TW * c, cq);
+      },
+      [&](char* t) {
+        put(t, rs, rq);
+        put(t + kTile, rs, ro);
+        put(t + 2 * kTile, cs, cq);
+      },
+      [&](int c, const char* t) {
+        if (!live || (CAUSAL && TW * c < k0)) return;
+        f32x4 s[2][2], dp[2][2];
+        score<2>(t, kb, s);
+        score<2>(t + kTile, vb, dp);
+        const bool masked = CAUSAL && TW * c == k0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const bool keep = !masked || TW * c + 16 * i + 4 * q + r >= k0 + 16 * n + lr;
+              mark = fmaf(0.f, s[i][n][r], mark);
+              const float p = __expf(ss * s[i][n][r] - m[n]) * il[n];
+              s[i][n][r] = keep ? p * (dp[i][n][r] * split::kUnscale - D[n]) : 0.f;
+            }
+        Frag f[2];
+        to_frag<2>(s, f);
+        accumulate<2>(t + 2 * kTile, f, hi, lo);
+      });
+  finish(hi, lo);
+  const bool bad = scale_lost(a) || (live && !(mark + finite_mark(hi) == 0.f));
+  if (__syncthreads_or(bad)) {
+    if (live) bwd_kv_tile<CAUSAL, true, false, false>(a, sl, k0);
+    return;
+  }
+  if (!live) return;
+  const __amdgpu_buffer_rsrc_t dKr = rsrc(a.dk, a.bytes);
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    const uint32_t row = sl.base + (uint32_t)(k0 + 16 * n + lr) * a.ld;
+    f32x4 old[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      old[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (a.acc_k) old[r] = bld4(dKr, row + 16 * q + 4 * r);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const f32x4 g = a.scale * f32x4{hi[0][n][r], hi[1][n][r], hi[2][n][r], hi[3][n][r]};
+      bst4(dKr, row + 16 * q + 4 * r, a.acc_k ? g + old[r] : g);
+    }
+  }
+}
+
 // dQ (and with KREF the reference's K gradient) of 128 queries: S^T = K Q^T,
 // dP^T = V dO^T, dS^T = P^T (dP^T - D), then dQ^T += K^T dS^T and X^T += Q^T
 // dS^T (Q's rows at the key positions) per 32 keys.  Twice the accumulators
@@ -1832,7 +1904,6 @@ int mle_attention_bwd(mle_stream stream, const float* q, const float* k, const f
   a.acc_k = acc_k != 0;
   a.acc_v = acc_v != 0;
   hipStream_t s = as_stream(stream);
-  const dim3 grid((unsigned)(seq / (2 * TW) * batch * heads));  // two 32-row tiles per workgroup
   const dim3 blocks((unsigned)((seq + CW - 1) / CW * batch * heads));
   const double flop = 8.0 * batch * heads * (double)seq * seq * HD;  // dP, dV, dQ, dK
   ProbeScope probe("attn_bwd", s, flop, 0.0);
@@ -1850,8 +1921,9 @@ int mle_attention_bwd(mle_stream stream, const float* q, const float* k, const f
     if (kref) {
       mle::launch(attn_bwd_kv_split_kernel<true>, blocks, 256, 0, s, a);
       mle::launch(attn_bwd_q_split_kernel<true, true>, blocks, 256, 0, s, a);
-    } else {  // dK needs a second pass over the finished D: the fp32 kernel
-      mle::launch(attn_bwd_kv_kernel<true>, grid, 128, 0, s, a);
+    } else {  // dK needs the finished D
+      mle::launch(attn_bwd_kv_split_kernel<true>, blocks, 256, 0, s, a);
+      mle::launch(attn_bwd_k_split_kernel<true>, blocks, 256, 0, s, a);
       mle::launch(attn_bwd_q_split_kernel<true, false>, blocks, 256, 0, s, a);
     }
   } else {
@@ -1859,7 +1931,8 @@ int mle_attention_bwd(mle_stream stream, const float* q, const float* k, const f
       mle::launch(attn_bwd_kv_split_kernel<false>, blocks, 256, 0, s, a);
       mle::launch(attn_bwd_q_split_kernel<false, true>, blocks, 256, 0, s, a);
     } else {
-      mle::launch(attn_bwd_kv_kernel<false>, grid, 128, 0, s, a);
+      mle::launch(attn_bwd_kv_split_kernel<false>, blocks, 256, 0, s, a);
+      mle::launch(attn_bwd_k_split_kernel<false>, blocks, 256, 0, s, a);
       mle::launch(attn_bwd_q_split_kernel<false, false>, blocks, 256, 0, s, a);
     }
   }

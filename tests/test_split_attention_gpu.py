@@ -133,3 +133,24 @@ def test_causal_block_order(hip, b, h, s, kref):
             want, mag = reference(q[i, :, c], k[i, :, c], v[i, :, c], do[i, :, c], 0.125, 1, kref)
             for name, g, w, m in zip(("out", "dq", "dk", "dv"), got, want, mag):
                 assert np.all(np.abs(g[i, :, c] - w) <= 1e-5 * m + 1e-30), (name, i, j)
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+def test_mathematical_k_gradient_error(hip, causal):
+    """dK = scale dS^T Q and dQ = scale dS K sum the same dS over the same number
+    of positions, so their relative errors (2-norm) are of one size.  Scores of
+    two different products in one column (statistics of one, probabilities of
+    the other) would show here: dK's error was 2.4 times dQ's."""
+    s, h = 512, 4
+    r = rng(31 + causal)
+    q, k, v, do = (r.standard_normal((1, s, h * HD), dtype=np.float32) for _ in range(4))
+    _, dq, dk, _ = run(hip, q, k, v, do, 1, h, s, h * HD, 0.125, causal, 0)
+    err, ref = np.zeros(2), np.zeros(2)
+    for j in range(h):
+        c = slice(j * HD, (j + 1) * HD)
+        want, _ = reference(q[0, :, c], k[0, :, c], v[0, :, c], do[0, :, c], 0.125, causal, 0)
+        for n, (g, w) in enumerate(((dq, want[1]), (dk, want[2]))):
+            err[n] += np.square(g[0, :, c] - w).sum()
+            ref[n] += np.square(w).sum()
+    rel = np.sqrt(err / ref)
+    assert rel[1] <= 1.5 * rel[0], rel
