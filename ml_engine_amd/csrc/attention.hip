@@ -27,7 +27,7 @@
 //   bwd q      (query blocks) : dQ = scale dS K (and the reference's dK)
 //
 // Up to 256 positions a workgroup runs a whole slice on the fp32 matrix cores;
-// past that, and without the mask past 128 (split_fwd, split_bwd), the passes
+// past that, and without the mask past 128 (split_passes), the passes
 // are kernels of their own on the bf16 matrix cores, and the fp32 tile
 // functions are what they fall back to.
 //
@@ -1732,7 +1732,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_q_split_kernel(AttnArgs a) {
   }
 }
 
-// Whole-slice kernels (seq <= 256, see split_fwd): workgroup z runs every tile of slice z
+// Whole-slice kernels (seq <= 256, see split_passes): workgroup z runs every tile of slice z
 // with one wave per tile (SW waves), the two passes of the forward (or the
 // backward) separated by a workgroup barrier instead of a kernel boundary.
 // Each kernel launch pays a ramp (every wave waits for its first operands
@@ -1792,24 +1792,19 @@ __global__ __launch_bounds__(SW * 64, 1) void attn_bwd_slice_kernel(AttnArgs a) 
   }
 }
 
-// Which kernels a call takes: the split passes (seq > 256) or the whole-slice
-// kernels.  The causal slice kernels keep scores and probabilities between
-// their passes and stay ahead up to 256 positions (32 x 8 heads of 256, forward
-// / backward us: 44 / 56 against 52 / 112).  Without the mask they recompute, and
-// past 128 positions the split forward is ahead at every batch (256 positions, 1
-// / 256 / 512 slices: 32 / 53 / 95 against 60 / 68 / 128 us; 192: 26 / 42 / 73
-// against 45 / 50 / 95; 128: 20 / 25 / 35 against 20 / 25 / 45, left where it
-// was).  The split backward halves the time while its workgroups, two a slice,
-// find a CU each (256 positions, 64 slices: 57 against 105 us); with more slices
-// it is ahead with whole column blocks and the reference's K gradient (256
-// positions, 256 / 512 slices: 111 / 212 against 114 / 224) and not otherwise
-// (192 positions: 86 against 84; the mathematical K gradient, whose kernel is
-// fp32, at 256: 150 against 145).  Both read and write the same statistics.
-bool split_fwd(int seq, bool causal) { return seq > SW * TW || (!causal && seq > CW); }
-bool split_bwd(int seq, long long slices, bool causal, bool kref) {
-  if (seq > SW * TW) return true;
-  return !causal && seq > CW && (2 * slices <= 256 || (kref && seq % CW == 0));
-}
+// Which kernels a call takes: the split passes or the whole-slice kernels.  The
+// causal slice kernels keep scores and probabilities between their passes and
+// stay ahead up to 256 positions (32 x 8 heads of 256, forward / backward us:
+// 44 / 56 against 52 / 112).  Without the mask they recompute, and past 128
+// positions the split passes are ahead (256 positions, 64 / 256 / 512 heads:
+// forward 32 / 50 / 92 against 62 / 65 / 127 us, backward 58 / 110 / 210 against
+// 105 / 116 / 225; 192: 26 / 39 / 70 against 47 / 48 / 95 and 48 / 87 / 166
+// against 79 / 85 / 165; 128 forward: 20 / 25 / 35 against 20 / 25 / 45, left
+// where it was).  One rule for both directions: a column's probabilities have to
+// come from the scores that its statistics came from.  (The mathematical K
+// gradient has a pass of its own: 192 positions, 256 heads, backward 122
+// against 105 us on the slice kernels, where dK lost 4 % in accuracy.)
+bool split_passes(int seq, bool causal) { return seq > SW * TW || (!causal && seq > CW); }
 
 // Operand addressing uses 32-bit byte offsets into buffer resources whose
 // extent is the tensor's byte size (AttnArgs::bytes), so every tensor must stay
@@ -1859,7 +1854,7 @@ int mle_attention_fwd(mle_stream stream, const float* q, const float* k, const f
   const dim3 blocks((unsigned)((seq + CW - 1) / CW * batch * heads));
   const double flop = 4.0 * batch * heads * (double)seq * seq * HD;  // S and P V, as the reference computes them
   ProbeScope probe("attn_fwd", s, flop, 0.0);
-  if (!split_fwd(seq, causal != 0)) {
+  if (!split_passes(seq, causal != 0)) {
     const dim3 slices((unsigned)(batch * heads));
     if (causal) mle::launch(attn_fwd_slice_kernel<true>, slices, SW * 64, 0, s, a);
     else mle::launch(attn_fwd_slice_kernel<false>, slices, SW * 64, 0, s, a);
@@ -1908,7 +1903,7 @@ int mle_attention_bwd(mle_stream stream, const float* q, const float* k, const f
   const double flop = 8.0 * batch * heads * (double)seq * seq * HD;  // dP, dV, dQ, dK
   ProbeScope probe("attn_bwd", s, flop, 0.0);
   const bool kref = k_reference_grad != 0;
-  if (!split_bwd(seq, (long long)batch * heads, causal != 0, kref)) {
+  if (!split_passes(seq, causal != 0)) {
     const dim3 slices((unsigned)(batch * heads));
     if (causal) {
       if (kref) mle::launch(attn_bwd_slice_kernel<true, true>, slices, SW * 64, 0, s, a);

@@ -51,8 +51,7 @@ def run(hip, q, k, v, do, b, h, s, ld, scale, causal, kref):
 
 
 # whole and half column blocks (128), several heads and batch items, a wider ld;
-# unmasked up to 256 positions: both directions split (up to 128 slices, or
-# whole blocks), the forward alone (more slices), neither (128 positions)
+# unmasked up to 256 positions: split past 128 positions, few slices and many
 @pytest.mark.parametrize("b,h,s,extra,causal,kref", [
     (2, 3, 320, 0, 1, 1), (1, 2, 448, 64, 0, 1), (2, 1, 512, 0, 1, 0), (1, 9, 576, 0, 0, 0), (1, 1, 1088, 128, 1, 1),
     (1, 2, 192, 64, 0, 1), (1, 2, 256, 0, 0, 0), (2, 64, 192, 0, 0, 1), (3, 43, 192, 0, 0, 1), (3, 43, 192, 0, 0, 0),
