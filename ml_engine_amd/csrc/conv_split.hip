@@ -13,7 +13,7 @@
 // (Channel and tap of each k by scalar multiplications in the loop: 61 against
 // 48 us for the forward of 32 x 128 -> 192 channels on 14 x 14.)
 // wgrad: the same table over the workgroup's pixels (source offset, tap bits,
-// dY offset).
+// dY offset), CHUNK of them at a time.
 #include "conv_args.hpp"
 #include "gemm_tiles.hpp"
 #include "split_core.hpp"
@@ -308,13 +308,14 @@ struct WgradArgs {
   ConvGeom g;
 };
 
-// The workgroup's pixels: source offset (bytes) of the pixel's corner, tap
-// bits, and dY offset (bytes, channel 0).  PAD more entries read as outside.
+// Up to CHUNK of the workgroup's pixels: source offset (bytes) of the pixel's
+// corner, tap bits, and dY offset (bytes, channel 0).  PAD more entries read as
+// outside.
 template <int CHUNK>
 struct PixTable {
   static constexpr int kPad = 5 * KS, kN = CHUNK + kPad;
-  uint32_t src[kN], dy[kN];
-  unsigned bits[kN];
+  static_assert(CHUNK % KS == 0, "whole stages");
+  uint32_t src[kN], dy[kN], bits[kN];
   __device__ __forceinline__ void fill(const WgradArgs& a, int kbeg, int klen, int t, int nth) {
     const ConvGeom& g = a.g;
     const int ohw = g.oh * g.ow, n = (klen + KS - 1) / KS * KS + 4 * KS;
@@ -349,12 +350,10 @@ struct RowLoad : Chunks<R * 4 / NTH, SUM> {
   const uint32_t* tab;
   uint32_t off[NC], e[8];
   int k, left;  // the stages left are this K group's: past them the rows read as 0 (the sums count every stage put)
-  __device__ __forceinline__ void init(const float* src, uint32_t bytes, int rows, int hw, const uint32_t* table, int k0,
-                                       int stages, int r0, int t) {
+  __device__ __forceinline__ void init(const float* src, uint32_t bytes, int rows, int hw, const uint32_t* table, int r0,
+                                       int t) {
     rs = rsrc(src, bytes);
     tab = table;
-    k = k0 + 4 * (t & 3);
-    left = stages;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       int r, q;
@@ -362,6 +361,11 @@ struct RowLoad : Chunks<R * 4 / NTH, SUM> {
       this->place(c, r, q);
       off[c] = r0 + r < rows ? (uint32_t)((r0 + r) * hw) * 4u : kOOB;
     }
+  }
+  // Start at pixel k0 of the table.
+  __device__ __forceinline__ void seek(int k0, int stages, int t) {
+    k = k0 + 4 * (t & 3);
+    left = stages;
   }
   __device__ __forceinline__ void pre() {
 #pragma unroll
@@ -396,13 +400,12 @@ struct XLoad : Chunks<R * 4 / NTH, false> {
   __amdgpu_buffer_rsrc_t rs;
   const T* tab;
   uint32_t off[NC], e[8];
-  unsigned bit[NC], m[8];
+  uint32_t bit[NC], m[8];
   int k;
-  __device__ __forceinline__ void init(const WgradArgs& a, const T* table, int k0, int n0, int t) {
+  __device__ __forceinline__ void init(const WgradArgs& a, const T* table, int n0, int t) {
     const ConvGeom& g = a.g;
     rs = rsrc(a.x, a.x_bytes);
     tab = table;
-    k = k0 + 4 * (t & 3);
     const int khw = g.kh * g.kw;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -414,6 +417,7 @@ struct XLoad : Chunks<R * 4 / NTH, false> {
       bit[c] = n < a.N ? 1u << tap : 0u;
     }
   }
+  __device__ __forceinline__ void seek(int k0, int, int t) { k = k0 + 4 * (t & 3); }
   __device__ __forceinline__ void pre() {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -441,25 +445,37 @@ __global__ __launch_bounds__(S::NTH * S::KG, 2) void wgrad_split_kernel(WgradArg
   gemm::item_tile(blockIdx.x, items, gx, gy, tm, tn, z);
   const int m0 = tm * S::TM, n0 = tn * S::TN, tid = threadIdx.x;
   const int kbeg = z * a.chunk, klen = min(a.K - kbeg, a.chunk);
-  tab.fill(a, kbeg, klen, tid, S::NTH * S::KG);
-  __syncthreads();
   f32x4 v[BI][BN], lo[BI][BN];
   {
     using LA = RowLoad<S::TM, S::NTH, V4, true>;
     LA la;
-    // With two K groups each takes half of the stages.
     const int group = k_group<S>(), t = tid % S::NTH;
-    const int nk = ((klen + KS - 1) / KS + S::KG - 1) / S::KG, k0 = group * nk * KS;
-    la.init(a.dy, a.dy_bytes, a.M, a.g.oh * a.g.ow, tab.dy, k0, nk, m0, t);
+    la.init(a.dy, a.dy_bytes, a.M, a.g.oh * a.g.ow, tab.dy, m0, t);
+    clear_sums<S>(v, lo);
+    auto chunks = [&](auto& lb) {
+#pragma unroll 1
+      for (int c0 = 0; c0 < klen; c0 += CHUNK) {
+        const int n = min(klen - c0, CHUNK);
+        if (c0 > 0) __syncthreads();  // the table and the stage buffers have been read
+        tab.fill(a, kbeg + c0, n, tid, S::NTH * S::KG);
+        __syncthreads();
+        // With two K groups each takes half of the stages.
+        const int nk = ((n + KS - 1) / KS + S::KG - 1) / S::KG, k0 = group * nk * KS;
+        la.seek(k0, nk, t);
+        lb.seek(k0, nk, t);
+        mma_stages<S>(lds + group * S::LDS, la, lb, nk, v, lo);
+      }
+    };
     if constexpr (ONE) {
       RowLoad<S::TN, S::NTH, V4, false> lb;
-      lb.init(a.x, a.x_bytes, a.N, a.g.h * a.g.w, tab.src, k0, nk, n0, t);
-      mma_loop<S>(lds + group * S::LDS, la, lb, nk, v, lo);
+      lb.init(a.x, a.x_bytes, a.N, a.g.h * a.g.w, tab.src, n0, t);
+      chunks(lb);
     } else {
       XLoad<S::TN, S::NTH, T> lb;
-      lb.init(a, &tab, k0, n0, t);
-      mma_loop<S>(lds + group * S::LDS, la, lb, nk, v, lo);
+      lb.init(a, &tab, n0, t);
+      chunks(lb);
     }
+    unscale_sums<S>(v, lo);
     if (a.db && tn == 0) {  // the lane groups' sums of each dY row, added in order
       float* red = reinterpret_cast<float*>(lds);
       __syncthreads();
@@ -565,29 +581,36 @@ void launch_gather_tile(hipStream_t s, const GatherArgs& a) {
   }
 }
 
-constexpr int kWgradChunk[2] = {3072, 768};  // pixels per workgroup at most: the table's LDS beside the tile's
+// Pixels of the table: what fits beside the tile's buffers in 160 KB (medium, one
+// workgroup per CU, and the paired small tile) or in half of it (small, two per CU).
+constexpr int kWgradChunk[2] = {3072, 2304};
 
 struct WgradPlan {
   int tile = 0, splits = 1, chunk = 0;
 };
 
 // Tile (medium or small) and pixel splits: the cheapest by the model, the
-// reduce of the partial gradients included.
+// reduce of the partial gradients and three stages per fill of the table included.
+// A stage with x gathered takes 1.6 / 0.64 us where the GEMM's takes 1.4 / 0.53
+// (16 x 128 -> 128 and 128 -> 32 on 64 x 64, one round).  The table does not bound
+// the splits, so the workspace does not grow with the pixels: four copies of dW
+// or what fills the chip (1024 -> 1024 on 32 x 32, batch 32: 151 MB for 3.7 ms,
+// where one split takes 4.8; 256 -> 256 on 128 x 128, batch 16: 17 MB).
 WgradPlan wgrad_plan(const ConvGeom& g) {
   const int M = g.cout, N = g.cin * g.kh * g.kw, K = g.n * g.oh * g.ow;
   const int st = (K + KS - 1) / KS;
   WgradPlan best;
   double best_us = 1e30;
   for (int i = 0; i < 2; ++i) {
-    const int tile = i == 0 ? gemm::kSplitMedium : gemm::kSplitSmall;
+    const int tile = i == 0 ? gemm::kSplitMedium : gemm::kSplitSmall, per_fill = kWgradChunk[i] / KS;
     const long long tiles = gemm::tiles_of(tile, M, N);
-    const long long least = (K + kWgradChunk[i] - 1) / kWgradChunk[i];
-    for (int half = 0; half <= 8; ++half) {  // grids of half a chip's workgroups and more
-      long long sp = std::max(least, half * (long long)(gemm::kChipCus / 2) / tiles);
-      sp = std::max(1LL, std::min<long long>(sp, std::max<long long>(least, st / 4)));
+    for (int c = 1; c <= 12; ++c) {  // 1 .. 4 splits, and grids of half a chip's workgroups and more
+      long long sp = c <= 4 ? c : (c - 4) * (long long)(gemm::kChipCus / 2) / tiles;
+      sp = std::max(1LL, std::min<long long>(sp, st / 4));
       const int depth = (int)((st + sp - 1) / sp);
       sp = (st + depth - 1) / depth;
-      double us = gemm::split_grid_us(tile, tiles * sp, depth + 2);
+      double us = (i == 0 ? 1.14 : 1.2) *
+                  gemm::split_grid_us(tile, tiles * sp, depth + 3 * ((depth + per_fill - 1) / per_fill) - 1);
       if (sp > 1) us += 5.0 + (double)(sp + 1) * M * N * 4.0 / 4.0e6;
       if (us < best_us) best_us = us, best = {tile, (int)sp, depth * KS};
     }

@@ -139,21 +139,37 @@ struct WaveMap {
   }
 };
 
-// hi + lo = A B^T over nk stages.  The loaders la / lb give CA / CB chunks of
+// Sums before the first stage, and after the last: mma_stages adds products of
+// scaled operands.
+template <class S>
+__device__ __forceinline__ void clear_sums(f32x4 (&hi)[S::BI][S::BN], f32x4 (&lo)[S::BI][S::BN]) {
+#pragma unroll
+  for (int i = 0; i < S::BI; ++i)
+#pragma unroll
+    for (int n = 0; n < S::BN; ++n) hi[i][n] = lo[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+template <class S>
+__device__ __forceinline__ void unscale_sums(f32x4 (&hi)[S::BI][S::BN], f32x4 (&lo)[S::BI][S::BN]) {
+#pragma unroll
+  for (int i = 0; i < S::BI; ++i)
+#pragma unroll
+    for (int n = 0; n < S::BN; ++n) {
+      hi[i][n] *= kUnscale;
+      lo[i][n] *= kUnscale;
+    }
+}
+
+// hi + lo += 2^48 A B^T over nk stages.  The loaders la / lb give CA / CB chunks of
 // 8 k values per thread and stage: load(x) fetches the next stage's raw values
 // (zeros outside the operand) into a register set, put(lds, x[c], c)
 // splits chunk c into the planes.  nk >= 0; stages past nk are loaded but
 // never multiplied.
 template <class S, class LA, class LB>
-__device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x4 (&hi)[S::BI][S::BN],
-                                         f32x4 (&lo)[S::BI][S::BN]) {
+__device__ __forceinline__ void mma_stages(char* lds, LA& la, LB& lb, int nk, f32x4 (&hi)[S::BI][S::BN],
+                                           f32x4 (&lo)[S::BI][S::BN]) {
   constexpr int BI = S::BI, BN = S::BN, PA = S::PA, PB = S::PB, STG = S::STAGE;
   constexpr int CA = LA::NC, CB = LB::NC, CT = CA + CB;
   const WaveMap<S> w;
-#pragma unroll
-  for (int i = 0; i < BI; ++i)
-#pragma unroll
-    for (int n = 0; n < BN; ++n) hi[i][n] = lo[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
   int ao[BI], bo[BN];  // this lane's fragment slots in plane 0
 #pragma unroll
   for (int i = 0; i < BI; ++i) ao[i] = (int)slot(w.row(i, w.lr), w.q);
@@ -264,13 +280,14 @@ __device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x
     for (int u = 0; u < D; ++u)
       if (kt + u < nk) stage(kt + u, xa[u], xb[u]);
   }
-#pragma unroll
-  for (int i = 0; i < BI; ++i)
-#pragma unroll
-    for (int n = 0; n < BN; ++n) {
-      hi[i][n] *= kUnscale;
-      lo[i][n] *= kUnscale;
-    }
+}
+// hi + lo = A B^T over nk stages.
+template <class S, class LA, class LB>
+__device__ __forceinline__ void mma_loop(char* lds, LA& la, LB& lb, int nk, f32x4 (&hi)[S::BI][S::BN],
+                                         f32x4 (&lo)[S::BI][S::BN]) {
+  clear_sums<S>(hi, lo);
+  mma_stages<S>(lds, la, lb, nk, hi, lo);
+  unscale_sums<S>(hi, lo);
 }
 
 // This thread's K group.

@@ -214,3 +214,40 @@ def test_empty_depth(hip, M, N):
     dW, db = hip.Buffer.from_array(C0), hip.Buffer.from_array(bias)
     hip.call("mle_linear_bwd_ex", None, 0, M, N, 1, gX.ptr, gX.ptr, 0, gW.ptr, 0, gX.ptr, 0, dW.ptr, db.ptr, 0, 0, None, 0)
     assert not dW.numpy().any() and not db.numpy().any()
+
+
+# Weight gradients whose workgroups walk more pixels than their table holds
+# (3072 and 2304): filled again, with a partial last fill, one-element loads
+# (odd maps), 1 x 1 and 3 x 3 filters, each tile, two K groups.
+REFILLS = [(1, 2048, 58, 58, 2048, 1), (1, 128, 113, 113, 4096, 3), (3, 4096, 56, 56, 64, 1), (3, 4096, 57, 57, 64, 1),
+           (4, 2100, 50, 50, 64, 3)]
+
+
+@pytest.mark.parametrize("n,cin,h,w,cout,k", REFILLS)
+def test_split_wgrad_refills_its_table(hip, n, cin, h, w, cout, k):
+    r = rng(cin + h)
+    x = r.standard_normal((n, cin, h, w), dtype=np.float32)
+    dy = r.standard_normal((n, cout, h, w), dtype=np.float32)
+    pad = k // 2
+    dims = (n, cin, h, w, cout, k, k, pad, 1)
+    nb = hip.lib().mle_conv2d_wgrad_ws_bytes(*dims)
+    K, splits = n * h * w, max(1, nb // (4 * (cout * cin * k * k + cout)))
+    assert K / splits > (2304 if cout == 64 else 3072)
+    B = hip.Buffer.from_array
+    gx, gdy, gdw, gdb = B(x), B(dy), B(np.full((cout, cin, k, k), np.nan, np.float32)), B(np.full(cout, np.nan, np.float32))
+    ws = hip.Buffer(nb) if nb else None
+    hip.call("mle_conv2d_wgrad_bias", None, gx.ptr, gdy.ptr, gdw.ptr, gdb.ptr, 0, *dims, ws.ptr if ws else None, nb)
+    got = gdw.numpy((cout, cin, k, k))
+    # 20 rows of dW and 20 of its columns, in float64
+    xp = np.zeros((n, cin, h + 2 * pad, w + 2 * pad), np.float32)
+    xp[:, :, pad:pad + h, pad:pad + w] = x
+    rows, cols = r.choice(cout, 20, replace=False), r.choice(cin, 20, replace=False)
+    for i in range(k):
+        for j in range(k):
+            xs = xp[:, :, i:i + h, j:j + w].transpose(1, 0, 2, 3).reshape(cin, -1)
+            d = dy.transpose(1, 0, 2, 3).reshape(cout, -1)
+            for ci, co in ((np.arange(cin), rows), (cols, np.arange(cout))):
+                a, b = d[co].astype(np.float64), xs[ci].astype(np.float64).T
+                assert np.all(np.abs(got[np.ix_(co, ci)][:, :, i, j] - a @ b) <= bound(K) * (np.abs(a) @ np.abs(b)))
+    db, dba = dy.astype(np.float64).sum((0, 2, 3)), np.abs(dy).sum((0, 2, 3))
+    assert np.all(np.abs(gdb.numpy() - db) <= (K / 4 + 8) * 2.0 ** -24 * dba)

@@ -14,3 +14,9 @@ def test_queries_take_empty_products(zero):
         for layers in (1, 3):
             dx = hip.lib().mle_gemm_sum_ws_bytes(sizes[0], sizes[1], layers)
             assert hip.lib().mle_linear_bwd_ws_bytes(*sizes[:3], layers) == dx
+
+
+@pytest.mark.parametrize("n,cin,side,cout,limit_mb", [(32, 1024, 32, 1024, 152), (16, 256, 128, 256, 20)])
+def test_weight_gradient_workspace_follows_the_chip_not_the_pixels(n, cin, side, cout, limit_mb):
+    """At most four partial gradients, or what fills the chip."""
+    assert hip.lib().mle_conv2d_wgrad_ws_bytes(n, cin, side, side, cout, 3, 3, 1, 1) <= limit_mb * 1e6
