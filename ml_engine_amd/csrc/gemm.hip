@@ -552,13 +552,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_ksplit_pair_kernel(GemmArgs g0, 
 // Tile and K splits of a product on the split kernel: the cheapest by a model
 // of its time in us -- rounds of workgroups times (stages x time of a stage +
 // prologue and epilogue), plus the reduce of the partial products.  A function
-// of the shape only, as mle_gemm_ws_bytes needs.
+// of the shape only, as mle_gemm_ws_bytes needs.  sum: K is the terms of a sum.
 struct SplitChoice {
   int tile = kSplitLarge, splits = 1, kchunk = 0;
   double us = 0;
 };
 
-SplitChoice choose_split(int M, int N, int K, int batch, bool may_split) {
+SplitChoice choose_split(int M, int N, int K, int batch, bool may_split, bool sum = false) {
   SplitChoice best;
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return best;  // nothing to multiply, nothing to divide
   best.us = 1e30;
@@ -577,7 +577,7 @@ SplitChoice choose_split(int M, int N, int K, int batch, bool may_split) {
       last = sp;
       int depth = (int)((st + sp - 1) / sp);
       sp = (st + depth - 1) / depth;
-      double us = split_grid_us(tile, tiles * sp, depth);
+      double us = split_grid_us(tile, tiles * sp, depth, !sum);
       // the reduce: 5 us and its bytes, element by element where rows are no multiple of 4
       if (sp > 1) us += 5.0 + (double)(sp + 1) * M * N * batch * 4.0 / (N % 4 == 0 ? 4.0e6 : 1.5e6);
       if (us < best.us) best = {tile, (int)sp, sp > 1 ? depth * 32 : K, us};
@@ -699,7 +699,7 @@ static int gemm_plan(GemmPlan& P, int trans_a, int trans_b, int M, int N, int K,
   const bool ksplit = !simple && ksplit_shape(M, N, K, batch, terms);
   SplitChoice ch;
   if (!simple && !ksplit && terms <= 1) ch = choose_split(M, N, K, batch, ws != nullptr);
-  if (terms > 1) ch = choose_split(M, N, (int)std::min(2147483000.0, (double)K * terms), batch, false);
+  if (terms > 1) ch = choose_split(M, N, (int)std::min(2147483000.0, (double)K * terms), batch, false, true);
   const double items = (double)tiles_of(ch.tile, M, N) * batch * std::max(ch.splits, std::max(terms, 1));
   split = split && items < 1073741824.0;
   if (terms > 1) {
@@ -1132,7 +1132,7 @@ static int linear_bwd_impl(mle_stream stream, int rows, int in, int out, int lay
   // One launch when both run on the split kernel without a K tail, and the
   // model says that sharing the chip beats one product after the other.
   if (!P0.empty && !P1.empty && P0.split && P1.split && !P0.tail && !P1.tail && !P0.g.grouped && !P1.g.grouped) {
-    const SplitChoice c0 = choose_split(rows, in, out * (layers > 1 ? layers : 1), 1, layers <= 1);
+    const SplitChoice c0 = choose_split(rows, in, out * layers, 1, layers <= 1, layers > 1);
     const SplitChoice c1 = choose_split(in, out, rows, layers, true);
     const PairChoice pc = choose_pair(rows, in, out, layers);
     const double parts = (double)pc.splits * layers * ((double)in * out + out) * sizeof(float);
