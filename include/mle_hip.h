@@ -213,8 +213,8 @@ int mle_gemm(mle_stream stream, int trans_a, int trans_b, int M, int N, int K, f
 
 /* Workspace that lets mle_gemm_ex split K across workgroups when the tile grid
  * alone would leave most CUs idle (0 when no split is used for this shape; a
- * small product that runs on one of the small-product kernels, K split over
- * a workgroup's waves, leaves it unused). */
+ * product that runs on one of the small-product kernels leaves it unused, and
+ * the size asked for it may not be 0). */
 size_t mle_gemm_ws_bytes(int M, int N, int K, int batch);
 /* mle_gemm plus two fusions:
  *   bias (nullable): C[b][r, c] += bias[c] after alpha/beta -- the Linear
@@ -308,12 +308,12 @@ int mle_gemm_act_bwd(mle_stream stream, int trans_a, int trans_b, int M, int N, 
  *   dW_l     += X^T dY_l
  *   db_l     += sum_rows dY_l          (db may be NULL)
  * Layer l's dY, W (and dW), db sit at l * stride_dy, l * stride_w, l * stride_db
- * floats (strides unused when layers == 1).  When both products run on the
- * split-bf16 GEMM at most one workgroup per CU each, or both on one of
- * the small-product kernels, they share one launch; otherwise dX then dW (a
- * weight gradient of one round of tiles beside a larger dX runs as two K
- * splits).  Needs mle_linear_bwd_ws_bytes(rows, in, out, layers) bytes of
- * workspace. */
+ * floats (strides unused when layers == 1).  The two products share one launch
+ * when both run on one of the small-product kernels, or both on the split-bf16
+ * GEMM without a K tail where the library's time model finds that faster;
+ * otherwise dX then dW.  dW may be split over rows either way, so the size of
+ * the workspace follows no simple rule: mle_linear_bwd_ws_bytes(rows, in, out,
+ * layers) bytes are needed. */
 size_t mle_linear_bwd_ws_bytes(int rows, int in, int out, int layers);
 int mle_linear_bwd(mle_stream stream, int rows, int in, int out, int layers,
                    const float* X, const float* dY, int64_t stride_dy,

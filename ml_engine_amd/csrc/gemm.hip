@@ -860,9 +860,11 @@ extern "C" {
 size_t mle_gemm_ws_bytes(int M, int N, int K, int batch) {
   int kchunk;
   int splits = choose_splits(M, N, K, batch, kchunk);
-  // A product of at most 4096 outputs runs on the simple kernel, which leaves
-  // the workspace unused; its size stays that of one split per 32 deep stage.
-  if ((double)M * N * batch <= 4096.0 && (double)M * N * batch > 0.0) splits = std::max(splits, (K + 31) / 32);
+  // A product of at most 4096 outputs and 4 Mi multiply-adds runs on the simple
+  // kernel, which leaves the workspace unused; its size stays that of one split
+  // per 32 deep stage, at most 768.
+  const double outs = (double)M * N * batch;
+  if (outs > 0.0 && outs <= 4096.0 && simple_shape(M, N, K, batch, 1, 0)) splits = std::max(splits, std::min(768, (K + 31) / 32));
   if (splits <= 1) return 0;
   return ((size_t)splits * batch * M * N + (size_t)splits * batch * N) * sizeof(float);
 }

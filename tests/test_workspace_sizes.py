@@ -16,6 +16,14 @@ def test_queries_take_empty_products(zero):
             assert hip.lib().mle_linear_bwd_ws_bytes(*sizes[:3], layers) == dx
 
 
+@pytest.mark.parametrize("rows", [65536, 1_000_000])
+def test_narrow_weight_gradient_workspace(rows):
+    """256 -> 10 over many rows: what the plan's splits need (the gradient's own
+    10 KB a split), not a split per 32 rows (21 MB and 321 MB)."""
+    assert hip.lib().mle_linear_bwd_ws_bytes(rows, 256, 10, 1) <= 4e6
+    assert hip.lib().mle_gemm_ws_bytes(64, 10, rows, 1) <= 4e6
+
+
 @pytest.mark.parametrize("n,cin,side,cout,limit_mb", [(32, 1024, 32, 1024, 152), (16, 256, 128, 256, 20)])
 def test_weight_gradient_workspace_follows_the_chip_not_the_pixels(n, cin, side, cout, limit_mb):
     """At most four partial gradients, or what fills the chip."""
