@@ -735,8 +735,10 @@ __global__ __launch_bounds__(NT * SUB, 4) void norm_bwd_group(const float* __res
 // f(SUB, CPS) for the groups of sh: a chunk per sub-block, except that with
 // more groups of 3 or 4 chunks than CUs two workgroups of half the threads share a
 // CU, one loading while the other reduces (512 groups of 16384, forward /
-// backward: 25 / 33 us with four sub-blocks, 22 / 29 so; not the backward of
-// GELU, which needs more registers than that leaves: 1024 groups, 52 against 61).
+// backward: 23.5 / 32.0 us with four sub-blocks, 19.3 / 27.2 so).  heavy: not the
+// backward of GELU, which needs more registers than that leaves (1024 groups, 51
+// against 61), nor the unaligned backward of a cheap activation, which spills
+// there (1024 groups of 16165 with ReLU: 49 against 66; with SiLU 65 against 68).
 template <class F>
 void with_group(const NormShape& sh, bool heavy, F f) {
   using std::integral_constant;
@@ -751,6 +753,25 @@ void with_group(const NormShape& sh, bool heavy, F f) {
 // forward / backward: 11 / 13 us in two passes, 17 / 23 in one).
 bool whole_group(const NormShape& sh) { return !sh.seg && sh.nchunk <= kGroupChunks; }
 
+// Whether one kernel beats two passes.  Where the activation costs an exponential
+// or more, a group of 3 or 4 chunks keeps one CU's vector unit busy for longer
+// than both passes take when they find two CUs' worth of chunks or fewer, and
+// a second round of workgroups has to be well filled.  SiLU, groups of 16384,
+// forward / backward us, two passes against one kernel: 64 groups 8.7 / 9.3 and 10.1
+// / 12.7; 160 11.7 / 14.9 and 10.7 / 14.0; 256 14.9 / 22.2 and 12.5 / 14.7; 288 16.1 /
+// 24.8 and 16.5 / 25.3; 512 21.0 / 37.7 and 19.3 / 27.2.  Of 12288: 160 10.5 / 12.0 and
+// 10.6 / 13.6; 288 14.0 / 20.2 and 16.1 / 24.1.  GELU, groups of 9400: 112 9.9 / 9.9
+// and 9.2 / 8.9.  Without alignment both passes are slower: the forward of 16 / 288
+// groups of 11529 11.3 / 19.6 and 9.8 / 17.5, the backward of 112 of 16165 16.9 and
+// 15.0 (GELU, 16 groups: 11.4 and 10.2).
+bool cheap_act(int act) { return act < 0 || act == MLE_RELU || act == MLE_LEAKY_RELU; }
+bool one_kernel(const NormShape& sh, int act, bool vec, bool bwd) {
+  if (!whole_group(sh) || sh.nchunk <= 2 || cheap_act(act) || (!vec && !bwd)) return whole_group(sh);
+  const long long chunks = (long long)sh.groups_tot * sh.nchunk;
+  if (sh.groups_tot > 256) return chunks >= 1280;
+  return chunks >= (act == MLE_GELU ? (vec ? 336 : 0) : (vec ? 544 : 400));
+}
+
 // act >= 0: the normalisation also writes act_out = act(y) (+ cbias[channel]).
 void launch_fwd(hipStream_t s, const NormShape& sh, const float* x, float* y, float* stats, void* ws, float eps,
                 bool stats_ready = false, int act = -1, float* act_out = nullptr, const float* cbias = nullptr,
@@ -758,7 +779,7 @@ void launch_fwd(hipStream_t s, const NormShape& sh, const float* x, float* y, fl
   dim3 grid(sh.nchunk, sh.groups_tot);
   double* part = static_cast<double*>(ws);
   const bool v = vec_ok(sh, {x, y}) && (act < 0 || aligned16(act_out)) && (!cbias || cb_hw % 4 == 0);
-  if (!stats_ready && whole_group(sh)) {
+  if (!stats_ready && one_kernel(sh, act, v, false)) {
     with_act(act, [&](auto K) {
       with_group(sh, false, [&](auto SUB, auto CPS) {
         constexpr int A = decltype(K)::value, B = decltype(SUB)::value, C = decltype(CPS)::value;
@@ -837,11 +858,11 @@ void launch_bwd_apply(hipStream_t s, const NormShape& sh, const float* y, const 
 void launch_bwd(hipStream_t s, const NormShape& sh, const float* y, const float* dy, float* dx, const float* stats,
                 void* ws, float eps, size_t quirk, int accumulate, int act = -1, const float* da = nullptr,
                 int acc_dy = 0) {
-  if (!quirk && whole_group(sh)) {
-    const bool v = vec_ok(sh, {y, dy, dx}) && (act < 0 || aligned16(da));
+  const bool v = vec_ok(sh, {y, dy, dx}) && (act < 0 || aligned16(da));
+  if (!quirk && one_kernel(sh, act, v, true)) {
     float* dyw = const_cast<float*>(dy);  // written only with act >= 0
     with_act(act, [&](auto K) {
-      with_group(sh, act == MLE_GELU, [&](auto SUB, auto CPS) {
+      with_group(sh, act == MLE_GELU || (!v && cheap_act(act)), [&](auto SUB, auto CPS) {
         constexpr int A = decltype(K)::value, B = decltype(SUB)::value, C = decltype(CPS)::value;
         const dim3 one(sh.groups_tot);
         if (v) norm_bwd_group<true, A, B, C><<<one, NT * B, 0, s>>>(y, dy, da, dyw, acc_dy, dx, accumulate, stats, sh, eps);

@@ -92,3 +92,33 @@ def test_norm_whole_group(hip, b, c, hw, g, acc):
     assert np.all(np.abs(dy.numpy() - want_dy) <= 32 * U * (np.abs(want_dy) + np.abs(da) + np.abs(dy0) * acc))
     if not (acc and hw % 4 == 0):
         assert np.all(np.abs(a.numpy() - silu(y.numpy().astype(np.float64))) <= 16 * U * np.abs(a.numpy()) + 1e-30)
+
+
+# groups of 3 and 4 chunks on both sides of the rule between one kernel and two
+# passes: few groups, just enough, more than CUs; aligned and not (odd sizes)
+@pytest.mark.parametrize("groups,m", [(16, 16384), (135, 16384), (136, 16384), (181, 12288), (182, 12288), (300, 12288),
+                                      (320, 16384), (427, 12288), (16, 11529), (134, 11529), (100, 16165), (300, 11529)])
+@pytest.mark.parametrize("act", ["relu", "gelu", "silu"])
+def test_norm_group_rule(hip, groups, m, act):
+    """Whichever route a call takes, its results are the two passes' bit for bit."""
+    r = rng(groups + m)
+    n = groups * m
+    x, da = (r.standard_normal(n, dtype=np.float32) for _ in range(2))
+    B, kind = hip.Buffer.from_array, hip.ACT[act]
+    nb = hip.lib().mle_norm_ws_bytes(groups, 1, m, 1)
+    ws, gx, gda, gz = hip.Buffer(nb), B(x), B(da), hip.Buffer.zeros(n)
+    new = lambda k=n: hip.Buffer.zeros(k)  # noqa: E731
+    dims = (groups, 1, m, 1, EPS)
+    y, a, st, y2, a2, st2 = new(), new(), new(2 * groups), new(), new(), new(2 * groups)
+    hip.call("mle_norm_fwd_act", None, gx.ptr, y.ptr, a.ptr, kind, st.ptr, *dims, ws.ptr, nb, 0)
+    hip.call("mle_add_norm_partials", None, gx.ptr, gz.ptr, n, new().ptr, groups, 1, m, 1, ws.ptr, nb)
+    hip.call("mle_norm_fwd_act", None, gx.ptr, y2.ptr, a2.ptr, kind, st2.ptr, *dims, ws.ptr, nb, 1)
+    for one, two in ((y, y2), (a, a2), (st, st2)):
+        np.testing.assert_array_equal(one.numpy(), two.numpy())
+    dy, dx, dy2, dx2 = new(), new(), new(), new()
+    hip.call("mle_norm_bwd_act", None, y.ptr, gda.ptr, kind, dy.ptr, 0, dx.ptr, st.ptr, *dims, 0, ws.ptr, nb, 0)
+    hip.call("mle_norm_bwd_partials", None, y.ptr, dy2.ptr, gda.ptr, kind, 0, groups, 1, m, 1, 0, ws.ptr, nb)
+    hip.call("mle_norm_bwd_apply_add", None, y.ptr, dy2.ptr, dx2.ptr, 0, None, new().ptr, 0, None, 0, st.ptr, *dims, 0,
+             ws.ptr, nb)
+    for one, two in ((dy, dy2), (dx, dx2)):
+        np.testing.assert_array_equal(one.numpy(), two.numpy())
