@@ -425,12 +425,9 @@ __global__ __launch_bounds__(NT) void norm_bwd_partial(const float* __restrict__
   }
 }
 
-// A gradient's old value plus v, v rounded first (no fma): every backward
-// kernel, whatever the compiler makes of its branches, adds the same bits.
-__device__ __forceinline__ float add_rounded(float old, float v) {
-#pragma clang fp contract(off)
-  return old + v;
-}
+// The gradient r t, or added to an old value with one rounding: every backward
+// kernel, whatever the compiler makes of its branches, gives the same bits.
+__device__ __forceinline__ float grad_of(bool acc, float old, float r, float t) { return acc ? fmaf(r, t, old) : r * t; }
 
 // Per group, once (the LayerNorm layout quirk reads other groups' sums per
 // element): fin[2g] = sum(dy), fin[2g+1] = sum(dy * y), same order as group_sums.
@@ -512,8 +509,7 @@ __global__ __launch_bounds__(NT) void norm_bwd_apply(const float* __restrict__ y
         if (!in[u]) continue;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          const float v = r * (gv[u][k] - (sg / fN) - yv[u][k] * (sgy / fN));
-          d[u][k] = acc ? add_rounded(d[u][k], v) : v;
+          d[u][k] = grad_of(acc, d[u][k], r, gv[u][k] - (sg / fN) - yv[u][k] * (sgy / fN));
           d2[u][k] = acc2 ? d2[u][k] + d[u][k] : d[u][k];
           d3[u][k] = acc3 ? d3[u][k] + d[u][k] : d[u][k];
         }
@@ -542,8 +538,7 @@ __global__ __launch_bounds__(NT) void norm_bwd_apply(const float* __restrict__ y
       }
       terms((int)(idx / quirk_hw), sg, sgy, r);
     }
-    const float v = r * (dy[idx] - (sg / fN) - y[idx] * (sgy / fN));
-    const float nv = acc ? add_rounded(dx_in[idx], v) : v;
+    const float nv = grad_of(acc, acc ? dx_in[idx] : 0.f, r, dy[idx] - (sg / fN) - y[idx] * (sgy / fN));
     dx[idx] = nv;
     if (EXTRA) dx2[idx] = acc2 ? dx2[idx] + nv : nv;
     if (EXTRA && dx3) dx3[idx] = acc3 ? dx3[idx] + nv : nv;
@@ -725,8 +720,7 @@ __global__ __launch_bounds__(NT * SUB, 4) void norm_bwd_group(const float* __res
     if (acc) load_chunk<false, VEC>(dx, sh, g, c0, d);
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const float v = r * (gv[j][i] - (sg / fN) - yv[j][i] * (sgy / fN));
-      d[i] = acc ? add_rounded(d[i], v) : v;
+      d[i] = grad_of(acc, acc ? d[i] : 0.f, r, gv[j][i] - (sg / fN) - yv[j][i] * (sgy / fN));
     }
     store_chunk<false, VEC>(dx, sh, g, c0, d);
   }

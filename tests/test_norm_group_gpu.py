@@ -122,3 +122,28 @@ def test_norm_group_rule(hip, groups, m, act):
              ws.ptr, nb)
     for one, two in ((dy, dy2), (dx, dx2)):
         np.testing.assert_array_equal(one.numpy(), two.numpy())
+
+
+@pytest.mark.parametrize("groups,m", [(3, 4096), (2, 11529), (300, 16384), (2, 40000), (2, 40001)])
+def test_norm_gradient_added_with_one_rounding(hip, groups, m):
+    """dx += g rounds once: added to the negative of the rounded gradient it leaves
+    what that rounding dropped, not 0."""
+    r = rng(groups + m)
+    n = groups * m
+    B = hip.Buffer.from_array
+    nb = hip.lib().mle_norm_ws_bytes(groups, 1, m, 1)
+    ws, x, dy = hip.Buffer(nb), B(r.standard_normal(n, dtype=np.float32)), B(r.standard_normal(n, dtype=np.float32))
+    y, st, g = hip.Buffer.zeros(n), hip.Buffer.zeros(2 * groups), hip.Buffer.zeros(n)
+    dims = (groups, 1, m, 1, EPS)
+    hip.call("mle_norm_fwd_ex", None, x.ptr, y.ptr, st.ptr, *dims, ws.ptr, nb, 0)
+    hip.call("mle_norm_bwd", None, y.ptr, dy.ptr, g.ptr, st.ptr, *dims, 0, ws.ptr, nb, 0)
+    rounded = g.numpy()
+    dx, dx2 = B(-rounded), B(-rounded)
+    hip.call("mle_norm_bwd", None, y.ptr, dy.ptr, dx.ptr, st.ptr, *dims, 0, ws.ptr, nb, 1)
+    hip.call("mle_norm_bwd_partials", None, y.ptr, dy.ptr, None, -1, 0, groups, 1, m, 1, 0, ws.ptr, nb)
+    hip.call("mle_norm_bwd_apply_add", None, y.ptr, dy.ptr, dx2.ptr, 1, None, hip.Buffer.zeros(n).ptr, 0, None, 0, st.ptr,
+             *dims, 0, ws.ptr, nb)
+    left = dx.numpy()
+    np.testing.assert_array_equal(left, dx2.numpy())
+    assert np.all(np.abs(left) <= 2.0 ** -24 * np.abs(rounded))
+    assert np.count_nonzero(left) > 0.9 * n
