@@ -477,7 +477,8 @@ __global__ __launch_bounds__(S::NTH * S::KG, 2) void wgrad_split_kernel(WgradArg
     }
     unscale_sums<S>(v, lo);
     if (a.db && tn == 0) {  // the lane groups' sums of each dY row, added in order
-      float* red = reinterpret_cast<float*>(lds);
+      double* red = reinterpret_cast<double*>(lds);
+      static_assert(4 * S::KG * S::TM * 8 <= S::LDS * S::KG, "row sums");
       __syncthreads();
 #pragma unroll
       for (int c = 0; c < LA::NC; ++c) {
@@ -487,9 +488,10 @@ __global__ __launch_bounds__(S::NTH * S::KG, 2) void wgrad_split_kernel(WgradArg
       }
       __syncthreads();
       if (tid < S::TM && m0 + tid < a.M) {
-        float b = red[tid];
+        double s = red[tid];
 #pragma unroll
-        for (int q = 1; q < 4 * S::KG; ++q) b += red[q * S::TM + tid];
+        for (int q = 1; q < 4 * S::KG; ++q) s += red[q * S::TM + tid];
+        const float b = (float)s;
         if (a.splits > 1) a.part_b[(size_t)z * a.M + m0 + tid] = b;
         else a.db[m0 + tid] = a.db_assign ? b : a.db[m0 + tid] + b;
       }

@@ -37,7 +37,8 @@ __device__ __forceinline__ void split_tile(const GemmArgs& g, int tm, int tn, in
     split::mma_loop<S>(lds + group * S::LDS, la, lb, g.kterms * nk, v, lo);
     if (COLSUM && tm == 0) {
       // the lane groups' sums of each column, added in order
-      float* red = reinterpret_cast<float*>(lds);
+      double* red = reinterpret_cast<double*>(lds);
+      static_assert(4 * S::KG * S::TN * 8 <= S::LDS * S::KG, "column sums");
       __syncthreads();
 #pragma unroll
       for (int c = 0; c < LB::NC; ++c) {
@@ -47,11 +48,11 @@ __device__ __forceinline__ void split_tile(const GemmArgs& g, int tm, int tn, in
       }
       __syncthreads();
       if (tid < S::TN && n0 + tid < g.N) {
-        float cs = red[tid];
+        double cs = red[tid];
 #pragma unroll
         for (int q = 1; q < 4 * S::KG; ++q) cs += red[q * S::TN + tid];
-        if (g.splits > 1) g.part_cs[(int64_t)bz * g.N + n0 + tid] = cs;
-        else put_colsum(g, z * g.scs + n0 + tid, cs);
+        if (g.splits > 1) g.part_cs[(int64_t)bz * g.N + n0 + tid] = (float)cs;
+        else put_colsum(g, z * g.scs + n0 + tid, (float)cs);
       }
     }
   }

@@ -369,10 +369,10 @@ struct Chunks {
   static constexpr int NC = NC_;
   static constexpr bool kBranch = false;
   uint32_t dst[NC];
-  float sum[SUM ? NC : 1];  // SUM: each chunk's sum over k
+  double sum[SUM ? NC : 1];  // SUM: each chunk's sum over k (one add per stage and chunk)
   __device__ __forceinline__ void place(int c, int r, int q) {
     dst[c] = slot(r, q);
-    if (SUM) sum[c] = 0.f;
+    if (SUM) sum[c] = 0.0;
   }
   __device__ __forceinline__ void pre() {}
   template <int PL>

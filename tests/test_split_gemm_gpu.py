@@ -251,3 +251,17 @@ def test_split_wgrad_refills_its_table(hip, n, cin, h, w, cout, k):
                 assert np.all(np.abs(got[np.ix_(co, ci)][:, :, i, j] - a @ b) <= bound(K) * (np.abs(a) @ np.abs(b)))
     db, dba = dy.astype(np.float64).sum((0, 2, 3)), np.abs(dy).sum((0, 2, 3))
     assert np.all(np.abs(gdb.numpy() - db) <= (K / 4 + 8) * 2.0 ** -24 * dba)
+
+
+def test_column_sums_of_a_long_depth(hip):
+    """The fused column sums (a bias gradient) round like sums of eight in a tree
+    (three roundings) and one final rounding, at any depth: the stages add in
+    double."""
+    M, N, K = 256, 320, 65536
+    r = rng(8)
+    A, Bm = r.random((K, M), dtype=np.float32), r.random((K, N), dtype=np.float32)
+    B = hip.Buffer.from_array
+    gA, gB, gC, gs = B(A), B(Bm), hip.Buffer.zeros((M, N)), hip.Buffer.zeros(N)
+    hip.call("mle_gemm_ex", None, 1, 0, M, N, K, 1.0, gA.ptr, M, 0, gB.ptr, N, 0, 0.0, gC.ptr, N, 0, 1, gs.ptr, None, None, 0)
+    want = Bm.astype(np.float64).sum(0)
+    assert np.all(np.abs(gs.numpy() - want) <= 4 * 2.0 ** -24 * want)
