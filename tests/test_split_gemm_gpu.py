@@ -265,3 +265,24 @@ def test_column_sums_of_a_long_depth(hip):
     hip.call("mle_gemm_ex", None, 1, 0, M, N, K, 1.0, gA.ptr, M, 0, gB.ptr, N, 0, 0.0, gC.ptr, N, 0, 1, gs.ptr, None, None, 0)
     want = Bm.astype(np.float64).sum(0)
     assert np.all(np.abs(gs.numpy() - want) <= 4 * 2.0 ** -24 * want)
+
+
+@pytest.mark.parametrize("K", [4096, 16384])
+@pytest.mark.parametrize("kind", ["uniform", "near one", "magnitudes"])
+def test_split_gemm_one_signed_error(hip, K, kind):
+    """Operands of one sign, where truncation inside the matrix core would add up:
+    the relative error (2-norm) stays below the fp32 MFMA kernel's, which a
+    column sum of an untransposed A still reaches."""
+    M, N = 300, 700
+    r = rng(K)
+    draw = {"uniform": lambda s: r.random(s), "near one": lambda s: 1 + 1e-3 * r.random(s),
+            "magnitudes": lambda s: np.abs(r.standard_normal(s))}[kind]
+    a, b = draw((M, K)).astype(np.float32), draw((K, N)).astype(np.float32)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    B = hip.Buffer.from_array
+    gA, gB, gC, gs = B(a), B(b), hip.Buffer.zeros((M, N)), hip.Buffer.zeros(N)
+    err = []
+    for colsum in (None, gs.ptr):  # without a workspace: one accumulation over all of K
+        hip.call("mle_gemm_ex", None, 0, 0, M, N, K, 1.0, gA.ptr, K, 0, gB.ptr, N, 0, 0.0, gC.ptr, N, 0, 1, colsum, None, None, 0)
+        err.append(np.linalg.norm(gC.numpy((M, N)) - want) / np.linalg.norm(want))
+    assert err[0] <= err[1], err
