@@ -314,24 +314,24 @@ template <bool DG, int KS, int D>
 __device__ __forceinline__ void conv1_kloop(f32x4 (&acc)[4][4], const Conv3Args& c, int m0, int lr, int q, int ks,
                                             bool gok, int b, int p);
 
-// One 64 WM x 64 WN tile of a 3 x 3 convolution: L is the workgroup's index
+// One 64 x 64 WN tile of a 3 x 3 convolution: L is the workgroup's index
 // among this product's workgroups (its XCD is L % 8).  EXTRA (input
 // gradient only): after the 3 x 3 stages the same accumulators also take the
 // input gradient of a 1 x 1 convolution of the same input (c1: its output
 // gradient and weights), so one tile writes dx = dgrad3 + dgrad1.
-template <bool DG, bool HALO, int WM, int WN, int KS, int U, int D, bool EXTRA = false>
+template <bool DG, bool HALO, int WN, int KS, int U, int D, bool EXTRA = false>
 __device__ __forceinline__ void conv3_direct_body(const Conv3Args& c, const Conv3Args& c1, int L) {
   constexpr int SG = DG ? -1 : 1;  // shift of tap t is SG * (t - 1)
   constexpr int CPS = 4 * U;       // channels per stage
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 15, q = lane >> 4;
-  const int wm = wave % WM, wn = (wave / WM) % WN, ks = wave / (WM * WN);
+  const int wn = wave % WN, ks = wave / WN;
   // Workgroup -> tile: consecutive tiles on one XCD (workgroups are dealt to
   // the 8 XCDs round robin), so neighbouring pixel tiles share its L2.
   const int xq = c.tiles / 8, xr = c.tiles % 8, xc = L % 8;
   const int item = xc * xq + min(xc, xr) + L / 8;
   const int tm = item % c.tiles_m, tn = item / c.tiles_m;
-  const int m0 = (tm * WM + wm) * 64;
+  const int m0 = tm * 64;
   const int g = (tn * WN + wn) * 64 + 4 * lr;
   const bool gok = g < c.npix;
   const int b = g / c.hw, p = g - b * c.hw, py = p / c.w, px = p - py * c.w;
@@ -430,12 +430,12 @@ __device__ __forceinline__ void conv3_direct_body(const Conv3Args& c, const Conv
     if (kt + s < k1) mfma(fa[s], fb[s], fh[s]);
   if (EXTRA) conv1_kloop<true, KS, 4>(acc, c1, m0, lr, q, ks, gok, b, p);
 
-  conv_block_out<DG, WM, WN, KS>(acc, c, m0, lane, wave, ks, gok, b, p);
+  conv_block_out<DG, 1, WN, KS>(acc, c, m0, lane, wave, ks, gok, b, p);
 }
 
-template <bool DG, bool HALO, int WM, int WN, int KS, int U, int D>
-__global__ __launch_bounds__(64 * WM * WN * KS, 2) void conv3_direct_kernel(Conv3Args c) {
-  conv3_direct_body<DG, HALO, WM, WN, KS, U, D>(c, c, blockIdx.x);
+template <bool DG, bool HALO, int WN, int KS, int U, int D>
+__global__ __launch_bounds__(64 * WN * KS, 2) void conv3_direct_kernel(Conv3Args c) {
+  conv3_direct_body<DG, HALO, WN, KS, U, D>(c, c, blockIdx.x);
 }
 
 // Register-direct 1 x 1 convolution (stride 1, pad 0), forward and input
@@ -607,18 +607,17 @@ __global__ __launch_bounds__(64 * WM * WN * KS, 2) void conv1_direct_kernel(Conv
 // 1 x 1 product as extra stages of each 3 x 3 tile.
 template <bool HALO>  // 64-row blocks
 __global__ __launch_bounds__(256, 2) void conv_pair_dgrad_kernel(Conv3Args a, Conv3Args b) {
-  conv3_direct_body<true, HALO, 1, 2, 2, kC3U, kC3D, true>(a, b, blockIdx.x);
+  conv3_direct_body<true, HALO, 2, 2, kC3U, kC3D, true>(a, b, blockIdx.x);
 }
 
 bool a16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 
 // 64-row blocks (M <= 64) split each block's stages over two waves, so the
-// grid still holds two waves per SIMD; the 3 x 3 kernel runs with them only
-// (direct_better).
+// grid still holds two waves per SIMD; the 3 x 3 kernel has no other.
 template <bool DG, bool HALO>
 void launch_conv3(hipStream_t s, const Conv3Args& c) {
-  mle::launch(conv3_direct_kernel<DG, HALO, 1, 2, 2, kC3U, kC3D>, c.tiles, 256, 0, s, c);
+  mle::launch(conv3_direct_kernel<DG, HALO, 2, 2, kC3U, kC3D>, c.tiles, 256, 0, s, c);
 }
 
 template <bool DG, int WM>
@@ -690,7 +689,7 @@ bool conv_direct(hipStream_t s, bool dg, const ConvGeom& g, const float* src, co
   Conv3Args c;
   bool k3, halo;
   int wm;
-  if (!direct_args(dg, g, src, wt, bias, out, acc, c, k3, wm, halo)) return false;
+  if (!direct_args(dg, g, src, wt, bias, out, acc, c, k3, wm, halo) || (k3 && wm != 1)) return false;
   if (!k3) {
     if (dg) wm == 1 ? launch_conv1<true, 1>(s, c) : launch_conv1<true, 2>(s, c);
     else wm == 1 ? launch_conv1<false, 1>(s, c) : launch_conv1<false, 2>(s, c);
