@@ -73,9 +73,9 @@ constexpr int kSplitTm[3] = {256, 128, 64}, kSplitTn[3] = {128, 128, 64};
 // at once), medium 1.4 + 5.5, small 0.53 + 4.5 (one workgroup per CU, two K
 // groups; 0.67 with one, where the terms of a sum follow each other: 3 terms of
 // 512 x 512 x 1024 in 70 us); 0.53 + 1.7 for each small tile of a CU that several
-// share, and 2.2 more (2500 x 512 x 64: small 9.0, medium 9.9).
+// share, and 3.0 more (2.2 for one or two stages; 2500 x 512 x 64: small 9.0, medium 9.9).
 constexpr double kStageUs[3] = {2.3, 1.4, 0.53}, kTileUs[3] = {8.0, 5.5, 4.5};
-constexpr double kFullTileUs = 13.0, kSharedTileUs = 1.7, kSharedUs = 2.2, kOneGroupStageUs = 0.67;
+constexpr double kFullTileUs = 13.0, kSharedTileUs = 1.7, kSharedUs = 3.0, kSharedShortUs = 2.2, kOneGroupStageUs = 0.67;
 constexpr int kChipCus = 256;
 
 inline long long tiles_of(int tile, int M, int N) {
@@ -88,7 +88,7 @@ inline double split_grid_us(int tile, long long n, int stages, bool k_groups = t
   const long long per = (n + kChipCus - 1) / kChipCus;  // workgroups per CU
   if (per == 1) return stages * (tile == kSplitSmall && !k_groups ? kOneGroupStageUs : kStageUs[tile]) + kTileUs[tile];
   const double t = tile == kSplitLarge ? kFullTileUs : tile == kSplitMedium ? kTileUs[tile] : kSharedTileUs;
-  return (double)per * (stages * kStageUs[tile] + t) + (tile == kSplitSmall ? kSharedUs : 0.0);
+  return (double)per * (stages * kStageUs[tile] + t) + (tile != kSplitSmall ? 0.0 : stages <= 2 ? kSharedShortUs : kSharedUs);
 }
 
 // trans: 2 * trans_a + trans_b.  tail: K % 4 != 0 beside a k-contiguous operand
