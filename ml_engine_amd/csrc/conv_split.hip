@@ -438,6 +438,11 @@ struct XLoad : Chunks<R * 4 / NTH, false> {
 template <class S, bool V4, bool ONE, int CHUNK>
 __global__ __launch_bounds__(S::NTH * S::KG, 2) void wgrad_split_kernel(WgradArgs a, int gx, int gy, int items) {
   constexpr int BI = S::BI, BN = S::BN;
+  // Stages summed before they join the total: 1536 pixels of the medium tile, 768
+  // of the small ones.  Error against 64 bits, one sum per split / so: 22 x 188 ->
+  // 16 on 56 x 56 (9 splits of two K groups) 3.8e-7 / 1.4e-7, 30 x 250 -> 250 on
+  // 28 x 28 (7 splits) 3.3e-7 / 2.3e-7.
+  constexpr int kRun = S::TM == 128 ? 48 : 24 / S::KG;
   using T = PixTable<CHUNK>;
   __shared__ __attribute__((aligned(16))) char lds[S::LDS * S::KG];
   __shared__ __attribute__((aligned(16))) T tab;
@@ -451,7 +456,9 @@ __global__ __launch_bounds__(S::NTH * S::KG, 2) void wgrad_split_kernel(WgradArg
     LA la;
     const int group = k_group<S>(), t = tid % S::NTH;
     la.init(a.dy, a.dy_bytes, a.M, a.g.oh * a.g.ow, tab.dy, m0, t);
+    Sums<S> total;
     clear_sums<S>(v, lo);
+    clear_sums<S>(total.v, lo);
     auto chunks = [&](auto& lb) {
 #pragma unroll 1
       for (int c0 = 0; c0 < klen; c0 += CHUNK) {
@@ -463,7 +470,7 @@ __global__ __launch_bounds__(S::NTH * S::KG, 2) void wgrad_split_kernel(WgradArg
         const int nk = ((n + KS - 1) / KS + S::KG - 1) / S::KG, k0 = group * nk * KS;
         la.seek(k0, nk, t);
         lb.seek(k0, nk, t);
-        mma_stages<S>(lds + group * S::LDS, la, lb, nk, v, lo);
+        mma_stages<S, kRun>(lds + group * S::LDS, la, lb, nk, v, lo, &total);
       }
     };
     if constexpr (ONE) {
@@ -475,6 +482,10 @@ __global__ __launch_bounds__(S::NTH * S::KG, 2) void wgrad_split_kernel(WgradArg
       lb.init(a, &tab, n0, t);
       chunks(lb);
     }
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int n = 0; n < BN; ++n) v[i][n] = total.v[i][n];
     unscale_sums<S>(v, lo);
     if (a.db && tn == 0) {  // the lane groups' sums of each dY row, added in order
       double* red = reinterpret_cast<double*>(lds);
@@ -594,7 +605,8 @@ struct WgradPlan {
 // Tile (medium or small) and pixel splits: the cheapest by the model, the
 // reduce of the partial gradients and three stages per fill of the table included.
 // A stage with x gathered takes 1.6 / 0.64 us where the GEMM's takes 1.4 / 0.53
-// (16 x 128 -> 128 and 128 -> 32 on 64 x 64, one round).  The table does not bound
+// (16 x 128 -> 128 and 128 -> 32 on 64 x 64, one round), 0.66 with two K groups (28 x
+// 144 -> 16 on 32 x 32: 58 us, 54.6 with two small tiles on a CU instead).  The table does not bound
 // the splits, so the workspace does not grow with the pixels: four copies of dW
 // or what fills the chip (1024 -> 1024 on 32 x 32, batch 32: 151 MB for 3.7 ms,
 // where one split takes 4.8; 256 -> 256 on 128 x 128, batch 16: 17 MB).
@@ -611,8 +623,10 @@ WgradPlan wgrad_plan(const ConvGeom& g) {
       sp = std::max(1LL, std::min<long long>(sp, st / 4));
       const int depth = (int)((st + sp - 1) / sp);
       sp = (st + depth - 1) / depth;
-      double us = (i == 0 ? 1.14 : 1.2) *
-                  gemm::split_grid_us(tile, tiles * sp, depth + 3 * ((depth + per_fill - 1) / per_fill) - 1);
+      // (two small tiles fit a CU beside their tables: full rounds are of 512)
+      const long long n = i == 1 && tiles * sp > gemm::kChipCus ? (tiles * sp + 511) / 512 * 512 : tiles * sp;
+      double us = (i == 0 ? 1.14 : n <= gemm::kChipCus ? 1.25 : 1.2) *
+                  gemm::split_grid_us(tile, n, depth + 3 * ((depth + per_fill - 1) / per_fill) - 1);
       if (sp > 1) us += 5.0 + (double)(sp + 1) * M * N * 4.0 / 4.0e6;
       if (us < best_us) best_us = us, best = {tile, (int)sp, depth * KS};
     }

@@ -142,6 +142,10 @@ struct WaveMap {
 // Sums before the first stage, and after the last: mma_stages adds products of
 // scaled operands.
 template <class S>
+struct Sums {  // of finished runs of stages
+  f32x4 v[S::BI][S::BN];
+};
+template <class S>
 __device__ __forceinline__ void clear_sums(f32x4 (&hi)[S::BI][S::BN], f32x4 (&lo)[S::BI][S::BN]) {
 #pragma unroll
   for (int i = 0; i < S::BI; ++i)
@@ -159,14 +163,16 @@ __device__ __forceinline__ void unscale_sums(f32x4 (&hi)[S::BI][S::BN], f32x4 (&
     }
 }
 
-// hi + lo += 2^48 A B^T over nk stages.  The loaders la / lb give CA / CB chunks of
+// hi + lo += 2^48 A B^T over nk stages.  RUN > 0 (a multiple of DEPTH): after every
+// RUN stages and at the end the sums move to `total`, so that a long K rounds
+// like the sum of short ones.  The loaders la / lb give CA / CB chunks of
 // 8 k values per thread and stage: load(x) fetches the next stage's raw values
 // (zeros outside the operand) into a register set, put(lds, x[c], c)
 // splits chunk c into the planes.  nk >= 0; stages past nk are loaded but
 // never multiplied.
-template <class S, class LA, class LB>
+template <class S, int RUN = 0, class LA, class LB>
 __device__ __forceinline__ void mma_stages(char* lds, LA& la, LB& lb, int nk, f32x4 (&hi)[S::BI][S::BN],
-                                           f32x4 (&lo)[S::BI][S::BN]) {
+                                           f32x4 (&lo)[S::BI][S::BN], Sums<S>* total = nullptr) {
   constexpr int BI = S::BI, BN = S::BN, PA = S::PA, PB = S::PB, STG = S::STAGE;
   constexpr int CA = LA::NC, CB = LB::NC, CT = CA + CB;
   const WaveMap<S> w;
@@ -275,10 +281,20 @@ __device__ __forceinline__ void mma_stages(char* lds, LA& la, LB& lb, int nk, f3
       }
     }
   };
-  for (int kt = 0; kt < nk; kt += D) {
+  static_assert(RUN % D == 0, "whole rounds of the register sets");
+  for (int k0 = 0; k0 < nk; k0 += RUN) {
+    const int end = RUN > 0 ? min(nk, k0 + RUN) : nk;
+    for (int kt = k0; kt < end; kt += D) {
 #pragma unroll
-    for (int u = 0; u < D; ++u)
-      if (kt + u < nk) stage(kt + u, xa[u], xb[u]);
+      for (int u = 0; u < D; ++u)
+        if (kt + u < end) stage(kt + u, xa[u], xb[u]);
+    }
+    if (RUN == 0) break;
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int n = 0; n < BN; ++n) total->v[i][n] += hi[i][n] + lo[i][n];
+    clear_sums<S>(hi, lo);
   }
 }
 // hi + lo = A B^T over nk stages.

@@ -220,7 +220,7 @@ def test_empty_depth(hip, M, N):
 # (3072 and 2304): filled again, with a partial last fill, one-element loads
 # (odd maps), 1 x 1 and 3 x 3 filters, each tile, two K groups.
 REFILLS = [(1, 2048, 58, 58, 2048, 1), (1, 128, 113, 113, 4096, 3), (3, 4096, 56, 56, 64, 1), (3, 4096, 57, 57, 64, 1),
-           (4, 2100, 50, 50, 64, 3)]
+           (4, 2100, 50, 50, 64, 3), (8, 4096, 57, 57, 64, 1)]
 
 
 @pytest.mark.parametrize("n,cin,h,w,cout,k", REFILLS)
@@ -286,3 +286,30 @@ def test_split_gemm_one_signed_error(hip, K, kind):
         hip.call("mle_gemm_ex", None, 0, 0, M, N, K, 1.0, gA.ptr, K, 0, gB.ptr, N, 0, 0.0, gC.ptr, N, 0, 1, colsum, None, None, 0)
         err.append(np.linalg.norm(gC.numpy((M, N)) - want) / np.linalg.norm(want))
     assert err[0] <= err[1], err
+
+
+def test_split_wgrad_long_sums_error(hip):
+    """Few splits over many pixels: the stages are summed in runs of at most 24.  A
+    running sum of n random stages is truncated by up to 2^-23 of itself, rms half
+    of that, at sizes that grow with the square root: 2^-24 sqrt(n / 2) of the
+    result.  One sum per split (over 100 stages) would be at 4.2e-7."""
+    n, cin, h, cout = 22, 188, 56, 16
+    r = rng(12)
+    x, dy = (r.standard_normal((n, c, h, h), dtype=np.float32) for c in (cin, cout))
+    dims = (n, cin, h, h, cout, 3, 3, 1, 1)
+    nb = hip.lib().mle_conv2d_wgrad_ws_bytes(*dims)
+    assert n * h * h / 32 / max(1, nb // (4 * (cout * cin * 9 + cout))) > 100
+    B = hip.Buffer.from_array
+    gx, gdy, gdw, ws = B(x), B(dy), hip.Buffer.zeros((cout, cin, 3, 3)), hip.Buffer(max(nb, 4))
+    hip.call("mle_conv2d_wgrad", None, gx.ptr, gdy.ptr, gdw.ptr, *dims, ws.ptr, nb)
+    got = gdw.numpy((cout, cin, 3, 3))
+    xp = np.zeros((n, cin, h + 2, h + 2), np.float32)
+    xp[:, :, 1:-1, 1:-1] = x
+    d = dy.transpose(1, 0, 2, 3).reshape(cout, -1).astype(np.float64)
+    err = ref = 0.0
+    for i in range(3):
+        for j in range(3):
+            want = d @ xp[:, :, i:i + h, j:j + h].transpose(1, 0, 2, 3).reshape(cin, -1).astype(np.float64).T
+            err += np.square(got[:, :, i, j] - want).sum()
+            ref += np.square(want).sum()
+    assert np.sqrt(err / ref) <= 2.0 ** -24 * np.sqrt(24 / 2)
