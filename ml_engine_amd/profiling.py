@@ -78,7 +78,7 @@ OTHER_FAMILIES = [("conv_wgrad", re.compile(r"wgrad_split_kernel<")),
                   ("adam_update", re.compile(r"adam(_vec)?_kernel<")),
                   ("sqnorm", re.compile(r"sqnorm_partial<")),
                   ("attn_fwd", re.compile(r"attn_(stats|fwd)(_slice|_split)?_kernel<")),
-                  ("attn_bwd", re.compile(r"attn_bwd_(kv|q|slice)(_split)?_kernel<"))]
+                  ("attn_bwd", re.compile(r"attn_bwd_(kv|k|q|slice)(_split)?_kernel<"))]
 
 
 def family_of(name: str) -> str | None:
